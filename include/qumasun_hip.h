@@ -168,9 +168,9 @@ int qm_nonlocal_add_f32(qm_ctx *ctx, float *d_out, const float *d_psi, int nb, i
  * qm_stencil_choice          candidate in use for that shape, -1 if not tuned yet
  *                            (kt bit 0: a k-point with |k_d| >= 1e-8 in some d;
  *                            kt bit 1: the shape of full qm_hpsi_apply_* calls).
- * A full qm_hpsi_apply_* runs the stencil beside the nonlocal projection; its
- * shape is tuned separately, on full applies, the first time that shape of
- * call is seen (and synchronises the stream then). */
+ * A full qm_hpsi_apply_* runs the stencil after the nonlocal projection or
+ * beside it; its shape and that order are tuned separately, on full applies,
+ * the first time that shape of call is seen (and synchronises the stream then). */
 int qm_stencil_num_candidates(void);
 int qm_stencil_candidate_name(int candidate, char *buf, int buflen);
 int qm_stencil_force(qm_ctx *ctx, int candidate);

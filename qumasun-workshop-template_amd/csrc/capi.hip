@@ -231,6 +231,12 @@ int launch_local(qm_ctx *ctx, T *out, const T *in, int nb, int ncomp, const doub
     else return launch_fd8_local_f32(ctx, out, in, nb, ncomp, k, st);
 }
 
+// Applies that take less than this one after the other never overlap: the
+// fork and the join cost ~12 us, more than the overlap gives there (32^3 x 24
+// FP64: 28 us in order, 45-50 us overlapped; at 64^3 x 128 FP32 the overlap
+// wins, 143 against 158 us on warm caches).
+constexpr float kOverlapMinMs = 0.1f;
+
 // part: 3 = local + nonlocal (overwrite), 1 = local only (overwrite), 2 = nonlocal only (accumulate)
 template <typename T>
 int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, void *stream, int part = 3) {
@@ -248,33 +254,47 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
     const KPoint &kp = ctx->kpts[ik];
     const bool nl = ctx->proj.natoms > 0 && ctx->proj.ptot > 0;
     if (part == 3 && nl) {
-        // The projection reads psi only and the stencil writes hpsi only: the
-        // projection (and its coefficient sum) runs on the context's second
-        // stream beside the stencil, and the scatter waits for both.  The fork
-        // event is recorded after everything the caller queued before, which
-        // includes the previous apply's scatter, the last reader of the
-        // coefficient buffer.
-        QM_TRY(side_stream(ctx));
+        // The projection reads psi only and the stencil writes hpsi only, so
+        // there are two schedules, the same kernels and the same values:
+        // `in_order` runs projection, coefficient sums, local part and scatter
+        // one after the other on the caller's stream; `overlapped` runs the
+        // projection and its sums on the context's second stream beside the
+        // local part, and the scatter waits for both.  The fork event is
+        // recorded after everything the caller queued before, which includes
+        // the previous apply's scatter, the last reader of the coefficient
+        // buffer.
         const int prec = sizeof(T) == 8 ? 64 : 32;
         const int kt = (std::fabs(kp.k[0]) >= 1.0e-8 || std::fabs(kp.k[1]) >= 1.0e-8 ||
                         std::fabs(kp.k[2]) >= 1.0e-8) ? 1 : 0;
-        auto full = [&]() -> int {
+        auto project = [&](hipStream_t s) -> int {
+            if constexpr (sizeof(T) == 8) return nonlocal_project_f64(ctx, psi, nb, ncomp, kp, s);
+            else return nonlocal_project_f32(ctx, psi, nb, ncomp, kp, s);
+        };
+        auto scatter = [&]() -> int {
+            if constexpr (sizeof(T) == 8) return nonlocal_scatter_f64(ctx, hpsi, nb, ncomp, kp, st);
+            else return nonlocal_scatter_f32(ctx, hpsi, nb, ncomp, kp, st);
+        };
+        auto in_order = [&]() -> int {
+            QM_TRY(project(st));
+            QM_TRY(launch_local<T>(ctx, hpsi, psi, nb, ncomp, kp.k, st));
+            return scatter();
+        };
+        auto overlapped = [&]() -> int {
+            QM_TRY(side_stream(ctx));
             QM_HIP(hipEventRecord(ctx->ev_fork, st));
             QM_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-            if constexpr (sizeof(T) == 8) QM_TRY(nonlocal_project_f64(ctx, psi, nb, ncomp, kp, ctx->side));
-            else QM_TRY(nonlocal_project_f32(ctx, psi, nb, ncomp, kp, ctx->side));
+            QM_TRY(project(ctx->side));
             QM_HIP(hipEventRecord(ctx->ev_join, ctx->side));
             QM_TRY(launch_local<T>(ctx, hpsi, psi, nb, ncomp, kp.k, st));
             QM_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
-            if constexpr (sizeof(T) == 8) QM_TRY(nonlocal_scatter_f64(ctx, hpsi, nb, ncomp, kp, st));
-            else QM_TRY(nonlocal_scatter_f32(ctx, hpsi, nb, ncomp, kp, st));
-            return QM_OK;
+            return scatter();
         };
-        if (ctx->stencil_force >= 0 || ctx->kinetic == QM_KINETIC_FFT) return full();
-        // The stencil's tile shape for full applies is tuned on full applies:
-        // the shape that runs fastest alone is not always the one that leaves
-        // the projection the most room beside it.  Every shape gives the same
-        // values, so the timed applies also leave the right result.
+        if (ctx->stencil_force >= 0 || ctx->kinetic == QM_KINETIC_FFT) return overlapped();
+        // The schedule, and the stencil's tile shape in it, are tuned on full
+        // applies: the shape that runs fastest alone is not always the one
+        // that leaves the projection the most room beside it.  Every choice
+        // gives the same values, so the timed applies also leave the right
+        // result.
         struct Force {  // the shape for this call; restored on every return
             qm_ctx *c;
             ~Force() { c->stencil_force = -1; }
@@ -282,35 +302,50 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
         const int64_t key = stencil_full_key(prec, ncomp, kt, nb);
         auto it = ctx->stencil_choice.find(key);
         int cand = 0;
+        bool beside = true;
         if (it != ctx->stencil_choice.end()) {
             cand = it->second;
+            beside = ctx->apply_overlapped[key];
         } else {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             QM_HIP(hipStreamIsCapturing(st, &cs));
             if (cs == hipStreamCaptureStatusNone) {
+                // the local shape is tuned alone first (once per shape)
+                QM_TRY(in_order());
+                const int alone = stencil_choice(ctx, prec, ncomp, kt, nb);
+                QM_CHECK(alone >= 0, QM_ERR_STATE, "H.psi shape tuning: no local shape");
                 hipEvent_t ev[2] = {nullptr, nullptr};
                 QM_HIP(hipEventCreate(&ev[0]));
                 if (hipEventCreate(&ev[1]) != hipSuccess) {
                     (void)hipEventDestroy(ev[0]);
                     QM_CHECK(false, QM_ERR_HIP, "hipEventCreate failed");
                 }
-                float best_ms = 1e30f;
                 int status = QM_OK;
-                for (int c = 0; c < stencil_num_candidates() && status == QM_OK; ++c) {
-                    if (!stencil_feasible(ctx, c, prec, ncomp)) continue;
-                    ctx->stencil_force = c;
-                    // one warm-up apply, then the mean of 4: overlapped applies vary
-                    // by ~10 % from run to run
-                    if (status == QM_OK) status = full();
+                // mean of `reps` applies after a warm-up
+                auto timed = [&](auto &&run, int reps) -> float {
                     float ms = 0.0f;
+                    status = run();
                     if (status == QM_OK && hipEventRecord(ev[0], st) != hipSuccess) status = QM_ERR_HIP;
-                    for (int rep = 0; rep < 4 && status == QM_OK; ++rep) status = full();
+                    for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
                     if (status == QM_OK && hipEventRecord(ev[1], st) != hipSuccess) status = QM_ERR_HIP;
                     if (status == QM_OK && hipEventSynchronize(ev[1]) != hipSuccess) status = QM_ERR_HIP;
                     if (status == QM_OK && hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) status = QM_ERR_HIP;
-                    if (status == QM_OK && ms < best_ms) {
-                        best_ms = ms;
-                        cand = c;
+                    return ms / (float)reps;
+                };
+                cand = alone;
+                beside = false;
+                ctx->stencil_force = alone;
+                float best_ms = timed(in_order, 4);
+                if (best_ms > kOverlapMinMs) {
+                    for (int c = 0; c < stencil_num_candidates() && status == QM_OK; ++c) {
+                        if (!stencil_near_best(ctx, prec, ncomp, kt, nb, c)) continue;
+                        ctx->stencil_force = c;
+                        const float ms = timed(overlapped, 4);
+                        if (status == QM_OK && ms < best_ms) {
+                            best_ms = ms;
+                            cand = c;
+                            beside = true;
+                        }
                     }
                 }
                 (void)hipEventDestroy(ev[0]);
@@ -318,10 +353,11 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 if (status == QM_ERR_HIP) set_error("H.psi shape tuning: HIP event failure");
                 if (status != QM_OK) return status;
                 ctx->stencil_choice[key] = cand;
+                ctx->apply_overlapped[key] = beside;
             }
         }
         ctx->stencil_force = cand;
-        return full();
+        return beside ? overlapped() : in_order();
     }
     if (part & 1) QM_TRY(launch_local<T>(ctx, hpsi, psi, nb, ncomp, kp.k, st));
     if constexpr (sizeof(T) == 8) {

@@ -130,6 +130,8 @@ struct qm_ctx {
     qm::DevBuf gemm_part; // Gram partial sums of qm_gram_*
     qm::DevBuf nl_part;   // per-chunk projection partials (FP64)
     std::map<int64_t, int> stencil_choice;  // autotuned stencil candidate per shape
+    std::map<int64_t, std::vector<float>> stencil_ms;  // each candidate's time when its shape was tuned (ms)
+    std::map<int64_t, bool> apply_overlapped;  // tuned schedule of full applies (by their stencil_choice key)
     int stencil_force = -1;                 // >= 0: use this candidate, no tuning
     std::map<int64_t, int> nl_choice;       // autotuned column tiles per projection workgroup per shape
     int nl_force = 0;                       // > 0: use this many column tiles, no tuning
@@ -175,7 +177,10 @@ int stencil_choice(const qm_ctx *ctx, int precision, int ncomp, int kt, int nb);
 // key of the tile shape a full H.psi apply (stencil beside the nonlocal
 // projection) uses, tuned on full applies; and whether a shape can run
 int64_t stencil_full_key(int precision, int ncomp, int kt, int nb);
-bool stencil_feasible(const qm_ctx *ctx, int cand, int precision, int ncomp);
+// whether a shape, timed alone when the local shape was tuned, came within
+// 12 % of the fastest (the shapes worth timing beside the projection: on 64^3
+// x 128 FP32 the best one there is 4 % off the best alone)
+bool stencil_near_best(const qm_ctx *ctx, int precision, int ncomp, int kt, int nb, int cand);
 
 // eigen.hip: FP64 symmetric eigensolver pieces (rocblas_handle passed as void *)
 int sytrd_lower(void *blas, int n, double *C, int lda, double *trd, double *VW, hipStream_t st);

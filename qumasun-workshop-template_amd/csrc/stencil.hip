@@ -46,6 +46,7 @@
 //
 // Both kernels do the same arithmetic in the same order for every point, so
 // every candidate gives bit-identical results.
+#include <algorithm>
 #include <cmath>
 
 #include "qm_internal.h"
@@ -610,6 +611,7 @@ constexpr Candidate kCandidates[] = {
     {false, 4, 0, 64}, {false, 8, 0, 16}, {false, 8, 0, 32}, {false, 8, 0, 64},
     {true, 4, 16, 32}, {true, 4, 16, 64}, {true, 4, 16, 0},  {true, 2, 16, 0},
     {true, 4, 8, 0},   {true, 4, 10, 0},  {true, 4, 12, 0},  {true, 2, 16, 32},
+    {false, 2, 0, 8},  {false, 4, 0, 8},
 };
 constexpr int kNumCandidates = sizeof(kCandidates) / sizeof(kCandidates[0]);
 
@@ -761,10 +763,12 @@ int64_t tune_key(int precision, int ncomp, bool kt, int nb) {
 }
 
 // Times every candidate on the caller's buffers (each run overwrites out with
-// the same values) and returns the fastest in *best.
+// the same values) and returns the fastest in *best, their times in *cand_ms
+// (1e30 where a candidate does not run).
 template <typename T>
 int autotune(const qm_ctx *ctx, int ncomp, bool kt, T *out, const T *in, const T *vloc, int nb, const FD8Coef<T> &c,
-             hipStream_t st, int *best) {
+             hipStream_t st, int *best, std::vector<float> *cand_ms) {
+    cand_ms->assign(kNumCandidates, 1e30f);
     hipEvent_t ev[2];
     QM_HIP(hipEventCreate(&ev[0]));
     if (hipEventCreate(&ev[1]) != hipSuccess) {
@@ -786,6 +790,7 @@ int autotune(const qm_ctx *ctx, int ncomp, bool kt, T *out, const T *in, const T
             if (status == QM_OK && hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) status = QM_ERR_HIP;
             if (status == QM_OK && rep > 0) t_min = std::min(t_min, ms);
         }
+        (*cand_ms)[cand] = t_min;
         if (status == QM_OK && t_min < best_ms) {
             best_ms = t_min;
             *best = cand;
@@ -818,7 +823,9 @@ int launch_fd8(qm_ctx *ctx, T *out, const T *in, const T *vloc, int nb, int ncom
             if (cs != hipStreamCaptureStatusNone) {
                 cand = 0;  // no timing inside a capture: the default shape
             } else {
-                QM_TRY(autotune<T>(ctx, ncomp, kt, out, in, vloc, nb, c, st, &cand));
+                std::vector<float> ms;
+                QM_TRY(autotune<T>(ctx, ncomp, kt, out, in, vloc, nb, c, st, &cand, &ms));
+                ctx->stencil_ms[key] = ms;
                 ctx->stencil_choice[key] = cand;
             }
         }
@@ -844,8 +851,11 @@ int64_t stencil_full_key(int precision, int ncomp, int kt, int nb) {
     return tune_key(precision, ncomp, kt != 0, nb) | ((int64_t)1 << 60);
 }
 
-bool stencil_feasible(const qm_ctx *ctx, int cand, int precision, int ncomp) {
-    return precision == 64 ? feasible_any<double>(ctx, cand, ncomp) : feasible_any<float>(ctx, cand, ncomp);
+bool stencil_near_best(const qm_ctx *ctx, int precision, int ncomp, int kt, int nb, int cand) {
+    auto it = ctx->stencil_ms.find(tune_key(precision, ncomp, kt != 0, nb));
+    if (it == ctx->stencil_ms.end()) return false;
+    const std::vector<float> &ms = it->second;
+    return ms[cand] <= 1.12f * *std::min_element(ms.begin(), ms.end());
 }
 
 int stencil_choice(const qm_ctx *ctx, int precision, int ncomp, int kt, int nb) {
