@@ -383,14 +383,8 @@ int band_density_impl(qm_ctx *ctx, double *rho, const T *psi, const double *occ,
     if (nb == 0) return QM_OK;
     QM_TRY(activate(ctx));
     hipStream_t st = (hipStream_t)stream;
-    QM_TRY(ctx->fwork.reserve(sizeof(double) * nb));
-    double *d_occ = ctx->fwork.as<double>();
-    QM_HIP(hipMemcpyAsync(d_occ, occ, sizeof(double) * nb, hipMemcpyHostToDevice, st));
-    if constexpr (sizeof(T) == 8) QM_TRY(launch_band_density_f64(ctx, rho, psi, d_occ, nb, ncomp, st));
-    else QM_TRY(launch_band_density_f32(ctx, rho, psi, d_occ, nb, ncomp, st));
-    // the occupancy staging buffer is reused by the next call: finish first
-    QM_HIP(hipStreamSynchronize(st));
-    return QM_OK;
+    if constexpr (sizeof(T) == 8) return launch_band_density_f64(ctx, rho, psi, occ, nb, ncomp, st);
+    else return launch_band_density_f32(ctx, rho, psi, occ, nb, ncomp, st);
 }
 
 template <typename T>

@@ -31,8 +31,6 @@
 namespace qm {
 namespace {
 
-constexpr int NL_THREADS = 256;
-
 // Workgroup numbering: hardware block b runs on XCD b % 8, so giving each XCD a
 // contiguous range of logical blocks puts consecutive logical blocks (the
 // column groups of one item or point block) on one XCD, where they share its
@@ -315,105 +313,212 @@ __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
         if (cg + q < ncol) hpsi[(int64_t)(cg + q) * ng + g] = hv[q];
 }
 
-// Per (atom, band group, group of MM projectors): E_nl and
-// F = 2 sum occ E Re(conj(<p|psi>) <dp/dr|psi>) over the projectors
-// MM blockIdx.z .. MM blockIdx.z + MM - 1 of the atom.
-// out[((blockIdx.z * gridDim.y + blockIdx.y) * natoms + a) * 4 + {0: E, 1..3: F}]
-template <typename T, int MM, int NBG, int NC, bool PH>
-__global__ __launch_bounds__(NL_THREADS) void nl_force_kernel(
-    double *__restrict__ out, const T *__restrict__ psi, int64_t ng, int nb, int natoms, const double *__restrict__ occ,
-    const int *__restrict__ nproj, const int *__restrict__ proj_off, const int64_t *__restrict__ vox_off,
-    const int64_t *__restrict__ tab_off, int64_t ttot, const int *__restrict__ vox_grid, const T *__restrict__ table,
-    const T *__restrict__ dtable, const T *__restrict__ phase, const double *__restrict__ energy, double dV) {
-    constexpr int NV = 4 * MM * NBG * NC;
-    __shared__ double red[NL_THREADS / 64][NV];
-    __shared__ double tot[4];
-    const int a = blockIdx.x;
-    const int n0 = blockIdx.y * NBG;
-    const int64_t v0 = vox_off[a];
-    const int V = (int)(vox_off[a + 1] - v0);
-    const int w0 = blockIdx.z * MM;
-    const int M = min(nproj[a] - w0, MM);  // projectors of this block (may be <= 0)
-    const int64_t t0 = tab_off[a] + (int64_t)w0 * V;
-    const T *tabs[4] = {table + t0, dtable + t0, dtable + ttot + t0, dtable + 2 * ttot + t0};
+// ---- forces -------------------------------------------------------------
+// E_nl and F_a = 2 sum occ E Re(conj(<p|psi>) <dp/dr|psi>) need four projections
+// per projector: by the table and by its three gradient tables.  They run as
+// one projection with 4 max_m rows per atom (row q max_m + w: table q of
+// projector w) in MT MFMA row tiles over the same voxel chunks as
+// nl_project_kernel, so a psi value is gathered once for all four tables and
+// the tables are read once per 16 columns.  Bound by the gather's latency, as
+// the projection is.  64^3, 64 real FP64 bands, 8 atoms with 9 projectors: the
+// earlier form (one workgroup per atom and band, 36 VALU accumulators a thread,
+// every table re-read for every band) took 113 us; density + forces as one
+// caller's sequence went from 206 to 90 us with this one.
+//
+// The tables are the caller's column-major ones (V_a values per row), so lane
+// group g takes the 16 consecutive voxels 16 g .. 16 g + 15 of a 64-voxel
+// sub-chunk: a lane's A operands of 16 K steps are then contiguous, and the
+// K order of the sum is free as long as A and B agree on it.
 
-    T acc[4][MM][NBG][NC];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int w = 0; w < MM; ++w)
-#pragma unroll
-            for (int b = 0; b < NBG; ++b)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) acc[q][w][b][c] = T(0);
+// Column slice of one launch and the occupations of its bands, by value: no
+// staging buffer, no upload.
+constexpr int kForceBands = 128;
+struct ForceOcc {
+    double occ[kForceBands];
+};
 
-    for (int v = threadIdx.x; v < V; v += NL_THREADS) {
-        const int g = vox_grid[v0 + v];
+// AS consecutive table values from p (aligned to T only)
+template <typename T, int AS>
+__device__ __forceinline__ void load_row(T (&out)[AS], const T *__restrict__ p) {
+    typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+    constexpr int VEC = 16 / sizeof(T);
+#pragma unroll
+    for (int i = 0; i < AS; i += VEC) {
+        const vec_t v = *reinterpret_cast<const vec_t *>(p + i);
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) out[i + c] = v[c];
+    }
+}
+
+// part[(item * 16 MT + r) * ncol + col]: row r of the item's voxels (see above)
+// for the 16 columns of group g (logical block = item slot * groups + g).
+template <typename T, int NC, bool PH, int MT>
+__global__ __launch_bounds__(256) void nl_grad_project_kernel(
+    double *__restrict__ part, const T *__restrict__ psi, int64_t ng, int ncol, int mm,
+    const int *__restrict__ chunk_atom, const int *__restrict__ chunk_v0, const int64_t *__restrict__ vox_off,
+    const int64_t *__restrict__ tab_off, int64_t ttot, const int *__restrict__ nproj,
+    const int *__restrict__ vox_grid, const T *__restrict__ table, const T *__restrict__ dtable,
+    const T *__restrict__ phase, const int *__restrict__ item_order, int groups, int nblk, int per_xcd) {
+    constexpr int AS = MT == 1 ? 16 : (MT <= 4 ? 8 : 4);  // K steps whose A operands are held at once
+    using M = Mfma<T>;
+    using acc_t = typename M::acc_t;
+    __shared__ T stage[4][PJ_SUB][16 + 1];
+    __shared__ double red[4][16 * 16];
+    const int lb = xcd_block(nblk, per_xcd);
+    if (lb < 0) return;  // the whole workgroup
+    const int slot = lb / groups;
+    const int item = item_order[slot];
+    const int c0 = (lb - slot * groups) * 16;
+    const int a = chunk_atom[item];
+    const int64_t vg0 = vox_off[a];
+    const int V = (int)(vox_off[a + 1] - vg0);
+    const int na = nproj[a];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int j = lane & 15, g = lane >> 4;
+    const int vb = chunk_v0[item] + wave * PJ_VPW;
+    // the lane's table row of each tile (row 0 of the table, unused, where there is none)
+    const T *row[MT];
+    bool has[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int r = 16 * mt + j, q = r / mm, w = r - q * mm;
+        has[mt] = q < 4 && w < na;
+        row[mt] = has[mt] && q > 0 ? dtable + (q - 1) * ttot + tab_off[a] + (int64_t)w * V
+                                   : table + tab_off[a] + (has[mt] ? (int64_t)w * V : 0);
+    }
+    acc_t acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = acc_t{0, 0, 0, 0};
+    for (int sc = 0; sc < PJ_VPW / PJ_SUB; ++sc) {
+        const int vs = vb + sc * PJ_SUB;
+        if (vs >= V) break;  // wave-uniform
+        const int v = vs + lane;
+        const bool in = v < V;
+        const int64_t vid = vg0 + (in ? v : 0);
+        const int gi = in ? vox_grid[vid] : 0;
         T cs = T(1), sn = T(0);
         if constexpr (PH) {
-            cs = phase[2 * (v0 + v)];
-            sn = phase[2 * (v0 + v) + 1];
+            cs = phase[2 * vid];
+            sn = phase[2 * vid + 1];
         }
-        T br[NBG], bi[NBG];
+        T gv[16];
 #pragma unroll
-        for (int b = 0; b < NBG; ++b) {
-            const int n = min(n0 + b, nb - 1);
-            T re = psi[(int64_t)n * NC * ng + g];
-            T im = T(0);
-            if constexpr (NC == 2) im = psi[((int64_t)n * NC + 1) * ng + g];
-            br[b] = PH ? cs * re - sn * im : re;
-            bi[b] = PH ? cs * im + sn * re : im;
-        }
+        for (int jj = 0; jj < 16; ++jj)
+            gv[jj] = (in && c0 + jj < ncol) ? psi[(int64_t)(c0 + jj) * ng + gi] : T(0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int w = 0; w < MM; ++w) {
-                const T pv = (w < M) ? tabs[q][(int64_t)w * V + v] : T(0);
-#pragma unroll
-                for (int b = 0; b < NBG; ++b) {
-                    acc[q][w][b][0] += pv * br[b];
-                    if constexpr (NC == 2) acc[q][w][b][1] += pv * bi[b];
-                }
+        for (int jj = 0; jj < 16; jj += NC) {
+            const T re = gv[jj];
+            if constexpr (NC == 2) {
+                const T im = gv[jj + 1];
+                stage[wave][lane][jj] = PH ? cs * re - sn * im : re;
+                stage[wave][lane][jj + 1] = PH ? cs * im + sn * re : im;
+            } else {
+                stage[wave][lane][jj] = re;
             }
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        }
+        // written and read by this wave only (see nl_project_kernel)
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const bool whole = vs + PJ_SUB <= V && na > 0;  // wave-uniform: every row holds the sub-chunk's 64 values
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+        for (int h = 0; h < 16; h += AS) {
+            T av[MT][AS];
+            if (whole) {
 #pragma unroll
-        for (int w = 0; w < MM; ++w)
+                for (int mt = 0; mt < MT; ++mt) {
+                    load_row<T, AS>(av[mt], row[mt] + vs + 16 * g + h);
 #pragma unroll
-            for (int b = 0; b < NBG; ++b)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const double s = wave_sum<T>((double)acc[q][w][b][c]);
-                    if (lane == 0) red[wid][((q * MM + w) * NBG + b) * NC + c] = s;
+                    for (int s = 0; s < AS; ++s) av[mt][s] = has[mt] ? av[mt][s] : T(0);
                 }
-    if (threadIdx.x < 4) tot[threadIdx.x] = 0.0;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double e = 0.0, f[3] = {0.0, 0.0, 0.0};
-        for (int b = 0; b < NBG; ++b) {
-            if (n0 + b >= nb) break;
-            const double o = occ[n0 + b];
-            for (int w = 0; w < M; ++w) {
-                double s[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-                for (int q = 0; q < 4; ++q)
-                    for (int c = 0; c < NC; ++c) {
-                        double t = 0.0;
-                        for (int k = 0; k < NL_THREADS / 64; ++k) t += red[k][((q * MM + w) * NBG + b) * NC + c];
-                        s[q][c] = t * dV;
+            } else {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int s = 0; s < AS; ++s) {
+                        const int vv = vs + 16 * g + h + s;
+                        av[mt][s] = has[mt] && vv < V ? row[mt][vv] : T(0);
                     }
-                const double eo = energy[proj_off[a] + w0 + w] * o;
-                e += (s[0][0] * s[0][0] + s[0][1] * s[0][1]) * eo;
-                for (int d = 0; d < 3; ++d) f[d] += 2.0 * (s[0][0] * s[d + 1][0] + s[0][1] * s[d + 1][1]) * eo;
+            }
+#pragma unroll
+            for (int s = 0; s < AS; ++s) {
+                const T b = stage[wave][16 * g + h + s][j];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[mt] = M::mma(av[mt][s], b, acc[mt]);
             }
         }
-        double *o4 = out + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * natoms + a) * 4;
-        o4[0] = e;
-        o4[1] = f[0];
-        o4[2] = f[1];
-        o4[3] = f[2];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
+    // sum of the four waves in a fixed order
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][M::row(g, r) * 16 + j] = (double)acc[mt][r];
+        __syncthreads();
+        const int e = threadIdx.x;  // 256 = 16 rows x 16 columns
+        const int r = 16 * mt + (e >> 4), col = c0 + (e & 15);
+        if (col < ncol && r < 4 * mm)
+            part[((int64_t)item * (16 * MT) + r) * ncol + col] =
+                (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+        __syncthreads();
+    }
+}
+
+// Per (atom a, group of 16 columns): the chunk partials summed in order, then
+// out[(blockIdx.y * natoms + a) * 4 + {0: E, 1..3: F}] over the group's bands.
+// rows = 16 MT, mm = max_m.
+template <int NC>
+__global__ __launch_bounds__(256) void nl_force_sum_kernel(double *__restrict__ out, const double *__restrict__ part,
+                                                           int ncol, int natoms, int mm, int rows, ForceOcc occ,
+                                                           const int *__restrict__ atom_chunk_off,
+                                                           const int *__restrict__ nproj,
+                                                           const int *__restrict__ proj_off,
+                                                           const double *__restrict__ energy, double dV) {
+    __shared__ double S[4 * kMaxProj][16];
+    __shared__ double red[4][4];
+    const int a = blockIdx.x, c0 = blockIdx.y * 16;
+    const int it0 = atom_chunk_off[a], it1 = atom_chunk_off[a + 1];
+    const int64_t step = (int64_t)rows * ncol;
+    for (int e = threadIdx.x; e < 4 * mm * 16; e += 256) {
+        const int r = e >> 4, cl = e & 15;
+        double s = 0.0;
+        if (c0 + cl < ncol) {
+            const double *src = part + (int64_t)r * ncol + c0 + cl;
+            for (int it = it0; it < it1; it += kCoefLoads) {
+                double v[kCoefLoads];
+#pragma unroll
+                for (int u = 0; u < kCoefLoads; ++u) v[u] = src[min(it + u, it1 - 1) * step];
+#pragma unroll
+                for (int u = 0; u < kCoefLoads; ++u)
+                    if (it + u < it1) s += v[u];
+            }
+        }
+        S[r][cl] = s * dV;
+    }
+    __syncthreads();
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    const int M = nproj[a];
+    for (int e = threadIdx.x; e < M * (16 / NC); e += 256) {
+        const int b = e / M, w = e - b * M;
+        const int cl = b * NC;
+        if (c0 + cl >= ncol) break;  // columns past the slice hold no band
+        const double eo = energy[proj_off[a] + w] * occ.occ[(c0 + cl) / NC];
+        const double pr = S[w][cl], pi = NC == 2 ? S[w][cl + NC - 1] : 0.0;
+        t[0] += (pr * pr + pi * pi) * eo;
+#pragma unroll
+        for (int d = 1; d < 4; ++d) {
+            const double gr = S[d * mm + w][cl], gim = NC == 2 ? S[d * mm + w][cl + NC - 1] : 0.0;
+            t[d] += 2.0 * (pr * gr + pi * gim) * eo;
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const double s = wave_sum<double>(t[d]);
+        if (lane == 0) red[wave][d] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < 4)
+        out[((int64_t)blockIdx.y * natoms + a) * 4 + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 template <typename T>
@@ -620,16 +725,39 @@ int launch_nonlocal(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, const
     return QM_OK;
 }
 
-template <typename T, int MM, int NC, bool PH>
-void launch_force(qm_ctx *ctx, double *out, const T *psi, int nb, const double *d_occ, const T *phase, int nz,
-                  hipStream_t st) {
-    constexpr int NBG = 1;
+template <typename T, int NC, bool PH, int MT>
+void launch_grad_project(qm_ctx *ctx, double *part, const T *psi, int ncol, const T *phase, hipStream_t st) {
     const Projectors &p = ctx->proj;
-    dim3 grid(p.natoms, (nb + NBG - 1) / NBG, nz);
-    hipLaunchKernelGGL((nl_force_kernel<T, MM, NBG, NC, PH>), grid, dim3(NL_THREADS), 0, st, out, psi, ctx->ng, nb,
-                       p.natoms, d_occ, p.d_nproj, p.d_proj_off, p.d_vox_off, p.d_tab_off, p.ttot, p.d_vox_grid,
-                       table_of<T>(p), dtable_of<T>(p), phase, p.d_energy, ctx->hx * ctx->hy * ctx->hz);
+    const int groups = (ncol + 15) / 16;
+    const int64_t nblk = (int64_t)p.nchunk * groups;
+    const int per_xcd = (int)((nblk + 7) / 8);
+    hipLaunchKernelGGL((nl_grad_project_kernel<T, NC, PH, MT>), dim3(8 * per_xcd), dim3(256), 0, st, part, psi,
+                       ctx->ng, ncol, p.max_m, p.d_chunk_atom, p.d_chunk_v0, p.d_vox_off, p.d_tab_off, p.ttot,
+                       p.d_nproj, p.d_vox_grid, table_of<T>(p), dtable_of<T>(p), phase, p.d_item_order, groups,
+                       (int)nblk, per_xcd);
 }
+
+// One slice of bands: the projections, then the sums into out (groups x natoms x 4)
+template <typename T, int NC, bool PH>
+int launch_force(qm_ctx *ctx, double *out, double *part, int mt, const T *psi, int nb, const ForceOcc &occ,
+                 const T *phase, hipStream_t st) {
+    const Projectors &p = ctx->proj;
+    const int ncol = nb * NC;
+    switch (mt) {
+        case 1: launch_grad_project<T, NC, PH, 1>(ctx, part, psi, ncol, phase, st); break;
+        case 3: launch_grad_project<T, NC, PH, 3>(ctx, part, psi, ncol, phase, st); break;
+        case 4: launch_grad_project<T, NC, PH, 4>(ctx, part, psi, ncol, phase, st); break;
+        default: launch_grad_project<T, NC, PH, 8>(ctx, part, psi, ncol, phase, st); break;
+    }
+    QM_HIP(hipGetLastError());
+    hipLaunchKernelGGL((nl_force_sum_kernel<NC>), dim3(p.natoms, (ncol + 15) / 16), dim3(256), 0, st, out, part, ncol,
+                       p.natoms, p.max_m, 16 * mt, occ, p.d_atom_chunk_off, p.d_nproj, p.d_proj_off, p.d_energy,
+                       ctx->hx * ctx->hy * ctx->hz);
+    QM_HIP(hipGetLastError());
+    return QM_OK;
+}
+
+constexpr int64_t kForcePartBytes = (int64_t)128 << 20;  // partial sums of one slice of bands
 
 template <typename T>
 int nonlocal_forces(qm_ctx *ctx, const T *psi, const double *occ, int nb, int ncomp, const KPoint &kp,
@@ -639,45 +767,50 @@ int nonlocal_forces(qm_ctx *ctx, const T *psi, const double *occ, int nb, int nc
     QM_CHECK(ncomp == 1 || ncomp == 2, QM_ERR_ARG, "ncomp must be 1 or 2");
     const bool ph = !kp.gamma;
     QM_CHECK(ncomp == 2 || !ph, QM_ERR_ARG, "real (ncomp=1) bands need a Gamma k-point");
-    // one band per force block (see launch_force); projectors in groups of 16
-    // over blockIdx.z when an atom has more than 16
-    const int nz = p.max_m > 16 ? 2 : 1;
-    const int ngrp = nb * nz;
-    const size_t out_bytes = sizeof(double) * (size_t)ngrp * p.natoms * 4;
-    QM_TRY(ctx->fwork.reserve(out_bytes + sizeof(double) * nb));
-    double *d_out = ctx->fwork.as<double>();
-    double *d_occ = d_out + (size_t)ngrp * p.natoms * 4;
-    QM_HIP(hipMemcpyAsync(d_occ, occ, sizeof(double) * nb, hipMemcpyHostToDevice, st));
+    *e_nl = 0.0;
+    for (int i = 0; i < 3 * p.natoms; ++i) forces[i] = 0.0;
+    if (p.nchunk == 0 || p.max_m == 0) return QM_OK;  // no voxels or no projectors: nothing to sum
+    // MFMA row tiles of the 4 max_m projections (1, 3, 4 or 8 are built: up to
+    // 4, 12, 16 and 32 projectors per atom)
+    const int need = (4 * p.max_m + 15) / 16;
+    const int mt = need <= 1 ? 1 : (need <= 3 ? 3 : (need == 4 ? 4 : 8));
+    // bands per slice: what the partial sums' limit allows, in whole groups of
+    // 16 columns, at most kForceBands
+    const int64_t per_band = (int64_t)p.nchunk * 16 * mt * ncomp * (int64_t)sizeof(double);
+    const int slice = (int)std::max<int64_t>(16, std::min<int64_t>(kForceBands, kForcePartBytes / per_band / 16 * 16));
+    QM_CHECK((int64_t)p.nchunk * ((slice * ncomp + 15) / 16) < (int64_t)INT32_MAX / 16, QM_ERR_ARG,
+             "nonlocal forces: too many projector voxels");
+    const int gmax = (slice * ncomp + 15) / 16;  // column groups of a slice
+    const int nslice = (nb + slice - 1) / slice;
+    const size_t part_bytes = (size_t)per_band * std::min(slice, nb);
+    const size_t out_n = (size_t)nslice * gmax * p.natoms * 4;
+    const size_t part_al = (part_bytes + 255) & ~(size_t)255;
+    QM_TRY(ctx->fwork.reserve(part_al + sizeof(double) * out_n));
+    double *part = ctx->fwork.as<double>();
+    double *d_out = reinterpret_cast<double *>(ctx->fwork.as<unsigned char>() + part_al);
     const T *phase = phase_of<T>(kp);
-    const bool small = p.max_m <= 9;
-    if (ncomp == 1) {
-        if (small) launch_force<T, 9, 1, false>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
-        else launch_force<T, 16, 1, false>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
-    } else if (!ph) {
-        if (small) launch_force<T, 9, 2, false>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
-        else launch_force<T, 16, 2, false>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
-    } else {
-        if (small) launch_force<T, 9, 2, true>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
-        else launch_force<T, 16, 2, true>(ctx, d_out, psi, nb, d_occ, phase, nz, st);
+    size_t used = 0;  // output blocks of 4 natoms values written so far
+    for (int n0 = 0; n0 < nb; n0 += slice) {
+        const int n = std::min(slice, nb - n0);
+        ForceOcc fo;
+        for (int i = 0; i < kForceBands; ++i) fo.occ[i] = i < n ? occ[n0 + i] : 0.0;
+        double *out = d_out + used * p.natoms * 4;
+        const T *src = psi + (int64_t)n0 * ncomp * ctx->ng;
+        if (ncomp == 1) QM_TRY((launch_force<T, 1, false>(ctx, out, part, mt, src, n, fo, phase, st)));
+        else if (!ph) QM_TRY((launch_force<T, 2, false>(ctx, out, part, mt, src, n, fo, phase, st)));
+        else QM_TRY((launch_force<T, 2, true>(ctx, out, part, mt, src, n, fo, phase, st)));
+        used += (n * ncomp + 15) / 16;
     }
-    QM_HIP(hipGetLastError());
-    std::vector<double> h((size_t)ngrp * p.natoms * 4);
-    QM_HIP(hipMemcpyAsync(h.data(), d_out, out_bytes, hipMemcpyDeviceToHost, st));
+    std::vector<double> h(used * p.natoms * 4);
+    QM_HIP(hipMemcpyAsync(h.data(), d_out, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
     double e = 0.0;
-    for (int a = 0; a < p.natoms; ++a) {
-        double f[3] = {0, 0, 0};
-        for (int g = 0; g < ngrp; ++g) {
-            const double *o4 = &h[((size_t)g * p.natoms + a) * 4];
+    for (int a = 0; a < p.natoms; ++a)
+        for (size_t g = 0; g < used; ++g) {
+            const double *o4 = &h[(g * p.natoms + a) * 4];
             e += o4[0];
-            f[0] += o4[1];
-            f[1] += o4[2];
-            f[2] += o4[3];
+            for (int d = 0; d < 3; ++d) forces[3 * a + d] += o4[1 + d];
         }
-        forces[3 * a] = f[0];
-        forces[3 * a + 1] = f[1];
-        forces[3 * a + 2] = f[2];
-    }
     *e_nl = e;
     return QM_OK;
 }

@@ -287,10 +287,10 @@ int band_reduce(DevBuf &part, int mode, double *out0, double *out1, T *r, const 
 template <typename T>
 int scale_bands(T *y, const T *x, const double *f, double fconst, int nb, int ncomp, int64_t ng, hipStream_t st);
 
-// adjoint.hip
-int launch_band_density_f64(const qm_ctx *ctx, double *rho, const double *psi, const double *d_occ,
+// adjoint.hip (occ: host)
+int launch_band_density_f64(const qm_ctx *ctx, double *rho, const double *psi, const double *occ,
                             int nb, int ncomp, hipStream_t st);
-int launch_band_density_f32(const qm_ctx *ctx, double *rho, const float *psi, const double *d_occ,
+int launch_band_density_f32(const qm_ctx *ctx, double *rho, const float *psi, const double *occ,
                             int nb, int ncomp, hipStream_t st);
 
 }  // namespace qm
