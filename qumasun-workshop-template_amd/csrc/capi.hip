@@ -289,7 +289,49 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
             QM_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
             return scatter();
         };
-        if (ctx->stencil_force >= 0 || ctx->kinetic == QM_KINETIC_FFT) return overlapped();
+        // mean time of `reps` applies after a warm-up
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        int status = QM_OK;
+        auto timed = [&](auto &&run, int reps) -> float {
+            float ms = 0.0f;
+            status = run();
+            if (status == QM_OK && hipEventRecord(ev[0], st) != hipSuccess) status = QM_ERR_HIP;
+            for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
+            if (status == QM_OK && hipEventRecord(ev[1], st) != hipSuccess) status = QM_ERR_HIP;
+            if (status == QM_OK && hipEventSynchronize(ev[1]) != hipSuccess) status = QM_ERR_HIP;
+            if (status == QM_OK && hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) status = QM_ERR_HIP;
+            return ms / (float)reps;
+        };
+        struct Events {
+            hipEvent_t *e;
+            int create() {
+                QM_HIP(hipEventCreate(&e[0]));
+                QM_HIP(hipEventCreate(&e[1]));
+                return QM_OK;
+            }
+            ~Events() {
+                for (int i = 0; i < 2; ++i)
+                    if (e[i]) (void)hipEventDestroy(e[i]);
+            }
+        } events{ev};
+        if (ctx->kinetic == QM_KINETIC_FFT) {
+            // the spectral kernels have one shape: only the schedule is timed
+            const int64_t key = stencil_full_key(prec, ncomp, kt, nb) | ((int64_t)1 << 59);
+            auto it = ctx->apply_overlapped.find(key);
+            if (it == ctx->apply_overlapped.end()) {
+                if (capturing || g_internal_capture) return overlapped();
+                QM_TRY(in_order());  // the projection's shape is tuned alone first
+                QM_TRY(events.create());
+                const float ms = timed(in_order, 3);
+                bool beside = false;
+                if (status == QM_OK && ms > kOverlapMinMs) beside = timed(overlapped, 3) < ms;
+                if (status == QM_ERR_HIP) set_error("H.psi schedule tuning: HIP event failure");
+                if (status != QM_OK) return status;
+                it = ctx->apply_overlapped.emplace(key, beside).first;
+            }
+            return it->second ? overlapped() : in_order();
+        }
+        if (ctx->stencil_force >= 0) return overlapped();
         // The schedule, and the stencil's tile shape in it, are tuned on full
         // applies: the shape that runs fastest alone is not always the one
         // that leaves the projection the most room beside it.  Every choice
@@ -314,24 +356,7 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 QM_TRY(in_order());
                 const int alone = stencil_choice(ctx, prec, ncomp, kt, nb);
                 QM_CHECK(alone >= 0, QM_ERR_STATE, "H.psi shape tuning: no local shape");
-                hipEvent_t ev[2] = {nullptr, nullptr};
-                QM_HIP(hipEventCreate(&ev[0]));
-                if (hipEventCreate(&ev[1]) != hipSuccess) {
-                    (void)hipEventDestroy(ev[0]);
-                    QM_CHECK(false, QM_ERR_HIP, "hipEventCreate failed");
-                }
-                int status = QM_OK;
-                // mean of `reps` applies after a warm-up
-                auto timed = [&](auto &&run, int reps) -> float {
-                    float ms = 0.0f;
-                    status = run();
-                    if (status == QM_OK && hipEventRecord(ev[0], st) != hipSuccess) status = QM_ERR_HIP;
-                    for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
-                    if (status == QM_OK && hipEventRecord(ev[1], st) != hipSuccess) status = QM_ERR_HIP;
-                    if (status == QM_OK && hipEventSynchronize(ev[1]) != hipSuccess) status = QM_ERR_HIP;
-                    if (status == QM_OK && hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) status = QM_ERR_HIP;
-                    return ms / (float)reps;
-                };
+                QM_TRY(events.create());
                 cand = alone;
                 beside = false;
                 ctx->stencil_force = alone;
@@ -348,8 +373,6 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                         }
                     }
                 }
-                (void)hipEventDestroy(ev[0]);
-                (void)hipEventDestroy(ev[1]);
                 if (status == QM_ERR_HIP) set_error("H.psi shape tuning: HIP event failure");
                 if (status != QM_OK) return status;
                 ctx->stencil_choice[key] = cand;

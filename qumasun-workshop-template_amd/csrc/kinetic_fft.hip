@@ -8,7 +8,9 @@
 //   psi <- IFFT( e^{-i dt |G + k|^2 / 2} FFT psi ) / N
 // (EvolveKineticInKspace / mEvolveK_FFT, qumasun_symplectic.kinetic_fft.h:14-60, 65-140).
 //
-// GPU structure: rocFFT batched 3-D transforms.  Complex bands are packed
+// GPU structure: the kinetic operator and propagator run as the plane and line
+// kernels of spectral.hip.  The rocFFT batched 3-D transforms here serve the
+// Poisson solve and the grids those kernels do not take.  Complex bands are packed
 // from the SoA (re, im) arrays into one interleaved block (the reference's
 // GatherExchangeD2Z, without the DDM exchange) and transformed in place; the
 // unpack after the inverse transform is fused with V_loc psi.  Real
@@ -290,9 +292,21 @@ void launch_kspace(qm_ctx *ctx, C2<T> *spec, int64_t per_band, int nb, int ncomp
                        ctx->nx, ctx->ny, ctx->nz, gx, gy, gz, k[0], k[1], k[2], 1.0 / (double)ctx->ng, dt);
 }
 
+// The tables of the plane and line kernels (spectral.hip), null where the
+// library transforms below run instead: a grid those kernels do not take, or
+// tables that do not exist yet inside a capture.
+template <typename T>
+int own_tables(qm_ctx *ctx, hipStream_t st, SpectralTables **t) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    QM_HIP(hipStreamIsCapturing(st, &cs));
+    return spectral_tables<T>(ctx, cs != hipStreamCaptureStatusNone || g_internal_capture, t);
+}
+
 }  // namespace
 
 void fft_destroy(qm_ctx *ctx) {
+    spectral_destroy(ctx->spectral);
+    ctx->spectral = nullptr;
     if (!ctx->fft) return;
     for (auto &kv : ctx->fft->plans) destroy_pair(kv.second);
     ctx->fft->spec.release();
@@ -306,6 +320,9 @@ template <typename T>
 int launch_fft_local(qm_ctx *ctx, T *out, const T *psi, int nb, int ncomp, const double k[3], hipStream_t st) {
     const bool kt = k[0] != 0.0 || k[1] != 0.0 || k[2] != 0.0;
     QM_CHECK(ncomp == 2 || !kt, QM_ERR_ARG, "real (ncomp=1) bands need a Gamma k-point");
+    SpectralTables *t = nullptr;
+    QM_TRY(own_tables<T>(ctx, st, &t));
+    if (t) return spectral_kinetic<T>(ctx, t, out, psi, nb, ncomp, k, st);
     FftPair *pair = nullptr;
     C2<T> *spec = nullptr;
     int64_t pb = 0;
@@ -327,6 +344,9 @@ template int launch_fft_local<float>(qm_ctx *, float *, const float *, int, int,
 // psi <- IFFT(e^{-i dt |G + k|^2 / 2} FFT psi) / N, SoA complex bands
 template <typename T>
 int fft_kinetic_step(qm_ctx *ctx, T *psi, int nb, const double k[3], double dt, hipStream_t st) {
+    SpectralTables *t = nullptr;
+    QM_TRY(own_tables<T>(ctx, st, &t));
+    if (t) return spectral_step<T>(ctx, t, psi, nb, k, dt, st);
     FftPair *pair = nullptr;
     C2<T> *spec = nullptr;
     int64_t pb = 0;

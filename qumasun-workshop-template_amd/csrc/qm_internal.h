@@ -104,7 +104,8 @@ struct Projectors {
 };
 
 
-struct FftState;  // rocFFT plans and buffers of the spectral kinetic term (kinetic_fft.hip)
+struct FftState;  // rocFFT plans and buffers (kinetic_fft.hip)
+struct SpectralTables;  // axis tables of the spectral kinetic kernels (spectral.hip)
 
 struct KPoint {
     double k[3] = {0, 0, 0};
@@ -150,7 +151,8 @@ struct qm_ctx {
     // (QM_ERR_STATE) until qm_release_captures.
     int capture_pins = 0;
     int kinetic = QM_KINETIC_FD8;  // kinetic term of every apply (qm_set_kinetic)
-    qm::FftState *fft = nullptr;   // created on the first spectral apply
+    qm::FftState *fft = nullptr;   // created on the first library transform
+    qm::SpectralTables *spectral = nullptr;  // created on the first spectral apply
 };
 
 namespace qm {
@@ -233,6 +235,21 @@ int subspace_route();
 template <typename T>
 int launch_fft_local(qm_ctx *ctx, T *out, const T *psi, int nb, int ncomp, const double k[3], hipStream_t st);
 void fft_destroy(qm_ctx *ctx);
+
+// spectral.hip: the kinetic operator and propagator as one plane and one line
+// kernel.  spectral_tables: the context's tables, null where the grid does not
+// fit them (a prime factor above 13, or a plane larger than the LDS)
+template <typename T>
+int spectral_tables(qm_ctx *ctx, bool capturing, SpectralTables **out);
+// out = kinetic psi + V_loc psi (overwrites)
+template <typename T>
+int spectral_kinetic(const qm_ctx *ctx, const SpectralTables *t, T *out, const T *psi, int nb, int ncomp,
+                     const double k[3], hipStream_t st);
+// psi <- e^{-i dt |G + k|^2 / 2} psi, SoA complex bands
+template <typename T>
+int spectral_step(const qm_ctx *ctx, const SpectralTables *t, T *psi, int nb, const double k[3], double dt,
+                  hipStream_t st);
+void spectral_destroy(SpectralTables *t);
 
 // nonlocal.hip
 int launch_nonlocal_f64(qm_ctx *ctx, double *hpsi, const double *psi, int nb, int ncomp,
