@@ -141,6 +141,7 @@ struct qm_ctx {
     qm::DevBuf eig_work;                    // qm_sygvd_f64 workspace
     qm::DevBuf td_work;                     // two band blocks of the Taylor propagator
     qm::DevBuf scf_part;                    // partial sums of qm_grid_dot_f64
+    double *h_dot = nullptr;                // its result: pinned host memory the device writes
     // second stream of a full H.psi apply: the nonlocal projection runs on it
     // beside the stencil, joined by events (created on first use)
     hipStream_t side = nullptr;

@@ -6,7 +6,7 @@
 //   - integrals over the grid, sum_i a_i b_i, in a fixed summation order (the
 //     energy terms of mGetTotalEnergy, qumasun_base1.energy.h:19-160);
 //   - density mixing (MixingSimple and MixingDIIS, mixing_simple.h:45-75,
-//     mixing_DIIS.h:48-229) on device fields, the small DIIS matrix on the host;
+//     mixing_DIIS.h:48-229) on device fields and matrix;
 //   - occupations (mSetOccupancyZero / mSetOccupancyTemperature,
 //     qumasun_base1.occupancy.h:35-175 with SetOccupancy.h), host code.
 // The Hartree potential (FFT Poisson solve) is in kinetic_fft.hip.
@@ -26,9 +26,10 @@ struct qm_mixer {
     int64_t n = 0;
     double *rho = nullptr;  // DIIS: hist fields; simple: the previous field
     double *R = nullptr;    // DIIS residual fields
-    double *part = nullptr; // per-block partial sums (kMixBlocks x (hist + 1))
-    double *coef = nullptr; // DIIS coefficients (hist)
-    std::vector<double> M;  // (hist + 1)^2 bordered R.R matrix, column-major
+    double *part = nullptr; // per-block partial sums (kRedBlocks x (hist + 1))
+    double *coef = nullptr; // DIIS coefficients (hist + 1)
+    double *M = nullptr;    // (hist + 1)^2 bordered R.R matrix, column-major, and 2 (hist + 1)^2 of work
+    double *h_diff = nullptr;  // pinned host memory: sum |R| of the last step, written by the device
 };
 
 namespace qm {
@@ -87,25 +88,138 @@ __global__ __launch_bounds__(kRedThreads) void reduce_kernel(const double *__res
     }
 }
 
-// R = out - rho_k and part = per-block sums of |R|
-__global__ __launch_bounds__(kRedThreads) void residual_kernel(double *__restrict__ R, const double *__restrict__ out,
-                                                               const double *__restrict__ rk, int64_t n,
-                                                               double *__restrict__ part) {
-    __shared__ double red[kRedThreads / 64];
-    double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (int64_t)kRedBlocks * kRedThreads) {
-        const double g = out[i] - rk[i];
-        R[i] = g;
-        s += fabs(g);
+// Sums of N per-thread values over the workgroup, in a fixed order, to dst[q * kRedBlocks]
+template <int N>
+__device__ __forceinline__ void block_sums(double (&s)[N], int count, double *__restrict__ dst) {
+    __shared__ double red[kRedThreads / 64][N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        for (int m = 32; m >= 1; m >>= 1) s[q] += __shfl_xor(s[q], m);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][q] = s[q];
     }
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if ((int)threadIdx.x < count) {
         double t = 0.0;
-        for (int w = 0; w < kRedThreads / 64; ++w) t += red[w];
-        part[blockIdx.x] = t;
+        for (int w = 0; w < kRedThreads / 64; ++w) t += red[w][threadIdx.x];
+        dst[(size_t)threadIdx.x * kRedBlocks + blockIdx.x] = t;
     }
+}
+
+// DIIS residual and its overlaps in one pass over the history: R_k = out -
+// rho_k, per-block sums of |R_k|, R_k . R_k and R_k . R_m for up to kDotFields
+// older residuals (HBM bound; one kernel for each overlap read R_k again each
+// time: 10 launches of 3 us at 64^3 with 9 fields, now one of 11 us).
+// FIRST false: further residuals of a longer history, R_k read back.
+constexpr int kDotFields = 8;
+struct DotFields {
+    const double *f[kDotFields];
+};
+template <bool FIRST>
+__global__ __launch_bounds__(kRedThreads) void residual_dots_kernel(double *__restrict__ Rk,
+                                                                    const double *__restrict__ out,
+                                                                    const double *__restrict__ rk, DotFields fields,
+                                                                    int nf, int64_t n, double *__restrict__ part) {
+    constexpr int B = FIRST ? 2 : 0;
+    double s[kDotFields + B];
+#pragma unroll
+    for (int q = 0; q < kDotFields + B; ++q) s[q] = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (int64_t)kRedBlocks * kRedThreads) {
+        double g;
+        if constexpr (FIRST) {
+            g = out[i] - rk[i];
+            Rk[i] = g;
+            s[0] += fabs(g);
+            s[1] += g * g;
+        } else {
+            g = Rk[i];
+        }
+#pragma unroll
+        for (int q = 0; q < kDotFields; ++q)
+            if (q < nf) s[B + q] += g * fields.f[q][i];
+    }
+    block_sums<kDotFields + B>(s, nf + B, part);
+}
+
+// out[q] = the kRedBlocks partials of sum q, added in order, for q < count <=
+// kSumRows (rows staged through LDS: the adds are a serial chain).  One
+// workgroup of kRedThreads.
+constexpr int kSumRows = 10;
+__device__ __forceinline__ void sum_rows(const double *__restrict__ part, int count, double *out) {
+    __shared__ double rows[kSumRows][kRedBlocks];
+    __syncthreads();
+    for (int i = threadIdx.x; i < count * kRedBlocks; i += kRedThreads) rows[i / kRedBlocks][i % kRedBlocks] = part[i];
+    __syncthreads();
+    if ((int)threadIdx.x < count) {
+        double t = 0.0;
+#pragma unroll 16
+        for (int b = 0; b < kRedBlocks; ++b) t += rows[threadIdx.x][b];
+        out[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(kRedThreads) void sum_kernel(double *__restrict__ out, const double *__restrict__ part) {
+    sum_rows(part, 1, out);
+}
+
+// After residual_dots_kernel: *diff = sum |R_k| (pinned host memory), row and
+// column k of the bordered overlap matrix M (L = hist + 1, column-major) and,
+// when the ring is full, the mixing coefficients c = the bordering row of M^-1
+// by the Gauss-Jordan elimination without pivoting of InverseM
+// (inverse_m.h:17-60), every element's operations in that routine's order and
+// unfused.  One workgroup: the matrix is at most 65 x 65, and a round trip to
+// the host between the overlaps and the mixing cost more than the elimination
+// (15 us at history 9; the copies and the
+// synchronisation it replaces ~30 us).  Mixing, Hartree, LDA and two integrals as
+// one caller's sequence at 64^3: 217 -> 137 us with the pinned results below.
+struct DiisSlots {
+    int m[64];  // history slot of each overlap; m[0] = k
+};
+constexpr int kLdsOrder = 32;  // largest L whose elimination runs in LDS
+__global__ __launch_bounds__(kRedThreads) void diis_coef_kernel(double *__restrict__ diff, double *__restrict__ c,
+                                                                double *M, const double *__restrict__ part,
+                                                                DiisSlots slots, int ndot, int L, int full) {
+#pragma clang fp contract(off)
+    __shared__ double lds[2 * kLdsOrder * kLdsOrder], sums[64 + 1], col[64 + 1];
+    const int H = L - 1, k = slots.m[0], tid = threadIdx.x;
+    for (int q = 0; q <= ndot; q += kSumRows)
+        sum_rows(part + (size_t)q * kRedBlocks, min(kSumRows, ndot + 1 - q), sums + q);
+    if (tid == 0) *diff = sums[0];
+    for (int q = tid; q < ndot; q += kRedThreads) M[slots.m[q] + L * k] = sums[q + 1];
+    __syncthreads();
+    for (int j = tid; j < H; j += kRedThreads) {
+        if (j != k) M[k + L * j] = M[j + L * k];
+        M[H + L * j] = 1.0;
+        M[j + L * H] = 1.0;
+    }
+    if (tid == 0) M[H + L * H] = 0.0;
+    __syncthreads();
+    if (!full) return;
+    double *m = L <= kLdsOrder ? lds : M + L * L, *inv = m + L * L;
+    for (int e = tid; e < L * L; e += kRedThreads) {
+        m[e] = M[e];
+        inv[e] = e % L == e / L ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    for (int i = 0; i < L; ++i) {
+        const double b = 1.0 / m[i + L * i];
+        for (int j = tid; j < L; j += kRedThreads) col[j] = m[j + L * i];  // the multipliers of this step
+        __syncthreads();
+        if (isfinite(b))
+            for (int j = tid; j < L; j += kRedThreads) {
+                m[i + L * j] *= b;
+                inv[i + L * j] *= b;
+            }
+        __syncthreads();
+        for (int e = tid; e < L * L; e += kRedThreads) {
+            const int j = e % L, q = e / L;
+            if (j == i) continue;
+            m[j + L * q] -= m[i + L * q] * col[j];
+            inv[j + L * q] -= inv[i + L * q] * col[j];
+        }
+        __syncthreads();
+    }
+    for (int j = tid; j < L; j += kRedThreads) c[j] = inv[H + L * j];
 }
 
 // simple mixing: out = (out - prev) ratio + prev; prev = out
@@ -154,45 +268,10 @@ inline unsigned grid_for(int64_t n) {
     return (unsigned)std::min<int64_t>(std::max<int64_t>((n + 255) / 256, 1), 4096);
 }
 
-// sum of the kRedBlocks partials in order (on the host)
-int sum_partials(const double *d_part, int count, double *out, hipStream_t st) {
-    std::vector<double> h((size_t)count * kRedBlocks);
-    QM_HIP(hipMemcpyAsync(h.data(), d_part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
-    QM_HIP(hipStreamSynchronize(st));
-    for (int c = 0; c < count; ++c) {
-        double t = 0.0;
-        for (int b = 0; b < kRedBlocks; ++b) t += h[(size_t)c * kRedBlocks + b];
-        out[c] = t;
-    }
-    return QM_OK;
-}
-
-// Gauss-Jordan inverse without pivoting of the column-major n x n m (destroyed),
-// as InverseM (inverse_m.h:17-60)
-void inverse_m(std::vector<double> &m, int n, std::vector<double> &inv) {
-    inv.assign((size_t)n * n, 0.0);
-    for (int i = 0; i < n; ++i) inv[i + (size_t)i * n] = 1.0;
-    for (int i = 0; i < n; ++i) {
-        const double b = 1.0 / m[i + (size_t)i * n];
-        if (std::isfinite(b))
-            for (int j = 0; j < n; ++j) {
-                m[i + (size_t)j * n] *= b;
-                inv[i + (size_t)j * n] *= b;
-            }
-        for (int j = 0; j < n; ++j) {
-            if (j == i) continue;
-            const double b2 = m[j + (size_t)i * n];
-            for (int k = 0; k < n; ++k) {
-                m[j + (size_t)k * n] -= m[i + (size_t)k * n] * b2;
-                inv[j + (size_t)k * n] -= inv[i + (size_t)k * n] * b2;
-            }
-        }
-    }
-}
-
 void mixer_free(qm_mixer *m) {
-    for (double **p : {&m->rho, &m->R, &m->part, &m->coef})
+    for (double **p : {&m->rho, &m->R, &m->part, &m->coef, &m->M})
         if (*p) (void)hipFree(*p);
+    if (m->h_diff) (void)hipHostFree(m->h_diff);
 }
 
 }  // namespace
@@ -219,7 +298,14 @@ int qm_grid_dot_f64(qm_ctx *ctx, const double *d_a, const double *d_b, double *r
     hipLaunchKernelGGL(reduce_kernel<0>, dim3(kRedBlocks), dim3(kRedThreads), 0, st, d_a, d_b, ctx->ng,
                        ctx->scf_part.as<double>());
     QM_HIP(hipGetLastError());
-    return sum_partials(ctx->scf_part.as<double>(), 1, result, st);
+    // the device writes the sum to pinned host memory: no copy back through a
+    // staging buffer
+    if (!ctx->h_dot) QM_HIP(hipHostMalloc((void **)&ctx->h_dot, sizeof(double), hipHostMallocDefault));
+    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(kRedThreads), 0, st, ctx->h_dot, ctx->scf_part.as<double>());
+    QM_HIP(hipGetLastError());
+    QM_HIP(hipStreamSynchronize(st));
+    *result = *ctx->h_dot;
+    return QM_OK;
 }
 
 int qm_mixer_create(qm_mixer **out, qm_ctx *ctx, int mode, int history, double ratio) {
@@ -241,13 +327,14 @@ int qm_mixer_create(qm_mixer **out, qm_ctx *ctx, int mode, int history, double r
     if (e == hipSuccess && mode == QM_MIX_DIIS) e = hipMalloc((void **)&m->R, fb);
     if (e == hipSuccess) e = hipMalloc((void **)&m->part, sizeof(double) * kRedBlocks * (m->hist + 1));
     if (e == hipSuccess) e = hipMalloc((void **)&m->coef, sizeof(double) * (m->hist + 1));
+    if (e == hipSuccess) e = hipMalloc((void **)&m->M, sizeof(double) * 3 * (m->hist + 1) * (m->hist + 1));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&m->h_diff, sizeof(double), hipHostMallocDefault);
     if (e != hipSuccess) {
         mixer_free(m);
         delete m;
         set_error("qm_mixer_create: hipMalloc failed");
         return QM_ERR_NOMEM;
     }
-    m->M.assign((size_t)(m->hist + 1) * (m->hist + 1), 0.0);
     *out = m;
     return QM_OK;
 }
@@ -266,9 +353,9 @@ int qm_mixer_init(qm_mixer *m, const double *d_rho, void *stream) {
     if (m->mode == QM_MIX_DIIS) {
         QM_HIP(hipMemsetAsync(m->rho, 0, fb * m->hist, st));
         QM_HIP(hipMemsetAsync(m->R, 0, fb * m->hist, st));
+        QM_HIP(hipMemsetAsync(m->M, 0, sizeof(double) * (m->hist + 1) * (m->hist + 1), st));
     }
     QM_HIP(hipMemcpyAsync(m->rho, d_rho, fb, hipMemcpyDeviceToDevice, st));
-    std::fill(m->M.begin(), m->M.end(), 0.0);
     m->step = 0;
     m->ready = true;
     return QM_OK;
@@ -280,14 +367,15 @@ int qm_mixer_predict(qm_mixer *m, double *d_rho, double *diff, void *stream) {
     QM_TRY(activate(m->ctx));
     hipStream_t st = (hipStream_t)stream;
     const int64_t n = m->n;
-    double d = 0.0;
     if (m->mode == QM_MIX_SIMPLE) {
         hipLaunchKernelGGL(reduce_kernel<1>, dim3(kRedBlocks), dim3(kRedThreads), 0, st, d_rho, m->rho, n, m->part);
         QM_HIP(hipGetLastError());
         hipLaunchKernelGGL(mix_simple_kernel, dim3(grid_for(n)), dim3(256), 0, st, d_rho, m->rho, m->ratio, n);
         QM_HIP(hipGetLastError());
-        QM_TRY(sum_partials(m->part, 1, &d, st));
-        if (diff) *diff = d;
+        hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(kRedThreads), 0, st, m->h_diff, m->part);
+        QM_HIP(hipGetLastError());
+        QM_HIP(hipStreamSynchronize(st));
+        if (diff) *diff = *m->h_diff;
         ++m->step;
         return QM_OK;
     }
@@ -295,43 +383,36 @@ int qm_mixer_predict(qm_mixer *m, double *d_rho, double *diff, void *stream) {
     auto idx = [H](int s) { return (s % H + H) % H; };
     const int k = idx(m->step);
     double *rk = m->rho + (int64_t)k * n, *Rk = m->R + (int64_t)k * n;
-    hipLaunchKernelGGL(residual_kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, st, Rk, d_rho, rk, n, m->part);
-    QM_HIP(hipGetLastError());
-    // R_k . R_m over the valid history
-    const int m_end = std::max(m->step - H + 1, 0);
-    std::vector<int> ms;
-    for (int m1 = m->step; m1 >= m_end; --m1) ms.push_back(idx(m1));
-    for (size_t q = 0; q < ms.size(); ++q) {
-        hipLaunchKernelGGL(reduce_kernel<0>, dim3(kRedBlocks), dim3(kRedThreads), 0, st, Rk,
-                           m->R + (int64_t)ms[q] * n, n, m->part + (size_t)(q + 1) * kRedBlocks);
+    // R_k . R_m over the valid history, newest (R_k itself) first
+    DiisSlots slots;
+    int ndot = 0;
+    for (int m1 = m->step; m1 >= std::max(m->step - H + 1, 0); --m1) slots.m[ndot++] = idx(m1);
+    for (int q = 1; q < ndot || q == 1; q += kDotFields) {
+        DotFields f = {};
+        const int nf = std::min(kDotFields, ndot - q);
+        for (int u = 0; u < nf; ++u) f.f[u] = m->R + (int64_t)slots.m[q + u] * n;
+        if (q == 1)
+            hipLaunchKernelGGL(residual_dots_kernel<true>, dim3(kRedBlocks), dim3(kRedThreads), 0, st, Rk, d_rho, rk,
+                               f, nf, n, m->part);
+        else
+            hipLaunchKernelGGL(residual_dots_kernel<false>, dim3(kRedBlocks), dim3(kRedThreads), 0, st, Rk, d_rho, rk,
+                               f, nf, n, m->part + (size_t)(q + 1) * kRedBlocks);
         QM_HIP(hipGetLastError());
     }
-    std::vector<double> sums(ms.size() + 1);
-    QM_TRY(sum_partials(m->part, (int)ms.size() + 1, sums.data(), st));
-    d = sums[0];
-    for (size_t q = 0; q < ms.size(); ++q) m->M[ms[q] + (size_t)L * k] = sums[q + 1];
-    for (int j = 0; j < H; ++j) {
-        m->M[k + (size_t)L * j] = m->M[j + (size_t)L * k];
-        m->M[H + (size_t)L * j] = 1.0;
-        m->M[j + (size_t)L * H] = 1.0;
-    }
-    m->M[H + (size_t)L * H] = 0.0;
     const int nxt = idx(m->step + 1);
-    if (m->step + 1 >= H) {
-        std::vector<double> cp(m->M), inv;
-        inverse_m(cp, L, inv);
-        std::vector<double> c(L);
-        for (int j = 0; j < L; ++j) c[j] = inv[H + (size_t)L * j];  // the bordering row
-        QM_HIP(hipMemcpyAsync(m->coef, c.data(), sizeof(double) * L, hipMemcpyHostToDevice, st));
+    const bool full = m->step + 1 >= H;
+    hipLaunchKernelGGL(diis_coef_kernel, dim3(1), dim3(kRedThreads), 0, st, m->h_diff, m->coef, m->M, m->part, slots,
+                       ndot, L, full ? 1 : 0);
+    QM_HIP(hipGetLastError());
+    if (full)
         hipLaunchKernelGGL(mix_diis_kernel, dim3(grid_for(n)), dim3(256), 0, st, d_rho, m->rho, m->R, m->coef, H,
                            nxt, m->ratio, n);
-    } else {
+    else
         hipLaunchKernelGGL(mix_first_kernel, dim3(grid_for(n)), dim3(256), 0, st, d_rho, m->rho + (int64_t)nxt * n,
                            rk, Rk, m->ratio, n);
-    }
     QM_HIP(hipGetLastError());
-    QM_HIP(hipStreamSynchronize(st));  // the coefficient upload reads host memory
-    if (diff) *diff = d;
+    QM_HIP(hipStreamSynchronize(st));
+    if (diff) *diff = *m->h_diff;
     ++m->step;
     return QM_OK;
 }
