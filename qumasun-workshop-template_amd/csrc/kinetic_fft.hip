@@ -9,8 +9,8 @@
 // (EvolveKineticInKspace / mEvolveK_FFT, qumasun_symplectic.kinetic_fft.h:14-60, 65-140).
 //
 // GPU structure: the kinetic operator and propagator run as the plane and line
-// kernels of spectral.hip.  The rocFFT batched 3-D transforms here serve the
-// Poisson solve and the grids those kernels do not take.  Complex bands are packed
+// kernels of spectral.hip, the Poisson solve as three kernels there.  The rocFFT
+// batched 3-D transforms here serve the grids those kernels do not take.  Complex bands are packed
 // from the SoA (re, im) arrays into one interleaved block (the reference's
 // GatherExchangeD2Z, without the DDM exchange) and transformed in place; the
 // unpack after the inverse transform is fused with V_loc psi.  Real
@@ -361,6 +361,14 @@ int fft_kinetic_step(qm_ctx *ctx, T *psi, int nb, const double k[3], double dt, 
 // mSetPotentialVhart (qumasun_base1.potential.h:32-116), without the
 // refined-grid up/down conversion.  rho and V_H are FP64 grid fields.
 int fft_poisson(qm_ctx *ctx, const double *rho, double *vh, hipStream_t st) {
+    SpectralTables *t = nullptr;
+    QM_TRY(own_tables<double>(ctx, st, &t));
+    const size_t need = sizeof(C2<double>) * (size_t)ctx->ng;
+    if (t && (ctx->capture_pins == 0 || (ctx->fft && ctx->fft->spec.bytes >= need))) {
+        if (!ctx->fft) ctx->fft = new FftState();
+        QM_TRY(ctx->fft->spec.reserve(need));
+        return spectral_poisson(ctx, t, ctx->fft->spec.p, vh, rho, st);
+    }
     FftPair *pair = nullptr;
     C2<double> *spec = nullptr;
     int64_t pb = 0;

@@ -250,6 +250,9 @@ int spectral_kinetic(const qm_ctx *ctx, const SpectralTables *t, T *out, const T
 template <typename T>
 int spectral_step(const qm_ctx *ctx, const SpectralTables *t, T *psi, int nb, const double k[3], double dt,
                   hipStream_t st);
+// V_H = IFFT(4 pi / |G|^2 FFT rho) / N without G = 0; spec: ng complex values of work
+int spectral_poisson(const qm_ctx *ctx, const SpectralTables *t, void *spec, double *vh, const double *rho,
+                     hipStream_t st);
 void spectral_destroy(SpectralTables *t);
 
 // nonlocal.hip

@@ -377,6 +377,139 @@ __global__ __launch_bounds__(256) void spectral_line_kernel(T *out, const T *psi
     }
 }
 
+// ---- Poisson solve ---------------------------------------------------------
+// 4 pi / |G|^2 is no sum over the axes, so the spectrum of the one real FP64
+// field goes through memory, and three kernels take the place of a library
+// transform pair and the scaling pass.  Latency bound (64^3 is 4 MB of spectrum):
+// 28 us of kernels for 31, two launches fewer, and the first solve of a context
+// builds small tables instead of library plans (4.4 -> 0.35 ms for the fields'
+// first pass); the fields' sequence 137 -> 125 us.
+
+// spec plane z = F_xy of real plane z, in the transforms' output positions
+template <bool BIG>
+__global__ __launch_bounds__(1024) void poisson_forward_kernel(Cx<double> *__restrict__ spec,
+                                                               const double *__restrict__ rho,
+                                                               const Cx<double> *__restrict__ twt, int pitch, Axis ax,
+                                                               Axis ay) {
+    using T = double;
+    extern __shared__ __align__(16) unsigned char spectral_lds[];
+    Cx<T> *twx = reinterpret_cast<Cx<T> *>(spectral_lds), *twy = twx + ax.n, *s = twy + ay.n;
+    const int nx = ax.n, ny = ay.n, plane = nx * ny;
+    const int64_t base = (int64_t)blockIdx.x * plane;
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) twx[i] = twt[ax.off + i];
+    for (int i = threadIdx.x; i < ny; i += blockDim.x) twy[i] = twt[ay.off + i];
+    __syncthreads();
+    auto ldg = [&](int c, int e) -> Cx<T> { return {rho[base + e * nx + c], 0.0}; };
+    auto ldy = [&](int c, int e) { return s[e * pitch + c]; };
+    auto sty = [&](int c, int e, Cx<T> v) { s[e * pitch + c] = v; };
+    auto ldx = [&](int c, int e) { return s[c * pitch + e]; };
+    auto stx = [&](int c, int e, Cx<T> v) { s[c * pitch + e] = v; };
+    int L = ny;
+    for (int q = 0; q < ay.ns; ++q) {
+        if (q == 0) stage<T, BIG, false>(ay.r[q], ldg, sty, nx, ny, L, twy);
+        else stage<T, BIG, false>(ay.r[q], ldy, sty, nx, ny, L, twy);
+        L /= ay.r[q];
+        __syncthreads();
+    }
+    L = nx;
+    for (int q = 0; q < ax.ns; ++q) {
+        stage<T, BIG, false>(ax.r[q], ldx, stx, ny, nx, L, twx);
+        L /= ax.r[q];
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < plane; i += blockDim.x) {
+        const int y = (unsigned)i / (unsigned)nx;
+        spec[base + i] = s[y * pitch + i - y * nx];
+    }
+}
+
+// C lines along z of the spectrum: forward, 4 pi / |G|^2 / N (0 at G = 0), back
+template <bool BIG>
+__global__ __launch_bounds__(256) void poisson_line_kernel(Cx<double> *__restrict__ spec,
+                                                           const Cx<double> *__restrict__ twt,
+                                                           const int *__restrict__ freq, int plane, int C, Axis ax,
+                                                           Axis ay, Axis az, double scale) {
+    using T = double;
+    extern __shared__ __align__(16) unsigned char spectral_lds[];
+    Cx<T> *tw = reinterpret_cast<Cx<T> *>(spectral_lds), *s = tw + az.n;
+    const int n = az.n, p0 = blockIdx.x * C, nc = min(C, plane - p0);
+    for (int i = threadIdx.x; i < n; i += blockDim.x) tw[i] = twt[az.off + i];
+    __syncthreads();
+    auto ldg = [&](int c, int e) -> Cx<T> {
+        return c < nc ? spec[(int64_t)e * plane + p0 + c] : Cx<T>{0.0, 0.0};
+    };
+    auto stg = [&](int c, int e, Cx<T> v) {
+        if (c < nc) spec[(int64_t)e * plane + p0 + c] = v;
+    };
+    auto lds = [&](int c, int e) { return s[e * C + c]; };
+    auto sts = [&](int c, int e, Cx<T> v) { s[e * C + c] = v; };
+    auto fac = [&](int c, int e, Cx<T> v) -> Cx<T> {
+        const int p = min(p0 + c, plane - 1), y = (unsigned)p / (unsigned)ax.n, x = p - y * ax.n;
+        const double qx = ax.g * (double)freq[ax.off + x], qy = ay.g * (double)freq[ay.off + y],
+                     qz = az.g * (double)freq[az.off + e];
+        const double e2 = 0.5 * (qx * qx + qy * qy + qz * qz);
+        const double f = e2 == 0.0 ? 0.0 : 2.0 * M_PI / e2 * scale;
+        return {v.x * f, v.y * f};
+    };
+    if (az.ns == 1) {
+        mid<T, BIG>(az.r[0], ldg, stg, fac, C, n);
+        return;
+    }
+    int L = n;
+    for (int q = 0; q < az.ns - 1; ++q) {
+        if (q == 0) stage<T, BIG, false>(az.r[q], ldg, sts, C, n, L, tw);
+        else stage<T, BIG, false>(az.r[q], lds, sts, C, n, L, tw);
+        L /= az.r[q];
+        __syncthreads();
+    }
+    mid<T, BIG>(az.r[az.ns - 1], lds, sts, fac, C, n);
+    __syncthreads();
+    for (int q = az.ns - 2; q >= 0; --q) {
+        L *= az.r[q];
+        if (q == 0) stage<T, BIG, true>(az.r[q], lds, stg, C, n, L, tw);
+        else stage<T, BIG, true>(az.r[q], lds, sts, C, n, L, tw);
+        __syncthreads();
+    }
+}
+
+// plane z of V_H = the real part of F_xy^-1 of spectrum plane z
+template <bool BIG>
+__global__ __launch_bounds__(1024) void poisson_inverse_kernel(double *__restrict__ vh,
+                                                               const Cx<double> *__restrict__ spec,
+                                                               const Cx<double> *__restrict__ twt, int pitch, Axis ax,
+                                                               Axis ay) {
+    using T = double;
+    extern __shared__ __align__(16) unsigned char spectral_lds[];
+    Cx<T> *twx = reinterpret_cast<Cx<T> *>(spectral_lds), *twy = twx + ax.n, *s = twy + ay.n;
+    const int nx = ax.n, ny = ay.n, plane = nx * ny;
+    const int64_t base = (int64_t)blockIdx.x * plane;
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) twx[i] = twt[ax.off + i];
+    for (int i = threadIdx.x; i < ny; i += blockDim.x) twy[i] = twt[ay.off + i];
+    for (int i = threadIdx.x; i < plane; i += blockDim.x) {
+        const int y = (unsigned)i / (unsigned)nx;
+        s[y * pitch + i - y * nx] = spec[base + i];
+    }
+    __syncthreads();
+    auto stg = [&](int c, int e, Cx<T> v) { vh[base + e * nx + c] = v.x; };
+    auto ldy = [&](int c, int e) { return s[e * pitch + c]; };
+    auto sty = [&](int c, int e, Cx<T> v) { s[e * pitch + c] = v; };
+    auto ldx = [&](int c, int e) { return s[c * pitch + e]; };
+    auto stx = [&](int c, int e, Cx<T> v) { s[c * pitch + e] = v; };
+    int L = 1;
+    for (int q = ax.ns - 1; q >= 0; --q) {
+        L *= ax.r[q];
+        stage<T, BIG, true>(ax.r[q], ldx, stx, ny, nx, L, twx);
+        __syncthreads();
+    }
+    L = 1;
+    for (int q = ay.ns - 1; q >= 0; --q) {
+        L *= ay.r[q];
+        if (q == 0) stage<T, BIG, true>(ay.r[q], ldy, stg, nx, ny, L, twy);
+        else stage<T, BIG, true>(ay.r[q], ldy, sty, nx, ny, L, twy);
+        __syncthreads();
+    }
+}
+
 // Radices of n, largest first so that few stages touch LDS and the middle
 // stage, whose elements stay in registers, is a small one; false when a prime
 // factor above 13 remains.
@@ -548,6 +681,29 @@ int launch_parts(const qm_ctx *ctx, const SpectralTables *t, T *out, const T *ps
     return QM_OK;
 }
 
+template <bool BIG>
+int launch_poisson(const qm_ctx *ctx, const SpectralTables *t, Cx<double> *spec, double *vh, const double *rho,
+                   hipStream_t st) {
+    const int nx = ctx->nx, ny = ctx->ny, nz = ctx->nz, plane = nx * ny;
+    int pitch = 0, threads = 0, C = 0;
+    size_t plds = 0, llds = 0;
+    QM_CHECK(plane_shape<double>(nx, ny, &pitch, &plds, &threads) && line_shape<double>(nz, &C, &llds), QM_ERR_STATE,
+             "Poisson solve: the grid does not fit the kernels");
+    auto *fk = poisson_forward_kernel<BIG>;
+    auto *ik = poisson_inverse_kernel<BIG>;
+    if (plds > (size_t)64 * 1024)
+        for (const void *f : {(const void *)fk, (const void *)ik})
+            QM_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plds));
+    hipLaunchKernelGGL(fk, dim3(nz), dim3(threads), plds, st, spec, rho, t->d_tw64, pitch, t->ax[0], t->ax[1]);
+    QM_HIP(hipGetLastError());
+    hipLaunchKernelGGL(poisson_line_kernel<BIG>, dim3((plane + C - 1) / C), dim3(256), llds, st, spec, t->d_tw64,
+                       t->d_freq, plane, C, t->ax[0], t->ax[1], t->ax[2], 1.0 / (double)ctx->ng);
+    QM_HIP(hipGetLastError());
+    hipLaunchKernelGGL(ik, dim3(nz), dim3(threads), plds, st, vh, spec, t->d_tw64, pitch, t->ax[0], t->ax[1]);
+    QM_HIP(hipGetLastError());
+    return QM_OK;
+}
+
 }  // namespace
 
 template <typename T>
@@ -574,5 +730,11 @@ template int spectral_step<double>(const qm_ctx *, const SpectralTables *, doubl
                                    hipStream_t);
 template int spectral_step<float>(const qm_ctx *, const SpectralTables *, float *, int, const double *, double,
                                   hipStream_t);
+
+int spectral_poisson(const qm_ctx *ctx, const SpectralTables *t, void *spec, double *vh, const double *rho,
+                     hipStream_t st) {
+    Cx<double> *z = static_cast<Cx<double> *>(spec);
+    return t->big ? launch_poisson<true>(ctx, t, z, vh, rho, st) : launch_poisson<false>(ctx, t, z, vh, rho, st);
+}
 
 }  // namespace qm

@@ -69,3 +69,25 @@ def test_spectral_step_edges(qm, torch_cuda, grid):
         err = float(np.abs(got - want).max() / np.abs(want).max())
         assert err <= tol, (grid, name, err)
     H.close()
+
+
+@pytest.mark.parametrize("grid", GRIDS, ids=["x".join(map(str, g)) for g in GRIDS])
+def test_poisson_edges(qm, torch_cuda, grid):
+    """V_H = IFFT(4 pi / |G|^2 FFT rho) without G = 0 against numpy's FFT, 1e-12 relative."""
+    torch = torch_cuda
+    s = _sys(qm, grid, 1)
+    H = qm.hamiltonian.Hamiltonian(s)
+    print(f"case Poisson {grid}", flush=True)
+    rho = np.random.default_rng(7).uniform(0.1, 1.0, s.ng)
+    g2 = 0.0
+    for ax, n in enumerate(grid):
+        g = np.fft.fftfreq(n, 1.0 / n) * 2 * np.pi / (0.25 * n)
+        g2 = g2 + (g * g).reshape([-1 if 2 - ax == d else 1 for d in range(3)])
+    f = np.fft.fftn(rho.reshape(grid[2], grid[1], grid[0]))
+    g2[0, 0, 0] = 1.0
+    f *= 4 * np.pi / g2
+    f[0, 0, 0] = 0.0
+    want = np.fft.ifftn(f).real.reshape(-1)
+    got = qm.scf.hartree(H, torch.from_numpy(rho).cuda()).cpu().numpy()
+    assert np.abs(got - want).max() <= 1e-12 * np.abs(want).max()
+    H.close()
