@@ -356,8 +356,8 @@ int qm_lobpcg_set_rollback_limit(qm_lobpcg *s, double limit);
 /* Generalized Hermitian eigenproblem A z = l B z in complex FP64, in place of
  * lapack_ZHEGVD_emu (w_zhegvd.h:227-272): B = U^H U (rocSOLVER zpotrf),
  * C = U^-H A U^-1 (two ztrsm), the cooperative tridiagonal reduction of C,
- * stedc (steqr where stedc does not converge) and the back-transformations.
- * Matrices are n x n column-major, complex interleaved (re, im) doubles;
+ * divide and conquer on it (rocSOLVER stedc / steqr above order 1024) and the
+ * back-transformations.  Matrices are n x n column-major, complex interleaved (re, im) doubles;
  * d_A and d_B: upper triangles referenced, not modified.  d_w: all n
  * eigenvalues, ascending.  d_Z: n x nev, the nev lowest eigenvectors,
  * B-orthonormal.  d_U: upper triangle receives the Cholesky factor of B.

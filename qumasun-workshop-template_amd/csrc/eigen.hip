@@ -453,19 +453,25 @@ int sytrd_lower(void *blas, int n, double *C, int lda, double *trd, double *VW, 
 // Eigenvalues (all, ascending, into w) and the eigenvectors of the nev lowest
 // into Z[:, :nev] (ldz >= n) of the symmetric matrix whose upper triangle C
 // holds (C overwritten).
-// Where the cooperative reduction fits (trd_coop.hip): that reduction,
-// rocSOLVER stedc + ormtr; else n <= kMaxN: the single-workgroup panel
+// Where the cooperative reduction fits (trd_coop.hip): that reduction, the own
+// divide and conquer (tridiag_dc.hip, work dcw; rocSOLVER stedc above its
+// order) and the own back-transformation; else n <= kMaxN: the single-workgroup panel
 // reduction below, stedc + ormtr (Z must hold n x n in both); larger n:
 // rocSOLVER syevd.  info receives rocSOLVER's status (or the cooperative
 // reduction's barrier error, -77).  trd holds 4 n doubles (d, e, tau, and a
 // copy of e for the steqr retry after a stedc failure).
 int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double *Z, int ldz, double *trd,
-               double *VW, int *info, hipStream_t st) {
+               double *VW, void *dcw, int *info, hipStream_t st) {
     rocblas_handle h = (rocblas_handle)blas;
     if (subspace_route() != 0 && trd_coop_supported(n, false) &&
         trd_coop_work_bytes(n, false) <= sizeof(double) * (size_t)kTrdPanelCols * n) {
         const int r = trd_coop_f64(n, C, lda, trd, trd + n, trd + 2 * n, VW,
                                    sizeof(double) * (size_t)kTrdPanelCols * n, st);
+        if (r == QM_OK && tridiag_dc_supported(n)) {
+            QM_TRY(tridiag_dc(n, nev, trd, trd + n, w, Z, ldz, false, dcw, info, st));
+            QM_TRY(trd_coop_check(VW, info, st));
+            return ormtr_lower_f64(n, nev, C, lda, trd + 2 * n, Z, ldz, VW, st);
+        }
         if (r == QM_OK) {
             double *e_copy = trd + 3 * n;  // stedc overwrites e
             QM_HIP(hipMemcpyAsync(e_copy, trd + n, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
@@ -598,12 +604,14 @@ int qm_sygvd_f64(qm_ctx *ctx, int n, const double *d_A, const double *d_B, doubl
     QM_EIG_BLAS(rocblas_set_stream(h, st));
     // workspace: C (n^2), Z (n^2), d e tau + e copy (4n), VW (96 n), U^-1 and T (n^2 each), info
     const size_t nn = (size_t)n * n;
+    const size_t dcb = tridiag_dc_supported(n) ? tridiag_dc_work_bytes(n) : 0;
     const size_t need = sizeof(double) * (4 * nn + 4 * (size_t)n + (size_t)kTrdPanelCols * n) + 256 + 512;
-    QM_TRY(ctx->eig_work.reserve(need));
+    QM_TRY(ctx->eig_work.reserve(need + dcb));
     double *C = ctx->eig_work.as<double>(), *Z = C + nn, *trd = Z + nn, *VW = trd + 4 * n;
     double *Ui = VW + (size_t)kTrdPanelCols * n, *T = Ui + nn;
     int *info = (int *)(T + nn);
     void *psync = reinterpret_cast<char *>(T + nn) + 256;  // the cooperative Cholesky's barrier words
+    void *dcw = reinterpret_cast<char *>(T + nn) + 256 + 512;
     hipLaunchKernelGGL(symmetrize_upper_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st, C, d_A, n);
     QM_HIP(hipGetLastError());
     QM_HIP(hipMemcpyAsync(d_U, d_B, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
@@ -615,7 +623,7 @@ int qm_sygvd_f64(qm_ctx *ctx, int n, const double *d_A, const double *d_B, doubl
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
              "qm_sygvd_f64: B is not positive definite (leading minor " + std::to_string(h_info) + ")");
     QM_TRY(chol_transform(h, n, d_U, C, Ui, T, st));
-    QM_TRY(syev_lower(h, n, nev, C, n, d_w, Z, n, trd, VW, info, st));
+    QM_TRY(syev_lower(h, n, nev, C, n, d_w, Z, n, trd, VW, dcw, info, st));
     QM_TRY(chol_back(h, n, nev, Ui, Z, n, d_Z, n));
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
@@ -645,13 +653,15 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
     // the cooperative reduction's work, info
     const size_t nn = (size_t)n * n;
     const size_t coopb = trd_coop_work_bytes(n, true);
+    const size_t dcb = tridiag_dc_supported(n) ? tridiag_dc_work_bytes(n) : 0;
     const size_t need = sizeof(zc) * 2 * nn + sizeof(double) * 5 * (size_t)n + coopb + 512;
-    QM_TRY(ctx->eig_work.reserve(need));
+    QM_TRY(ctx->eig_work.reserve(need + dcb));
     zc *C = ctx->eig_work.as<zc>(), *Z = C + nn;
     double *d = reinterpret_cast<double *>(Z + nn), *e = d + n, *e_copy = d + 4 * (size_t)n;
     zc *tau = reinterpret_cast<zc *>(d + 2 * (size_t)n);
     void *coop = d + 5 * (size_t)n;
     int *info = reinterpret_cast<int *>(static_cast<char *>(coop) + coopb);
+    void *dcw = reinterpret_cast<char *>(info) + 512;
     zc *U = static_cast<zc *>(d_U);
     QM_HIP(hipMemcpyAsync(C, d_A, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
     QM_HIP(hipMemcpyAsync(U, d_B, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
@@ -673,7 +683,11 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
     int r = QM_ERR_STATE;
     if (subspace_route() != 0 && trd_coop_supported(n, true))
         r = trd_coop_z64(n, C, n, d, e, tau, coop, coopb, st);
-    if (r == QM_OK) {
+    if (r == QM_OK && tridiag_dc_supported(n)) {
+        QM_TRY(tridiag_dc(n, nev, d, e, d_w, reinterpret_cast<double *>(Z), n, true, dcw, info, st));
+        QM_TRY(trd_coop_check(coop, info, st));
+        QM_TRY(unmtr_lower_z64(n, nev, C, n, tau, Z, n, coop, st));
+    } else if (r == QM_OK) {
         QM_HIP(hipMemcpyAsync(e_copy, e, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
         QM_HIP(hipMemcpyAsync(d_w, d, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
         QM_EIG_BLAS(rocsolver_zstedc(h, rocblas_evect_tridiagonal, n, d_w, e, Z, n, info));

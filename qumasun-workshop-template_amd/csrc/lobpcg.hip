@@ -13,8 +13,8 @@
 //                     lobpcg_z_multi_mpi.h:2254-2263, 2492-2511): real n <= 512 by
 //                     the own cooperative Cholesky, trtri + GEMMs; real and complex
 //                     by the own cooperative tridiagonal reduction (trd_coop.hip),
-//                     rocSOLVER stedc and the own back-transformation of the
-//                     wanted eigenvectors; complex Cholesky and the problems the
+//                     divide and conquer (tridiag_dc.hip) and back-transformation
+//                     of the wanted eigenvectors; complex Cholesky and the problems the
 //                     cooperative reduction does not fit by rocSOLVER potrf /
 //                     trsm / syevd or heevd
 //   recurrence        S' = Cb^H S Cb, H' = Cb^H H Cb with Cb = [C | C_P] (rocBLAS;
@@ -516,6 +516,7 @@ struct qm_lobpcg {
     double *evk = nullptr;   // Ritz values of the last accepted iteration (device, N)
     double *pen = nullptr;   // diagonal of dropped directions in the subspace problem (device, 1)
     void *rt = nullptr;      // S times the N lowest Ritz vectors (device, 3N x N subspace elements)
+    void *dcw = nullptr;     // workspace of the tridiagonal divide and conquer (device)
     void *psync = nullptr;   // barrier words of the cooperative Cholesky (device, 512 bytes)
     bool graphs = true;      // replay A.R + Gram of an iteration as a HIP graph
     hipStream_t gstream = nullptr;  // capture stream (graphs launch on the caller's stream)
@@ -549,6 +550,8 @@ void lfree(qm_lobpcg *s) {
     s->pen = nullptr;
     if (s->rt) (void)hipFree(s->rt);
     s->rt = nullptr;
+    if (s->dcw) (void)hipFree(s->dcw);
+    s->dcw = nullptr;
     if (s->psync) (void)hipFree(s->psync);
     s->psync = nullptr;
     if (s->gstream) (void)hipStreamDestroy(s->gstream);
@@ -591,7 +594,7 @@ int hpsi(qm_lobpcg *s, T *out, const T *in, int nb, int ik, hipStream_t st) {
 // C = U^-H H U^-1 (two trsm), eigh(C) (syevd), c = U^-1 y (trsm, first N columns).
 // Real n <= own_eig_max_n() instead factors S in one launch of the own
 // Cholesky, forms U^-1 once (trtri) and applies it by GEMMs, and diagonalises
-// C by the own tridiagonal reduction + stedc / ormtr.
+// C by the own tridiagonal reduction, divide and conquer and back-transformation.
 // Works on copies Sw, Hw; eigenvalues in s->evals, eigenvectors in Hw.  After
 // potrf the squared pivot ratio is written to s->svals[0] for the caller's
 // conditioning check; on potrf failure s->info > 0 and the rest is skipped by
@@ -622,23 +625,29 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
                               rocblas_diagonal_non_unit, n3, n3, &one, U, n3, C, n3));
         if (subspace_route() != 0 && trd_coop_supported(n3, true) &&
             trd_coop_work_bytes(n3, true) <= sizeof(double) * (size_t)kTrdPanelCols * n3) {
-            // own cooperative reduction C = Q T Q^H, stedc on T, Z = Q Y for the N
-            // lowest, c = U^-1 Z; eigenvectors in T1
+            // own cooperative reduction C = Q T Q^H, divide and conquer on T (stedc
+            // above its order), Z = Q Y for the N lowest, c = U^-1 Z; eigenvectors in T1
             double *d = s->trd, *e = s->trd + n3;
             auto *tau = (rocblas_double_complex *)(s->trd + 2 * n3);
             auto *Z = (rocblas_double_complex *)s->T1;
             const int r = trd_coop_z64(n3, C, n3, d, e, tau, s->VW, sizeof(double) * (size_t)kTrdPanelCols * n3, st);
             if (r == QM_OK) {
                 double *e_copy = s->trd + 4 * n3;  // stedc overwrites e
-                QM_HIP(hipMemcpyAsync(e_copy, e, sizeof(double) * n3, hipMemcpyDeviceToDevice, st));
-                QM_HIP(hipMemcpyAsync(s->evals, d, sizeof(double) * n3, hipMemcpyDeviceToDevice, st));
-                std::vector<double> hde(2 * (size_t)n3);
-                QM_HIP(hipMemcpyAsync(hde.data(), d, sizeof(double) * 2 * n3, hipMemcpyDeviceToHost, st));
-                QM_BLAS(rocsolver_zstedc(s->blas, rocblas_evect_tridiagonal, n3, s->evals, e, Z, n3, s->info));
+                const bool dc = tridiag_dc_supported(n3);
+                std::vector<double> hde(dc ? 0 : 2 * (size_t)n3);
+                if (dc) {
+                    QM_TRY(tridiag_dc(n3, N, d, e, s->evals, reinterpret_cast<double *>(Z), n3, true, s->dcw, s->info,
+                                      st));
+                } else {
+                    QM_HIP(hipMemcpyAsync(e_copy, e, sizeof(double) * n3, hipMemcpyDeviceToDevice, st));
+                    QM_HIP(hipMemcpyAsync(s->evals, d, sizeof(double) * n3, hipMemcpyDeviceToDevice, st));
+                    QM_HIP(hipMemcpyAsync(hde.data(), d, sizeof(double) * 2 * n3, hipMemcpyDeviceToHost, st));
+                    QM_BLAS(rocsolver_zstedc(s->blas, rocblas_evect_tridiagonal, n3, s->evals, e, Z, n3, s->info));
+                }
                 int h_info = 0;
                 QM_HIP(hipMemcpyAsync(&h_info, s->info, sizeof(int), hipMemcpyDeviceToHost, st));
                 QM_HIP(hipStreamSynchronize(st));
-                bool finite = true;
+                bool finite = !dc || h_info != 1;
                 for (size_t i = 0; i + 1 < hde.size(); ++i) finite = finite && std::isfinite(hde[i]);
                 if (!finite) {
                     // the tridiagonal is not finite: say whether its input was, then
@@ -662,7 +671,7 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
                     s->evec_t1 = false;
                     return QM_OK;
                 }
-                if (h_info != 0) {
+                if (h_info != 0 && !dc) {  // an unconverged root of the own solver is left to the caller's check
                     // divide and conquer did not converge (it can on nearly degenerate
                     // spectra): implicit QL/QR on the same tridiagonal instead
                     ++s->stedc_retries;
@@ -688,11 +697,11 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
         const double one = 1.0;
         auto *U = (double *)s->Sw, *C = (double *)s->Hw;
         if (n3 <= own_eig_max_n()) {
-            // C = U^-T H U^-1 through U^-1 and GEMMs, own tridiagonal reduction +
-            // rocSOLVER stedc / ormtr (eigenvectors in T1), then c = U^-1 y into Hw
+            // C = U^-T H U^-1 through U^-1 and GEMMs, own tridiagonal reduction, divide
+            // and conquer and back-transformation (eigenvectors in T1), then c = U^-1 y into Hw
             auto *Ui = (double *)s->Ev, *Z = (double *)s->T1;
             QM_TRY(chol_transform(s->blas, n3, U, C, Ui, Z, st));
-            QM_TRY(syev_lower(s->blas, n3, N, C, n3, s->evals, Z, n3, s->trd, s->VW, s->info, st));
+            QM_TRY(syev_lower(s->blas, n3, N, C, n3, s->evals, Z, n3, s->trd, s->VW, s->dcw, s->info, st));
             QM_TRY(chol_back(s->blas, n3, N, Ui, Z, n3, C, n3));
             s->evec_t1 = false;
             return QM_OK;
@@ -1480,6 +1489,8 @@ int qm_lobpcg_create(qm_lobpcg **out, qm_ctx *ctx, int nbands, int ncomp, int pr
     if (st == QM_OK) st = dalloc((void **)&s->pen, sizeof(double));
     if (st == QM_OK) st = dalloc(&s->rt, esz * (size_t)n3 * N);
     if (st == QM_OK) st = dalloc(&s->psync, 512);
+    // every order a solve can meet: up to 3 N, of which those above the limit take stedc
+    if (st == QM_OK) st = dalloc(&s->dcw, tridiag_dc_work_bytes(std::min(n3, tridiag_dc_max())));
     if (st == QM_OK && hipStreamCreateWithFlags(&s->gstream, hipStreamNonBlocking) != hipSuccess) {
         s->gstream = nullptr;
         set_error("qm_lobpcg_create: hipStreamCreateWithFlags failed");

@@ -188,7 +188,17 @@ bool stencil_near_best(const qm_ctx *ctx, int precision, int ncomp, int kt, int 
 // eigen.hip: FP64 symmetric eigensolver pieces (rocblas_handle passed as void *)
 int sytrd_lower(void *blas, int n, double *C, int lda, double *trd, double *VW, hipStream_t st);
 int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double *Z, int ldz, double *trd,
-               double *VW, int *info, hipStream_t st);
+               double *VW, void *dcw, int *info, hipStream_t st);
+// tridiag_dc.hip: all eigenvalues (ascending, w) and the nev lowest eigenvectors
+// (Z[:, :nev], ldz >= n; interleaved complex with zero imaginary parts when
+// cplx) of the symmetric tridiagonal (d, e), which is left as it is.  *info
+// (device): 0, 1 for a non-finite matrix, 2 where a root did not converge.
+// work: tridiag_dc_work_bytes; n up to tridiag_dc_max.
+int tridiag_dc_max();
+int tridiag_dc_supported(int n);
+size_t tridiag_dc_work_bytes(int n);
+int tridiag_dc(int n, int nev, const double *d, const double *e, double *w, double *Z, int ldz, bool cplx, void *work,
+               int *info, hipStream_t st);
 int own_eig_max_n();
 // A = U^T U, upper triangle of the column-major n x n A (FP64): with sync (512
 // bytes of device memory) and n <= 512, one workgroup per 32-row panel
