@@ -22,6 +22,7 @@
 
 #include "qm_internal.h"
 #include "qm_mfma.h"
+#include "qm_wave.h"
 
 namespace qm {
 namespace {
@@ -48,39 +49,6 @@ struct DcWork {
 
 // first row of node i at depth l
 __host__ __device__ __forceinline__ int node_start(int n, int l, int i) { return (int)(((int64_t)i * n) >> l); }
-
-// v of the lane `R` places on inside a row of 16 (rotation), through DPP
-template <int R>
-__device__ __forceinline__ double row_ror(double v) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x120 + R, 0xf, 0xf, false);
-    const unsigned hi =
-        (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)((unsigned long long)b >> 32), 0x120 + R, 0xf, 0xf, false);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)b >> 32), lane);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-// Sum over the wave, the same bits in every lane: rows of 16 by DPP rotations,
-// the four rows' sums through scalar registers (six exchanges through LDS each:
-// 13.8 us a level in the root kernel at n = 384, so 12.6).
-__device__ __forceinline__ double wave_sum(double v) {
-    v += row_ror<1>(v);
-    v += row_ror<2>(v);
-    v += row_ror<4>(v);
-    v += row_ror<8>(v);
-    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-__device__ __forceinline__ double wave_prod(double v) {
-    v *= row_ror<1>(v);
-    v *= row_ror<2>(v);
-    v *= row_ror<4>(v);
-    v *= row_ror<8>(v);
-    return (lane_value(v, 0) * lane_value(v, 16)) * (lane_value(v, 32) * lane_value(v, 48));
-}
 
 // scale, split offsets; *info = 1 for a non-finite input (T is then taken as 0)
 __global__ __launch_bounds__(256) void dc_init_kernel(DcWork w, const double *__restrict__ d,
