@@ -354,8 +354,8 @@ int qm_lobpcg_eigen_retries(qm_lobpcg *s, char *note, int len);
 int qm_lobpcg_set_rollback_limit(qm_lobpcg *s, double limit);
 
 /* Generalized Hermitian eigenproblem A z = l B z in complex FP64, in place of
- * lapack_ZHEGVD_emu (w_zhegvd.h:227-272): B = U^H U (rocSOLVER zpotrf),
- * C = U^-H A U^-1 (two ztrsm), the cooperative tridiagonal reduction of C,
+ * lapack_ZHEGVD_emu (w_zhegvd.h:227-272): B = U^H U and U^-1,
+ * C = U^-H A U^-1 (rocSOLVER / rocBLAS above order 1024), the cooperative tridiagonal reduction of C,
  * divide and conquer on it (rocSOLVER stedc / steqr above order 1024) and the
  * back-transformations.  Matrices are n x n column-major, complex interleaved (re, im) doubles;
  * d_A and d_B: upper triangles referenced, not modified.  d_w: all n
@@ -379,8 +379,8 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
  * (different summation orders). */
 int qm_subspace_force(int route);
 
-/* Bound of the grid-barrier waits in the cooperative kernels (the tridiagonal
- * reduction and the Cholesky), in polls, process-wide; no reference
+/* Bound of the grid-barrier waits in the cooperative kernel (the tridiagonal
+ * reduction), in polls, process-wide; no reference
  * counterpart (a diagnostic and test control).  A workgroup that waits past
  * it sets the launch's error word and stops waiting, so does every other
  * waiter within 256 polls, the kernel ends, and the solve reports it

@@ -514,12 +514,16 @@ int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double
 // part cleared) and two GEMMs: at the LOBPCG subspace size (n = 384) this is
 // 0.18 ms against 0.25 ms for two triangular solves.  Ui is kept for
 // chol_back; T is n x n work.
-int chol_transform(void *blas, int n, const double *U, double *C, double *Ui, double *T, hipStream_t st) {
+int chol_transform(void *blas, int n, const double *U, double *C, double *Ui, bool have_ui, double *T,
+                   hipStream_t st) {
     rocblas_handle h = (rocblas_handle)blas;
     const double one = 1.0, zero = 0.0;
-    QM_EIG_BLAS(rocblas_dtrtri(h, rocblas_fill_upper, rocblas_diagonal_non_unit, n, U, n, Ui, n));
-    hipLaunchKernelGGL(zero_lower_kernel, dim3((unsigned)(((int64_t)n * n + 255) / 256)), dim3(256), 0, st, Ui, n, n);
-    QM_HIP(hipGetLastError());
+    if (!have_ui) {
+        QM_EIG_BLAS(rocblas_dtrtri(h, rocblas_fill_upper, rocblas_diagonal_non_unit, n, U, n, Ui, n));
+        hipLaunchKernelGGL(zero_lower_kernel, dim3((unsigned)(((int64_t)n * n + 255) / 256)), dim3(256), 0, st, Ui, n,
+                           n);
+        QM_HIP(hipGetLastError());
+    }
     QM_EIG_BLAS(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, n, n, n, &one, Ui, n, C, n,
                               &zero, T, n));
     QM_EIG_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, T, n, Ui, n, &zero,
@@ -536,13 +540,7 @@ int chol_back(void *blas, int n, int nev, const double *Ui, const double *Z, int
     return QM_OK;
 }
 
-int potrf_upper(void *blas, int n, double *A, int lda, int *info, hipStream_t st, void *sync) {
-    // one workgroup per 32-row panel where the caller gives the barrier words
-    // (and the subspace route is not forced onto the single-workgroup kernels)
-    if (sync && subspace_route() < 0 && potrf_coop_supported(n)) {
-        const int rc = potrf_coop_f64(n, A, lda, info, sync, st);
-        if (rc != QM_ERR_STATE) return rc;
-    }
+int potrf_upper(void *blas, int n, double *A, int lda, int *info, hipStream_t st) {
     if (n > kMaxN) {
         QM_EIG_BLAS(rocsolver_dpotrf((rocblas_handle)blas, rocblas_fill_upper, n, A, lda, info));
         return QM_OK;
@@ -605,24 +603,27 @@ int qm_sygvd_f64(qm_ctx *ctx, int n, const double *d_A, const double *d_B, doubl
     // workspace: C (n^2), Z (n^2), d e tau + e copy (4n), VW (96 n), U^-1 and T (n^2 each), info
     const size_t nn = (size_t)n * n;
     const size_t dcb = tridiag_dc_supported(n) ? tridiag_dc_work_bytes(n) : 0;
-    const size_t need = sizeof(double) * (4 * nn + 4 * (size_t)n + (size_t)kTrdPanelCols * n) + 256 + 512;
+    const size_t need = sizeof(double) * (4 * nn + 4 * (size_t)n + (size_t)kTrdPanelCols * n) + 256;
     QM_TRY(ctx->eig_work.reserve(need + dcb));
     double *C = ctx->eig_work.as<double>(), *Z = C + nn, *trd = Z + nn, *VW = trd + 4 * n;
     double *Ui = VW + (size_t)kTrdPanelCols * n, *T = Ui + nn;
     int *info = (int *)(T + nn);
-    void *psync = reinterpret_cast<char *>(T + nn) + 256;  // the cooperative Cholesky's barrier words
-    void *dcw = reinterpret_cast<char *>(T + nn) + 256 + 512;
+    void *dcw = reinterpret_cast<char *>(T + nn) + 256;
     hipLaunchKernelGGL(symmetrize_upper_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st, C, d_A, n);
     QM_HIP(hipGetLastError());
-    QM_HIP(hipMemcpyAsync(d_U, d_B, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
-    QM_TRY(potrf_upper(h, n, d_U, n, info, st, psync));
+    const bool own = subspace_route() < 0 && chol_inverse_supported(n);
+    if (own) {
+        QM_TRY(chol_inverse(n, false, d_B, T, d_U, Ui, info, st));
+    } else {
+        QM_HIP(hipMemcpyAsync(d_U, d_B, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
+        QM_TRY(potrf_upper(h, n, d_U, n, info, st));
+    }
     int h_info = 0;
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
-    QM_CHECK(h_info != -77, QM_ERR_NUMERIC, "qm_sygvd_f64: the cooperative Cholesky's grid barrier timed out (info -77)");
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
              "qm_sygvd_f64: B is not positive definite (leading minor " + std::to_string(h_info) + ")");
-    QM_TRY(chol_transform(h, n, d_U, C, Ui, T, st));
+    QM_TRY(chol_transform(h, n, d_U, C, Ui, own, T, st));
     QM_TRY(syev_lower(h, n, nev, C, n, d_w, Z, n, trd, VW, dcw, info, st));
     QM_TRY(chol_back(h, n, nev, Ui, Z, n, d_Z, n));
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -649,37 +650,49 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
     rocblas_handle h = (rocblas_handle)ctx->blas;
     QM_EIG_BLAS(rocblas_set_stream(h, st));
     using zc = rocblas_double_complex;
-    // workspace: C and Z (n^2 complex each), d, e, tau (complex), e copy (5n doubles),
-    // the cooperative reduction's work, info
+    // workspace: C, Z and U^-1 (n^2 complex each), d, e, tau (complex), e copy (5n
+    // doubles), the cooperative reduction's work, info, divide and conquer
     const size_t nn = (size_t)n * n;
     const size_t coopb = trd_coop_work_bytes(n, true);
     const size_t dcb = tridiag_dc_supported(n) ? tridiag_dc_work_bytes(n) : 0;
-    const size_t need = sizeof(zc) * 2 * nn + sizeof(double) * 5 * (size_t)n + coopb + 512;
+    const size_t need = sizeof(zc) * 3 * nn + sizeof(double) * 5 * (size_t)n + coopb + 512;
     QM_TRY(ctx->eig_work.reserve(need + dcb));
-    zc *C = ctx->eig_work.as<zc>(), *Z = C + nn;
-    double *d = reinterpret_cast<double *>(Z + nn), *e = d + n, *e_copy = d + 4 * (size_t)n;
+    zc *C = ctx->eig_work.as<zc>(), *Z = C + nn, *Ui = Z + nn;
+    double *d = reinterpret_cast<double *>(Ui + nn), *e = d + n, *e_copy = d + 4 * (size_t)n;
     zc *tau = reinterpret_cast<zc *>(d + 2 * (size_t)n);
     void *coop = d + 5 * (size_t)n;
     int *info = reinterpret_cast<int *>(static_cast<char *>(coop) + coopb);
     void *dcw = reinterpret_cast<char *>(info) + 512;
     zc *U = static_cast<zc *>(d_U);
     QM_HIP(hipMemcpyAsync(C, d_A, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
-    QM_HIP(hipMemcpyAsync(U, d_B, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
-    QM_EIG_BLAS(rocsolver_zpotrf(h, rocblas_fill_upper, n, U, n, info));
+    const bool own = subspace_route() < 0 && chol_inverse_supported(n);
+    if (own) {
+        QM_TRY(chol_inverse(n, true, d_B, Z, U, Ui, info, st));
+    } else {
+        QM_HIP(hipMemcpyAsync(U, d_B, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
+        QM_EIG_BLAS(rocsolver_zpotrf(h, rocblas_fill_upper, n, U, n, info));
+    }
     int h_info = 0;
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
              "qm_hegvd_z64: B is not positive definite (leading minor " + std::to_string(h_info) + ")");
-    const zc one{1.0, 0.0};
+    const zc one{1.0, 0.0}, zero{0.0, 0.0};
     // C = U^-H A U^-1 (the upper triangle defines A)
     hipLaunchKernelGGL(hermitian_from_upper_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<double *>(C), n);
     QM_HIP(hipGetLastError());
-    QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_conjugate_transpose,
-                              rocblas_diagonal_non_unit, n, n, &one, U, n, C, n));
-    QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                              rocblas_diagonal_non_unit, n, n, &one, U, n, C, n));
+    if (own) {
+        QM_EIG_BLAS(rocblas_zgemm(h, rocblas_operation_conjugate_transpose, rocblas_operation_none, n, n, n, &one, Ui,
+                                  n, C, n, &zero, Z, n));
+        QM_EIG_BLAS(rocblas_zgemm(h, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, Z, n, Ui, n, &zero,
+                                  C, n));
+    } else {
+        QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_conjugate_transpose,
+                                  rocblas_diagonal_non_unit, n, n, &one, U, n, C, n));
+        QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
+                                  rocblas_diagonal_non_unit, n, n, &one, U, n, C, n));
+    }
     int r = QM_ERR_STATE;
     if (subspace_route() != 0 && trd_coop_supported(n, true))
         r = trd_coop_z64(n, C, n, d, e, tau, coop, coopb, st);
@@ -705,9 +718,14 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
         QM_HIP(hipMemcpyAsync(Z, C, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
     }
     // z = U^-1 y for the nev lowest
-    QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_none,
-                              rocblas_diagonal_non_unit, n, nev, &one, U, n, Z, n));
-    QM_HIP(hipMemcpyAsync(d_Z, Z, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
+    if (own) {
+        QM_EIG_BLAS(rocblas_zgemm(h, rocblas_operation_none, rocblas_operation_none, n, nev, n, &one, Ui, n, Z, n,
+                                  &zero, static_cast<zc *>(d_Z), n));
+    } else {
+        QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_none,
+                                  rocblas_diagonal_non_unit, n, nev, &one, U, n, Z, n));
+        QM_HIP(hipMemcpyAsync(d_Z, Z, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
+    }
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,

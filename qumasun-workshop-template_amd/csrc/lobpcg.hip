@@ -10,12 +10,11 @@
 //                     the real Gram of the SoA columns (AoSComplexFrom2by2Real,
 //                     matrix_2x2real_to_complex.h:8-56)
 //   H c = l S c       the Cholesky route of lapack_ZHEGVD_emu (w_zhegvd.h:227-272;
-//                     lobpcg_z_multi_mpi.h:2254-2263, 2492-2511): real n <= 512 by
-//                     the own cooperative Cholesky, trtri + GEMMs; real and complex
-//                     by the own cooperative tridiagonal reduction (trd_coop.hip),
-//                     divide and conquer (tridiag_dc.hip) and back-transformation
-//                     of the wanted eigenvectors; complex Cholesky and the problems the
-//                     cooperative reduction does not fit by rocSOLVER potrf /
+//                     lobpcg_z_multi_mpi.h:2254-2263, 2492-2511): the own blocked
+//                     Cholesky with its inverse (chol.hip) + GEMMs, cooperative
+//                     tridiagonal reduction (trd_coop.hip), divide and conquer
+//                     (tridiag_dc.hip) and back-transformation of the wanted
+//                     eigenvectors; orders these do not fit by rocSOLVER potrf /
 //                     trsm / syevd or heevd
 //   recurrence        S' = Cb^H S Cb, H' = Cb^H H Cb with Cb = [C | C_P] (rocBLAS;
 //                     NextMatrix_z_blasmp, 1104-1436); P' normalised by its norm
@@ -517,7 +516,6 @@ struct qm_lobpcg {
     double *pen = nullptr;   // diagonal of dropped directions in the subspace problem (device, 1)
     void *rt = nullptr;      // S times the N lowest Ritz vectors (device, 3N x N subspace elements)
     void *dcw = nullptr;     // workspace of the tridiagonal divide and conquer (device)
-    void *psync = nullptr;   // barrier words of the cooperative Cholesky (device, 512 bytes)
     bool graphs = true;      // replay A.R + Gram of an iteration as a HIP graph
     hipStream_t gstream = nullptr;  // capture stream (graphs launch on the caller's stream)
     int graph_replays = 0;   // replays in the last solve
@@ -552,8 +550,6 @@ void lfree(qm_lobpcg *s) {
     s->rt = nullptr;
     if (s->dcw) (void)hipFree(s->dcw);
     s->dcw = nullptr;
-    if (s->psync) (void)hipFree(s->psync);
-    s->psync = nullptr;
     if (s->gstream) (void)hipStreamDestroy(s->gstream);
     s->gstream = nullptr;
     for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
@@ -590,11 +586,14 @@ int hpsi(qm_lobpcg *s, T *out, const T *in, int nb, int ik, hipStream_t st) {
     else return qm_hpsi_apply_f32(s->ctx, out, in, nb, s->c, ik, st);
 }
 
-// H c = l S c as in lapack_ZHEGVD_emu (w_zhegvd.h:227-272): S = U^H U (potrf),
-// C = U^-H H U^-1 (two trsm), eigh(C) (syevd), c = U^-1 y (trsm, first N columns).
-// Real n <= own_eig_max_n() instead factors S in one launch of the own
-// Cholesky, forms U^-1 once (trtri) and applies it by GEMMs, and diagonalises
-// C by the own tridiagonal reduction, divide and conquer and back-transformation.
+// whether S's Cholesky factor comes with its inverse (chol.hip), which the
+// solve then applies by GEMMs; else the library's factor and triangular solves
+bool own_chol(int n) { return subspace_route() < 0 && chol_inverse_supported(n); }
+
+// H c = l S c as in lapack_ZHEGVD_emu (w_zhegvd.h:227-272): S = U^H U with U^-1
+// in Ev (chol.hip), C = U^-H H U^-1 by two GEMMs, C diagonalised by the own
+// tridiagonal reduction, divide and conquer and back-transformation, c = U^-1 y
+// (N columns); orders above the own kernels' by potrf, trsm and syevd / heevd.
 // Works on copies Sw, Hw; eigenvalues in s->evals, eigenvectors in Hw.  After
 // potrf the squared pivot ratio is written to s->svals[0] for the caller's
 // conditioning check; on potrf failure s->info > 0 and the rest is skipped by
@@ -602,12 +601,16 @@ int hpsi(qm_lobpcg *s, T *out, const T *in, int nb, int ik, hipStream_t st) {
 template <bool CPLX>
 int chol_factor(qm_lobpcg *s, int n3, hipStream_t st) {
     using SmT = typename Sm<CPLX>::t;
-    QM_HIP(hipMemcpyAsync(s->Sw, s->S, sizeof(SmT) * n3 * n3, hipMemcpyDeviceToDevice, st));
     QM_HIP(hipMemcpyAsync(s->Hw, s->H, sizeof(SmT) * n3 * n3, hipMemcpyDeviceToDevice, st));
-    if constexpr (CPLX)
-        QM_BLAS(rocsolver_zpotrf(s->blas, rocblas_fill_upper, n3, (rocblas_double_complex *)s->Sw, n3, s->info));
-    else
-        QM_TRY(potrf_upper(s->blas, n3, (double *)s->Sw, n3, s->info, st, s->psync));
+    if (own_chol(n3)) {
+        QM_TRY(chol_inverse(n3, CPLX, s->S, s->T1, s->Sw, s->Ev, s->info, st));
+    } else {
+        QM_HIP(hipMemcpyAsync(s->Sw, s->S, sizeof(SmT) * n3 * n3, hipMemcpyDeviceToDevice, st));
+        if constexpr (CPLX)
+            QM_BLAS(rocsolver_zpotrf(s->blas, rocblas_fill_upper, n3, (rocblas_double_complex *)s->Sw, n3, s->info));
+        else
+            QM_TRY(potrf_upper(s->blas, n3, (double *)s->Sw, n3, s->info, st));
+    }
     hipLaunchKernelGGL((pivot_ratio_kernel<CPLX>), dim3(1), dim3(256), 0, st, s->svals, (const SmT *)s->Sw, n3);
     QM_HIP(hipGetLastError());
     return QM_OK;
@@ -619,10 +622,21 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
     if constexpr (CPLX) {
         const rocblas_double_complex one{1.0, 0.0};
         auto *U = (rocblas_double_complex *)s->Sw, *C = (rocblas_double_complex *)s->Hw;
-        QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_left, rocblas_fill_upper, rocblas_operation_conjugate_transpose,
-                              rocblas_diagonal_non_unit, n3, n3, &one, U, n3, C, n3));
-        QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                              rocblas_diagonal_non_unit, n3, n3, &one, U, n3, C, n3));
+        const rocblas_double_complex zero{0.0, 0.0};
+        const auto *Ui = (const rocblas_double_complex *)s->Ev;
+        if (own_chol(n3)) {
+            auto *T = (rocblas_double_complex *)s->T1;
+            QM_BLAS(rocblas_zgemm(s->blas, rocblas_operation_conjugate_transpose, rocblas_operation_none, n3, n3, n3,
+                                  &one, Ui, n3, C, n3, &zero, T, n3));
+            QM_BLAS(rocblas_zgemm(s->blas, rocblas_operation_none, rocblas_operation_none, n3, n3, n3, &one, T, n3, Ui,
+                                  n3, &zero, C, n3));
+        } else {
+            QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_left, rocblas_fill_upper,
+                                  rocblas_operation_conjugate_transpose, rocblas_diagonal_non_unit, n3, n3, &one, U,
+                                  n3, C, n3));
+            QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
+                                  rocblas_diagonal_non_unit, n3, n3, &one, U, n3, C, n3));
+        }
         if (subspace_route() != 0 && trd_coop_supported(n3, true) &&
             trd_coop_work_bytes(n3, true) <= sizeof(double) * (size_t)kTrdPanelCols * n3) {
             // own cooperative reduction C = Q T Q^H, divide and conquer on T (stedc
@@ -682,6 +696,12 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
                 }
                 QM_TRY(trd_coop_check(s->VW, s->info, st));
                 QM_TRY(unmtr_lower_z64(n3, N, C, n3, tau, Z, n3, s->VW, st));
+                if (own_chol(n3)) {  // C's reflectors have been applied: it takes the result
+                    QM_BLAS(rocblas_zgemm(s->blas, rocblas_operation_none, rocblas_operation_none, n3, N, n3, &one, Ui,
+                                          n3, Z, n3, &zero, C, n3));
+                    s->evec_t1 = false;
+                    return QM_OK;
+                }
                 QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_left, rocblas_fill_upper, rocblas_operation_none,
                                       rocblas_diagonal_non_unit, n3, N, &one, U, n3, Z, n3));
                 s->evec_t1 = true;
@@ -700,7 +720,7 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
             // C = U^-T H U^-1 through U^-1 and GEMMs, own tridiagonal reduction, divide
             // and conquer and back-transformation (eigenvectors in T1), then c = U^-1 y into Hw
             auto *Ui = (double *)s->Ev, *Z = (double *)s->T1;
-            QM_TRY(chol_transform(s->blas, n3, U, C, Ui, Z, st));
+            QM_TRY(chol_transform(s->blas, n3, U, C, Ui, own_chol(n3), Z, st));
             QM_TRY(syev_lower(s->blas, n3, N, C, n3, s->evals, Z, n3, s->trd, s->VW, s->dcw, s->info, st));
             QM_TRY(chol_back(s->blas, n3, N, Ui, Z, n3, C, n3));
             s->evec_t1 = false;
@@ -807,6 +827,26 @@ int svqb_eig(qm_lobpcg *s, int n3, double tau, hipStream_t st) {
     return QM_OK;
 }
 
+// W = [-XRn V; V] (2N x N) of the R orthonormalisation, V an N x N matrix
+template <bool CPLX>
+int rorth_basis(qm_lobpcg *s, const void *V, hipStream_t st) {
+    using SmT = typename Sm<CPLX>::t;
+    const int N = s->na;
+    if constexpr (CPLX) {
+        const rocblas_double_complex mone{-1.0, 0.0}, zero{0.0, 0.0};
+        QM_BLAS(rocblas_zgemm(s->blas, rocblas_operation_none, rocblas_operation_none, N, N, N, &mone,
+                              (rocblas_double_complex *)s->XRn, N, (const rocblas_double_complex *)V, N, &zero,
+                              (rocblas_double_complex *)s->Wr, 2 * N));
+    } else {
+        const double mone = -1.0, zero = 0.0;
+        QM_BLAS(rocblas_dgemm(s->blas, rocblas_operation_none, rocblas_operation_none, N, N, N, &mone,
+                              (double *)s->XRn, N, (const double *)V, N, &zero, (double *)s->Wr, 2 * N));
+    }
+    QM_HIP(hipMemcpy2DAsync((SmT *)s->Wr + N, sizeof(SmT) * 2 * N, V, sizeof(SmT) * N, sizeof(SmT) * N, N,
+                            hipMemcpyDeviceToDevice, st));
+    return QM_OK;
+}
+
 // R' = [X R] W: R orthogonalised against X (X^H X = I) and orthonormalised by a
 // Cholesky QR of M = Rn^H Rn - (X^H Rn)^H (X^H Rn), Rn = R diag(dr); when M is not
 // well conditioned, by its eigenbasis with the near-null directions dropped
@@ -838,12 +878,17 @@ int orthonormalise_r(qm_lobpcg *s, T *Rout, const T *X, const T *R, hipStream_t 
         QM_BLAS(rocblas_dgemm(s->blas, rocblas_operation_transpose, rocblas_operation_none, N, N, N, &mone,
                               (double *)s->XRn, N, (double *)s->XRn, N, &one, (double *)s->Mr, N));
     }
-    // Cholesky attempt on a copy (Sw is free at this point)
-    QM_HIP(hipMemcpyAsync(s->Sw, s->Mr, sizeof(SmT) * N * N, hipMemcpyDeviceToDevice, st));
-    if constexpr (CPLX)
-        QM_BLAS(rocsolver_zpotrf(s->blas, rocblas_fill_upper, N, (rocblas_double_complex *)s->Sw, N, s->info));
-    else
-        QM_TRY(potrf_upper(s->blas, N, (double *)s->Sw, N, s->info, st, s->psync));
+    // Cholesky attempt (Sw, T1 and Ev are free at this point)
+    const bool own = own_chol(N);
+    if (own) {
+        QM_TRY(chol_inverse(N, CPLX, s->Mr, s->T1, s->Sw, s->Ev, s->info, st));
+    } else {
+        QM_HIP(hipMemcpyAsync(s->Sw, s->Mr, sizeof(SmT) * N * N, hipMemcpyDeviceToDevice, st));
+        if constexpr (CPLX)
+            QM_BLAS(rocsolver_zpotrf(s->blas, rocblas_fill_upper, N, (rocblas_double_complex *)s->Sw, N, s->info));
+        else
+            QM_TRY(potrf_upper(s->blas, N, (double *)s->Sw, N, s->info, st));
+    }
     hipLaunchKernelGGL((pivot_ratio_kernel<CPLX>), dim3(1), dim3(256), 0, st, s->svals, (const SmT *)s->Sw, N);
     QM_HIP(hipGetLastError());
     int h_info = 0;
@@ -854,18 +899,22 @@ int orthonormalise_r(qm_lobpcg *s, T *Rout, const T *X, const T *R, hipStream_t 
     const double drop = sizeof(T) == 8 ? s->rdrop64 : s->rdrop32;
     const unsigned gW = (unsigned)(((int64_t)2 * N * N + 255) / 256);
     if (h_info == 0 && h_ratio >= drop) {
-        hipLaunchKernelGGL((rorth_w_kernel<CPLX>), dim3(gW), dim3(256), 0, st, (SmT *)s->Wr, (const SmT *)s->XRn, N);
-        QM_HIP(hipGetLastError());
-        if constexpr (CPLX) {
-            const rocblas_double_complex one{1.0, 0.0};
-            QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                                  rocblas_diagonal_non_unit, 2 * N, N, &one, (rocblas_double_complex *)s->Sw, N,
-                                  (rocblas_double_complex *)s->Wr, 2 * N));
+        if (own) {
+            QM_TRY(rorth_basis<CPLX>(s, s->Ev, st));
         } else {
-            const double one = 1.0;
-            QM_BLAS(rocblas_dtrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                                  rocblas_diagonal_non_unit, 2 * N, N, &one, (double *)s->Sw, N, (double *)s->Wr,
-                                  2 * N));
+            hipLaunchKernelGGL((rorth_w_kernel<CPLX>), dim3(gW), dim3(256), 0, st, (SmT *)s->Wr, (const SmT *)s->XRn, N);
+            QM_HIP(hipGetLastError());
+            if constexpr (CPLX) {
+                const rocblas_double_complex one{1.0, 0.0};
+                QM_BLAS(rocblas_ztrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
+                                      rocblas_diagonal_non_unit, 2 * N, N, &one, (rocblas_double_complex *)s->Sw, N,
+                                      (rocblas_double_complex *)s->Wr, 2 * N));
+            } else {
+                const double one = 1.0;
+                QM_BLAS(rocblas_dtrsm(s->blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
+                                      rocblas_diagonal_non_unit, 2 * N, N, &one, (double *)s->Sw, N, (double *)s->Wr,
+                                      2 * N));
+            }
         }
         hipLaunchKernelGGL(fill_kernel, dim3((N + 63) / 64), dim3(64), 0, st, s->rkeep, 1.0, N);
         QM_HIP(hipGetLastError());
@@ -876,21 +925,7 @@ int orthonormalise_r(qm_lobpcg *s, T *Rout, const T *X, const T *R, hipStream_t 
         hipLaunchKernelGGL((rorth_svqb_kernel<CPLX>), dim3((unsigned)(((int64_t)N * N + 255) / 256)), dim3(256), 0,
                            st, (SmT *)s->Sw, s->rkeep, s->svals, N, drop);
         QM_HIP(hipGetLastError());
-        // W = [-XRn Vs ; Vs]
-        if constexpr (CPLX) {
-            const rocblas_double_complex mone{-1.0, 0.0}, zero{0.0, 0.0};
-            QM_BLAS(rocblas_zgemm(s->blas, rocblas_operation_none, rocblas_operation_none, N, N, N, &mone,
-                                  (rocblas_double_complex *)s->XRn, N, (rocblas_double_complex *)s->Sw, N, &zero,
-                                  (rocblas_double_complex *)s->Wr, 2 * N));
-            QM_HIP(hipMemcpy2DAsync((rocblas_double_complex *)s->Wr + N, sizeof(SmT) * 2 * N, s->Sw, sizeof(SmT) * N,
-                                    sizeof(SmT) * N, N, hipMemcpyDeviceToDevice, st));
-        } else {
-            const double mone = -1.0, zero = 0.0;
-            QM_BLAS(rocblas_dgemm(s->blas, rocblas_operation_none, rocblas_operation_none, N, N, N, &mone,
-                                  (double *)s->XRn, N, (double *)s->Sw, N, &zero, (double *)s->Wr, 2 * N));
-            QM_HIP(hipMemcpy2DAsync((double *)s->Wr + N, sizeof(SmT) * 2 * N, s->Sw, sizeof(SmT) * N, sizeof(SmT) * N,
-                                    N, hipMemcpyDeviceToDevice, st));
-        }
+        QM_TRY(rorth_basis<CPLX>(s, s->Sw, st));
         ++s->rdrops;
     }
     hipLaunchKernelGGL((rorth_scale_kernel<CPLX>), dim3(gW), dim3(256), 0, st, (SmT *)s->Wr, s->dr, N);
@@ -1488,7 +1523,6 @@ int qm_lobpcg_create(qm_lobpcg **out, qm_ctx *ctx, int nbands, int ncomp, int pr
     if (st == QM_OK) st = dalloc((void **)&s->evk, sizeof(double) * N);
     if (st == QM_OK) st = dalloc((void **)&s->pen, sizeof(double));
     if (st == QM_OK) st = dalloc(&s->rt, esz * (size_t)n3 * N);
-    if (st == QM_OK) st = dalloc(&s->psync, 512);
     // every order a solve can meet: up to 3 N, of which those above the limit take stedc
     if (st == QM_OK) st = dalloc(&s->dcw, tridiag_dc_work_bytes(std::min(n3, tridiag_dc_max())));
     if (st == QM_OK && hipStreamCreateWithFlags(&s->gstream, hipStreamNonBlocking) != hipSuccess) {

@@ -200,18 +200,18 @@ size_t tridiag_dc_work_bytes(int n);
 int tridiag_dc(int n, int nev, const double *d, const double *e, double *w, double *Z, int ldz, bool cplx, void *work,
                int *info, hipStream_t st);
 int own_eig_max_n();
-// A = U^T U, upper triangle of the column-major n x n A (FP64): with sync (512
-// bytes of device memory) and n <= 512, one workgroup per 32-row panel
-// (potrf_coop_f64); else one workgroup for n <= own_eig_max_n(), rocSOLVER
-// above; *info (device) as LAPACK's dpotrf.
-int potrf_upper(void *blas, int n, double *A, int lda, int *info, hipStream_t st, void *sync = nullptr);
-// trd_coop.hip: the cooperative Cholesky (QM_ERR_STATE when it cannot run: the
-// caller takes another kernel); *info as dpotrf, -77 if a barrier wait timed out
-int potrf_coop_supported(int n);
-int potrf_coop_f64(int n, double *A, int lda, int *info, void *sync, hipStream_t st);
+// A = U^T U, upper triangle of the column-major n x n A (FP64), in place: one
+// workgroup for n <= own_eig_max_n(), rocSOLVER above; *info (device) as LAPACK's dpotrf
+int potrf_upper(void *blas, int n, double *A, int lda, int *info, hipStream_t st);
+// chol.hip: A = U^H U and Ui = U^-1 (its strictly lower triangle zero), real or
+// complex, from A's upper triangle (not modified); W: n x n work; all leading
+// dimension n and distinct; only U's upper triangle is written; *info as potrf
+int chol_inverse_supported(int n);
+int chol_inverse(int n, bool cplx, const void *A, void *W, void *U, void *Ui, int *info, hipStream_t st);
 // C := U^-T C U^-1 with Ui = U^-1 kept (n x n each, leading dimension n; T: n x n work),
 // and Zout = Ui Z: the two halves of the Cholesky route around the eigensolve.
-int chol_transform(void *blas, int n, const double *U, double *C, double *Ui, double *T, hipStream_t st);
+// have_ui: Ui already holds U^-1 (chol_inverse), else it is formed here
+int chol_transform(void *blas, int n, const double *U, double *C, double *Ui, bool have_ui, double *T, hipStream_t st);
 int chol_back(void *blas, int n, int nev, const double *Ui, const double *Z, int ldz, double *Zout, int ldo);
 constexpr int kTrdPanelCols = 96;  // VW workspace columns (n x 96) of sytrd_lower
 
