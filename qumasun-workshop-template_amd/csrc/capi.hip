@@ -110,6 +110,9 @@ static void free_projectors(Projectors &p) {
     dfree(p.d_block_atom_off);
     dfree(p.d_block_atoms);
     dfree(p.d_cov_slot);
+    dfree(p.d_tile_row_off);
+    dfree(p.d_row_atom);
+    dfree(p.d_tile_vox);
     p = Projectors();
 }
 
@@ -190,6 +193,8 @@ static int build_projectors(const qm_ctx *ctx, Projectors &p, int natoms, const 
     p.ncov = (int)m.cov_grid.size();
     p.nchunk = (int)m.chunk_atom.size();
     p.nsblock = (int)m.block_atom_off.size() - 1;
+    p.ntile = (int)m.tile_row_off.size() - 1;
+    m.cov_grid.resize((size_t)p.ntile * kScatterTile, -1);
 
     std::vector<float> t32(table, table + p.ttot);
     QM_TRY(upload(&p.d_nproj, nproj, natoms));
@@ -220,6 +225,9 @@ static int build_projectors(const qm_ctx *ctx, Projectors &p, int natoms, const 
     QM_TRY(upload(&p.d_block_atom_off, m.block_atom_off.data(), m.block_atom_off.size()));
     QM_TRY(upload(&p.d_block_atoms, m.block_atoms.data(), m.block_atoms.size()));
     QM_TRY(upload(&p.d_cov_slot, m.cov_slot.data(), m.cov_slot.size()));
+    QM_TRY(upload(&p.d_tile_row_off, m.tile_row_off.data(), m.tile_row_off.size()));
+    QM_TRY(upload(&p.d_row_atom, m.row_atom.data(), m.row_atom.size()));
+    QM_TRY(upload(&p.d_tile_vox, m.tile_vox.data(), m.tile_vox.size()));
     return QM_OK;
 }
 

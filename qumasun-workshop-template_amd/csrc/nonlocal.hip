@@ -212,8 +212,7 @@ __global__ void nl_coef_kernel(T *__restrict__ coef, const double *__restrict__ 
 // g (logical block = point block * groups + g).  The coefficients of the (up to kScatterSlots) atoms a workgroup
 // touches are staged in LDS; each thread reads its point's entry list and
 // table rows once for the whole group.  MP: projector slots per entry (9 when
-// every atom has at most 9 projectors, l <= 2, else the table padding 16 or
-// 32); table rows are MS = 16 (MP <= 16) or 32 values apart.
+// every atom has at most 9 projectors, l <= 2, else the table padding of 16).
 template <typename T, int NC, bool PH, int NBS, int GT, int MP>
 __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
     T *__restrict__ hpsi, const T *__restrict__ coef, int64_t ng, int ncol, int ncov,
@@ -222,7 +221,7 @@ __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
     const int *__restrict__ vox_atom, const int *__restrict__ nproj, const int *__restrict__ proj_off,
     const T *__restrict__ tabp, const T *__restrict__ phase, int groups, int nblk, int per_xcd) {
     constexpr int NG = NBS * GT;  // columns of the group
-    constexpr int MS = MP > 16 ? 32 : 16;
+    constexpr int MS = 16;  // table row padding
     __shared__ T cf_s[kScatterSlots][MP][NG];
     const int lb = xcd_block(nblk, per_xcd);
     if (lb < 0) return;  // the whole workgroup
@@ -311,6 +310,143 @@ __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
 #pragma unroll
     for (int q = 0; q < NG; ++q)
         if (cg + q < ncol) hpsi[(int64_t)(cg + q) * ng + g] = hv[q];
+}
+
+// The same sums on the matrix cores, for FP64 and for more than 16 projectors,
+// where nl_scatter_kernel is bound by its broadcast LDS reads of the
+// coefficients (one per point, column and projector).  A wave owns 16 PT
+// covered points x 16 CT columns and takes the atoms of its tile one after the
+// other: columns are the rows of the result (A: coefficients), points its
+// columns (B: table rows) and projectors K, so each coefficient and table
+// value is read once per 16 x 16 outputs.  K may run in any order: lane group q takes
+// projectors KS q .. KS q + KS - 1, consecutive in the table row (KS: steps of
+// 4 projectors; rows MS values apart).  A lane's 4 results are 4 consecutive
+// columns in either precision (re and im of a band together, for the phase);
+// an atom's results are added only at the points its sphere covers.  The sums
+// then change lanes through LDS, so that Hpsi is read and written with lanes
+// along the points (without it 64^3 x 64 complex took 110 us instead of 95).
+// Hpsi's lines bound it: 64^3 x 64 complex FP64, 16 atoms, 0.41 GB of 128 B
+// lines, 103 -> 95 us (4.3 TB/s); 45x54x50 x 37 complex FP64, 32 projectors,
+// 45 -> 29 us (FP32 34 -> 22; 64^3 x 128 FP32 116 -> 82); 32^3 x 24 FP64 6.5 ->
+// 5.2 us.  FP32 with up to 16 projectors
+// stays with nl_scatter_kernel (64^3 x 128: 53 us there, 61 here; 160^3 x 512:
+// 3.19 and 3.41 ms): half the LDS bytes a coefficient, and 32 columns a thread.
+template <typename T, int NC, bool PH, int KS, int CT, int PT>
+__global__ __launch_bounds__(256) void nl_scatter_mfma_kernel(
+    T *__restrict__ hpsi, const T *__restrict__ coef, int64_t ng, int ncol, int ntile,
+    const int *__restrict__ cov_grid, const int *__restrict__ tile_row_off, const int *__restrict__ row_atom,
+    const int *__restrict__ tile_vox, const int *__restrict__ nproj, const int *__restrict__ proj_off,
+    const T *__restrict__ tabp, const T *__restrict__ phase, int groups, int nblk,
+    int per_xcd) {
+    using M = Mfma<T>;
+    using acc_t = typename M::acc_t;
+    constexpr int MS = KS > 4 ? 32 : 16;
+    constexpr int SUBS = 4 / PT;               // waves per tile
+    constexpr int P = 16 * PT, NV = CT * 4 * PT;  // a wave's points; values a lane moves
+    __shared__ T stage[4][16 * CT][P + 16 / (int)sizeof(T)];
+    const int lb = xcd_block(nblk, per_xcd);
+    if (lb < 0) return;
+    const int pb = lb / groups;
+    const int cg = (lb - pb * groups) * 16 * CT;
+    const int wave = threadIdx.x >> 6;
+    const int sub = __builtin_amdgcn_readfirstlane(pb * 4 + wave);
+    const int tile = sub / SUBS, t0 = (sub % SUBS) * PT;
+    if (tile >= ntile) return;  // the whole wave
+    const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+    // result row i of A holds column 4 (row's lane group) + (its item)
+    const int ai = sizeof(T) == 8 ? 4 * (j & 3) + (j >> 2) : j;
+    const int r0 = tile_row_off[tile], r1 = tile_row_off[tile + 1];  // r1 > r0: a covered point has an entry
+    // the values of Hpsi are read and written with lanes along the points
+    const int mp = lane & (P - 1), mc = lane / P;
+    const int gi = cov_grid[tile * kScatterTile + 16 * t0 + mp];
+    int vid[PT];
+    T a[CT][KS], b[PT][KS];
+    T cs[PT], sn[PT];
+    // one row's voxels, coefficients, table rows and phases
+    auto load_row = [&](int r) {
+        const int at = row_atom[r], po = proj_off[at], np = nproj[at];
+        const int *tv = tile_vox + (int64_t)r * kScatterTile + 4 * j + t0;
+#pragma unroll
+        for (int t = 0; t < PT; ++t) vid[t] = tv[t];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int col = cg + 16 * ct + ai;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int w = KS * q + s;
+                a[ct][s] = (w < np && col < ncol) ? coef[(int64_t)(po + w) * ncol + col] : T(0);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            const int64_t v = max(vid[t], 0);
+            const T *tr = tabp + v * MS + KS * q;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) b[t][s] = tr[s];
+            if constexpr (PH) {
+                cs[t] = phase[2 * v];
+                sn[t] = phase[2 * v + 1];
+            }
+        }
+    };
+    load_row(r0);
+    // requested behind the first row's operands, which the first products wait for
+    T *hp = hpsi + (int64_t)(cg + mc) * ng + max(gi, 0);
+    T hv[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+        hv[u] = cg + mc + u * (64 / P) < ncol ? hp[(int64_t)u * (64 / P) * ng] : T(0);
+    T sum[PT][CT][4];
+#pragma unroll
+    for (int t = 0; t < PT; ++t)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[t][ct][e] = T(0);
+    for (int r = r0;;) {
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            if (__ballot(vid[t] >= 0) == 0) continue;  // uniform
+            acc_t acc[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                acc[ct] = acc_t{0, 0, 0, 0};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) acc[ct] = M::mma(a[ct][s], b[t][s], acc[ct]);
+            }
+            // the table row behind a negative voxel is another point's: its
+            // sums stay in their own column and are not added
+            if (vid[t] >= 0) {
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int e = 0; e < 4; e += NC) {
+                        if constexpr (PH) {
+                            sum[t][ct][e] += cs[t] * acc[ct][e] + sn[t] * acc[ct][e + 1];
+                            sum[t][ct][e + 1] += cs[t] * acc[ct][e + 1] - sn[t] * acc[ct][e];
+                        } else {
+                            sum[t][ct][e] += acc[ct][e];
+                            if constexpr (NC == 2) sum[t][ct][e + 1] += acc[ct][e + 1];
+                        }
+                    }
+            }
+        }
+        if (++r >= r1) break;
+        load_row(r);
+    }
+    // the sums change lanes through the wave's own LDS slice
+#pragma unroll
+    for (int t = 0; t < PT; ++t)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) stage[wave][16 * ct + 4 * q + e][16 * t + j] = sum[t][ct][e];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (gi < 0) return;
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+        if (cg + mc + u * (64 / P) < ncol)
+            hp[(int64_t)u * (64 / P) * ng] = hv[u] + stage[wave][mc + u * (64 / P)][mp];
 }
 
 // ---- forces -------------------------------------------------------------
@@ -652,34 +788,57 @@ int nonlocal_project(qm_ctx *ctx, T *coef, double *part, const T *psi, int nb, c
     return QM_OK;
 }
 
+template <typename T, int NC, bool PH, int KS, int CT, int PT>
+int launch_scatter_mfma(qm_ctx *ctx, T *hpsi, const T *coef, int ncol, const T *phase, hipStream_t st) {
+    const Projectors &p = ctx->proj;
+    const int groups = (ncol + 16 * CT - 1) / (16 * CT);
+    const int64_t nblk = (int64_t)((p.ntile + PT - 1) / PT) * groups;
+    QM_CHECK(nblk < (int64_t)INT32_MAX / 16, QM_ERR_ARG, "nonlocal apply: too many bands per call");
+    const int per_xcd = (int)((nblk + 7) / 8);
+    hipLaunchKernelGGL((nl_scatter_mfma_kernel<T, NC, PH, KS, CT, PT>), dim3(8 * per_xcd), dim3(256), 0, st, hpsi,
+                       coef, ctx->ng, ncol, p.ntile, p.d_cov_grid, p.d_tile_row_off, p.d_row_atom, p.d_tile_vox,
+                       p.d_nproj, p.d_proj_off, tabp_of<T>(p), phase, groups, (int)nblk, per_xcd);
+    QM_HIP(hipGetLastError());
+    return QM_OK;
+}
+
+// 32 points x 32 columns a wave; 16 x 16 where that leaves less than 2 waves a
+// SIMD (32^3 x 24 FP64: 576 waves 6.9 us, 2272 waves 5.2 us; 36x40x42 x 45
+// complex: 3100 waves 21 us, 12400 waves 24 us)
+constexpr int64_t kScatterWaves = 2048;
+template <typename T, int NC, bool PH, int KS>
+int scatter_mfma(qm_ctx *ctx, T *hpsi, const T *coef, int ncol, const T *phase, hipStream_t st) {
+    const int64_t waves = (int64_t)ctx->proj.ntile * 2 * ((ncol + 31) / 32);
+    if (waves >= kScatterWaves) return launch_scatter_mfma<T, NC, PH, KS, 2, 2>(ctx, hpsi, coef, ncol, phase, st);
+    return launch_scatter_mfma<T, NC, PH, KS, 1, 1>(ctx, hpsi, coef, ncol, phase, st);
+}
+
 template <typename T, int NC, bool PH>
 int nonlocal_scatter(qm_ctx *ctx, T *hpsi, const T *coef, int nb, const T *phase, hipStream_t st) {
     const Projectors &p = ctx->proj;
     const int ncol = nb * NC;
-    // columns per scatter tile (16; 64 per thread measured 1.9x slower on
-    // 64^3 x 128) and tiles per workgroup (the staged coefficients, entry lists
-    // and table rows serve all of them)
-    constexpr int NBS = 16;
-    constexpr int SGT = sizeof(T) == 8 ? 1 : 2;
-    const int sgroups = (ncol + NBS * SGT - 1) / (NBS * SGT);
-    const int64_t nblk = (int64_t)p.nsblock * sgroups;
-    QM_CHECK(nblk < (int64_t)INT32_MAX / 16, QM_ERR_ARG, "nonlocal apply: too many bands per call");
-    const int per_xcd = (int)((nblk + 7) / 8);
-    if (p.max_m <= 9)
-        hipLaunchKernelGGL((nl_scatter_kernel<T, NC, PH, NBS, SGT, 9>), dim3(8 * per_xcd), dim3(kScatterBlock), 0, st,
-                           hpsi, coef, ctx->ng, ncol, p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox, p.d_cov_slot,
-                           p.d_block_atom_off, p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off,
-                           tabp_of<T>(p), phase, sgroups, (int)nblk, per_xcd);
-    else if (p.max_m <= 16)
-        hipLaunchKernelGGL((nl_scatter_kernel<T, NC, PH, NBS, SGT, 16>), dim3(8 * per_xcd), dim3(kScatterBlock),
-                           0, st, hpsi, coef, ctx->ng, ncol, p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox,
-                           p.d_cov_slot, p.d_block_atom_off, p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off,
-                           tabp_of<T>(p), phase, sgroups, (int)nblk, per_xcd);
-    else
-        hipLaunchKernelGGL((nl_scatter_kernel<T, NC, PH, NBS, SGT, 32>), dim3(8 * per_xcd), dim3(kScatterBlock),
-                           0, st, hpsi, coef, ctx->ng, ncol, p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox,
-                           p.d_cov_slot, p.d_block_atom_off, p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off,
-                           tabp_of<T>(p), phase, sgroups, (int)nblk, per_xcd);
+    if (p.max_m > 16) return scatter_mfma<T, NC, PH, 8>(ctx, hpsi, coef, ncol, phase, st);
+    if constexpr (sizeof(T) == 8) {
+        if (p.max_m > 12) return scatter_mfma<T, NC, PH, 4>(ctx, hpsi, coef, ncol, phase, st);
+        return scatter_mfma<T, NC, PH, 3>(ctx, hpsi, coef, ncol, phase, st);
+    } else {
+        // columns per scatter tile (16; 64 per thread measured 1.9x slower on
+        // 64^3 x 128) and tiles per workgroup (the staged coefficients, entry lists
+        // and table rows serve all of them)
+        constexpr int NBS = 16, SGT = 2;
+        const int sgroups = (ncol + NBS * SGT - 1) / (NBS * SGT);
+        const int64_t nblk = (int64_t)p.nsblock * sgroups;
+        QM_CHECK(nblk < (int64_t)INT32_MAX / 16, QM_ERR_ARG, "nonlocal apply: too many bands per call");
+        const int per_xcd = (int)((nblk + 7) / 8);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(8 * per_xcd), dim3(kScatterBlock), 0, st, hpsi, coef, ctx->ng, ncol,
+                               p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox, p.d_cov_slot, p.d_block_atom_off,
+                               p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off, tabp_of<T>(p), phase, sgroups,
+                               (int)nblk, per_xcd);
+        };
+        if (p.max_m <= 9) launch(nl_scatter_kernel<T, NC, PH, NBS, SGT, 9>);
+        else launch(nl_scatter_kernel<T, NC, PH, NBS, SGT, 16>);
+    }
     QM_HIP(hipGetLastError());
     return QM_OK;
 }

@@ -19,6 +19,7 @@ namespace qm {
 constexpr int kProjChunk = 512;     // voxels per projection work item (4 waves x 128)
 constexpr int kScatterBlock = 256;  // covered points per scatter workgroup
 constexpr int kScatterSlots = 8;    // atoms whose coefficients a scatter workgroup stages in LDS
+constexpr int kScatterTile = 64;    // covered points per tile of the MFMA scatter (4 x 16)
 
 // periodic wrap of a grid coordinate into 0 .. n-1
 inline int wrap_index(int i, int n) {
@@ -41,6 +42,12 @@ struct ProjectorMaps {
     // per scatter block of kScatterBlock covered points: its distinct atoms
     // (at most kScatterSlots staged) and each voxel entry's slot (-1: not staged)
     std::vector<int> block_atom_off, block_atoms, cov_slot;
+    // per tile of kScatterTile covered points, one row per atom that covers any
+    // of them: the atom's voxel at the tile's point 16 t + j is
+    // tile_vox[64 row + 4 j + t], -1 where its sphere does not reach.  An atom
+    // that covers a point more than once (a sphere wider than the cell) has
+    // further rows, so that every entry is in exactly one.
+    std::vector<int> tile_row_off, row_atom, tile_vox;
 };
 
 inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *nproj, const int64_t *vox_off,
@@ -135,6 +142,32 @@ inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *
         m.block_atom_off[b + 1] = (int)m.block_atoms.size();
     }
     if (m.block_atoms.empty()) m.block_atoms.push_back(0);
+    // MFMA scatter: every entry goes to the first row of its atom, in this tile,
+    // that has no entry yet at its point
+    const int ntile = (ncov + kScatterTile - 1) / kScatterTile;
+    m.tile_row_off.assign(ntile + 1, 0);
+    m.row_atom.clear();
+    m.tile_vox.clear();
+    for (int b = 0; b < ntile; ++b) {
+        const int i0 = b * kScatterTile, i1 = std::min(ncov, i0 + kScatterTile);
+        const size_t r0 = m.row_atom.size();
+        for (int i = i0; i < i1; ++i) {
+            const int p = 4 * ((i - i0) & 15) + ((i - i0) >> 4);
+            for (int e = m.cov_off[i]; e < m.cov_off[i + 1]; ++e) {
+                const int a = m.atom[m.cov_vox[e]];
+                size_t r = r0;
+                while (r < m.row_atom.size() &&
+                       (m.row_atom[r] != a || m.tile_vox[r * kScatterTile + p] >= 0))
+                    ++r;
+                if (r == m.row_atom.size()) {
+                    m.row_atom.push_back(a);
+                    m.tile_vox.resize((r + 1) * kScatterTile, -1);
+                }
+                m.tile_vox[r * kScatterTile + p] = m.cov_vox[e];
+            }
+        }
+        m.tile_row_off[b + 1] = (int)m.row_atom.size();
+    }
 }
 
 }  // namespace qm

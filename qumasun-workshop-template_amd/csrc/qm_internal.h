@@ -82,7 +82,7 @@ struct Projectors {
     float *d_table32 = nullptr, *d_dtable32 = nullptr;
     // owner-computes scatter map: covered grid points, each with its list of voxels
     int ncov = 0;
-    int *d_cov_grid = nullptr;           // [ncov] grid index
+    int *d_cov_grid = nullptr;           // [ntile * kScatterTile] grid index, -1 past ncov
     int *d_cov_off = nullptr;            // [ncov+1]
     int *d_cov_vox = nullptr;            // [vtot] global voxel ids grouped by covered point
     // atom work list for the projection launch, longest atoms first
@@ -101,6 +101,10 @@ struct Projectors {
     // the block touches more than kScatterSlots atoms)
     int nsblock = 0;
     int *d_block_atom_off = nullptr, *d_block_atoms = nullptr, *d_cov_slot = nullptr;
+    // MFMA scatter: rows of each tile of kScatterTile covered points (one per
+    // atom that reaches it), their atoms and voxels (ProjectorMaps::tile_vox)
+    int ntile = 0;
+    int *d_tile_row_off = nullptr, *d_row_atom = nullptr, *d_tile_vox = nullptr;
 };
 
 
