@@ -741,6 +741,12 @@ int update_tiled(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int
 
 template <typename T>
 int update(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int n, int64_t ng, hipStream_t st) {
+    if constexpr (sizeof(T) == 4) {
+        // from 192 workgroups on (128 x 128 over 32,768 points, 128 workgroups: 42 us
+        // split, 32 tiled; 192 x 128 over 64,000, 250: 51 and 53; 270 x 180 over
+        // 60,480, 237: 83 and 119 us)
+        if (n >= 128 && split_update_fits(Z, m, n, ng)) return split_update(Z, Y, Cm, m, n, ng, st);
+    }
     if (n >= UT_N && ng % UT_P == 0 && m % UpdShape<T>::KT == 0 && aligned16(Z) && aligned16(Y) &&
         reinterpret_cast<uintptr_t>(Cm) % 16 == 0)
         return update_tiled<T>(Z, Y, Cm, m, n, ng, st);

@@ -316,6 +316,9 @@ int gram(DevBuf &partial, double *C, const ColBlocks &A, const ColBlocks &B, int
          hipStream_t st);
 template <typename T>
 int update(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int n, int64_t ng, hipStream_t st);
+// split_gemm.hip: the FP32 update on the bf16 matrix cores, where it fits (any ng and alignment)
+bool split_update_fits(const ColBlocks &Z, int m, int n, int64_t ng);
+int split_update(const ColBlocks &Z, const ColBlocks &Y, const float *Cm, int m, int n, int64_t ng, hipStream_t st);
 template <typename T>
 int band_reduce(DevBuf &part, int mode, double *out0, double *out1, T *r, const T *x, const T *ax, const double *lam,
                 int nb, int ncomp, int64_t ng, hipStream_t st);
