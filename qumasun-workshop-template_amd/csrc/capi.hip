@@ -189,7 +189,7 @@ static int build_projectors(const qm_ctx *ctx, Projectors &p, int natoms, const 
 
     ProjectorMaps m;
     build_projector_maps(ctx->nx, ctx->ny, ctx->nz, natoms, nproj, vox_off, vox_xyz, table, tab_off, proj_off,
-                         p.mpad, m);
+                         p.mpad, m, false);
     p.ncov = (int)m.cov_grid.size();
     p.nchunk = (int)m.chunk_atom.size();
     p.nsblock = (int)m.block_atom_off.size() - 1;
@@ -216,8 +216,7 @@ static int build_projectors(const qm_ctx *ctx, Projectors &p, int natoms, const 
     QM_TRY(upload(&p.d_cov_vox, m.cov_vox.data(), m.cov_vox.size()));
     QM_TRY(upload(&p.d_atom_order, m.atom_order.data(), m.atom_order.size()));
     QM_TRY(upload(&p.d_item_order, m.item_order.data(), m.item_order.size()));
-    QM_TRY(upload(&p.d_tabp_64, m.tabp64.data(), m.tabp64.size()));
-    QM_TRY(upload(&p.d_tabp_32, m.tabp32.data(), m.tabp32.size()));
+    QM_TRY(padded_tables(p));
     QM_TRY(upload(&p.d_chunk_atom, m.chunk_atom.data(), m.chunk_atom.size()));
     QM_TRY(upload(&p.d_chunk_v0, m.chunk_v0.data(), m.chunk_v0.size()));
     QM_TRY(upload(&p.d_atom_chunk_off, m.atom_chunk_off.data(), m.atom_chunk_off.size()));

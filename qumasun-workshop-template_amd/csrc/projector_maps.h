@@ -33,7 +33,7 @@ struct ProjectorMaps {
     // its voxels cov_vox[cov_off[i] .. cov_off[i+1]-1]
     std::vector<int> cov_grid, cov_off, cov_vox;
     std::vector<int> atom_order;  // heaviest atoms (V_a M_a) first
-    // voxel-major tables padded to mpad projectors: tabp[v mpad + w]
+    // voxel-major tables padded to mpad projectors: tabp[v mpad + w] (with_tables)
     std::vector<double> tabp64;
     std::vector<float> tabp32;
     // projection work items (chunks of kProjChunk voxels of one atom), the
@@ -52,7 +52,7 @@ struct ProjectorMaps {
 
 inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *nproj, const int64_t *vox_off,
                                  const int *vox_xyz, const double *table, const int64_t *tab_off,
-                                 const int *proj_off, int mpad, ProjectorMaps &m) {
+                                 const int *proj_off, int mpad, ProjectorMaps &m, bool with_tables = true) {
     const int64_t vtot = vox_off[natoms];
     const int ptot = proj_off[natoms];
     m.grid.assign(vtot, 0);
@@ -63,19 +63,21 @@ inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *
                         nx * (wrap_index(vox_xyz[3 * v + 1], ny) + ny * wrap_index(vox_xyz[3 * v + 2], nz));
             m.atom[v] = a;
         }
-    // covered-point map: voxels sorted by grid point
-    m.cov_vox.resize(vtot);
-    std::iota(m.cov_vox.begin(), m.cov_vox.end(), 0);
-    std::stable_sort(m.cov_vox.begin(), m.cov_vox.end(), [&](int x, int y) { return m.grid[x] < m.grid[y]; });
+    // covered-point map: voxels sorted by grid point, in their own order at each
+    // (a counting sort over the grid)
+    std::vector<int> at((size_t)nx * ny * nz + 1, 0);
+    for (int64_t v = 0; v < vtot; ++v) ++at[m.grid[v] + 1];
     m.cov_grid.clear();
     m.cov_off.clear();
-    m.cov_off.reserve(vtot + 1);
-    for (int64_t i = 0; i < vtot; ++i) {
-        if (i == 0 || m.grid[m.cov_vox[i]] != m.grid[m.cov_vox[i - 1]]) {
-            m.cov_grid.push_back(m.grid[m.cov_vox[i]]);
-            m.cov_off.push_back((int)i);
+    for (size_t g = 0; g + 1 < at.size(); ++g) {
+        if (at[g + 1] > 0) {
+            m.cov_grid.push_back((int)g);
+            m.cov_off.push_back(at[g]);
         }
+        at[g + 1] += at[g];
     }
+    m.cov_vox.resize(vtot);
+    for (int64_t v = 0; v < vtot; ++v) m.cov_vox[at[m.grid[v]]++] = (int)v;
     m.cov_off.push_back((int)vtot);
     const int ncov = (int)m.cov_grid.size();
     m.atom_order.resize(natoms);
@@ -84,8 +86,8 @@ inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *
         return (vox_off[x + 1] - vox_off[x]) * nproj[x] > (vox_off[y + 1] - vox_off[y]) * nproj[y];
     });
     // padded voxel-major tables and the projection work list
-    m.tabp64.assign((size_t)vtot * mpad, 0.0);
-    m.tabp32.assign((size_t)vtot * mpad, 0.0f);
+    m.tabp64.assign(with_tables ? (size_t)vtot * mpad : 0, 0.0);
+    m.tabp32.assign(with_tables ? (size_t)vtot * mpad : 0, 0.0f);
     m.chunk_atom.clear();
     m.chunk_v0.clear();
     m.atom_chunk_off.assign(natoms + 1, 0);
@@ -94,7 +96,7 @@ inline void build_projector_maps(int nx, int ny, int nz, int natoms, const int *
         const int64_t V = vox_off[a + 1] - vox_off[a];
         for (int w = 0; w < nproj[a]; ++w) {
             m.proj_atom[proj_off[a] + w] = a;
-            for (int64_t v = 0; v < V; ++v) {
+            for (int64_t v = 0; with_tables && v < V; ++v) {
                 const double val = table[tab_off[a] + w * V + v];
                 m.tabp64[(size_t)(vox_off[a] + v) * mpad + w] = val;
                 m.tabp32[(size_t)(vox_off[a] + v) * mpad + w] = (float)val;

@@ -270,6 +270,8 @@ int spectral_poisson(const qm_ctx *ctx, const SpectralTables *t, void *spec, dou
 void spectral_destroy(SpectralTables *t);
 
 // nonlocal.hip
+// allocates and fills the voxel-major padded tables from the uploaded ones (null stream)
+int padded_tables(Projectors &p);
 int launch_nonlocal_f64(qm_ctx *ctx, double *hpsi, const double *psi, int nb, int ncomp,
                         const KPoint &kp, hipStream_t st);
 int launch_nonlocal_f32(qm_ctx *ctx, float *hpsi, const float *psi, int nb, int ncomp,
