@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "qm_cols.h"
 #include "qm_internal.h"
 #include "qm_mfma.h"
 
@@ -39,11 +40,6 @@ __device__ __forceinline__ T *col_ptr_out(const ColBlocks &c, int j, int64_t ng)
     return const_cast<T *>(col_ptr<T>(c, j, ng));
 }
 
-constexpr int GRAM_FLUSH = 16;  // MFMA K-steps between FP32 -> FP64 flushes
-constexpr int kGramTN = 4;      // 16-column MFMA tiles per wave along n (workgroup tile 64 x 32 kGramTN)
-
-// Wave tile 32 x 16 TN (2 x TN MFMA tiles), workgroup tile 64 x 32 TN (4 waves).
-// partial[chunk][j * m + i] = sum_{k in chunk} A[k][i] B[k][j]
 // Hardware workgroup b runs on XCD b % 8.  Workgroups are renumbered so that
 // consecutive numbers (the tiles of one K chunk) share an XCD and read the
 // chunk's rows of A and B from that XCD's L2 instead of once per XCD.
@@ -53,129 +49,8 @@ __device__ __forceinline__ int xcd_block(int nblk, int per_xcd) {
     return lb < nblk ? lb : -1;
 }
 
-template <typename T, bool VECLOAD, int TN>
-__global__ __launch_bounds__(256) void gram_partial_kernel(ColBlocks A, ColBlocks B, int m, int n, int64_t ng,
-                                                           int64_t kchunk, int tiles_n, int tiles, int nblk,
-                                                           int per_xcd, double *__restrict__ partial) {
-    using M = Mfma<T>;
-    using acc_t = typename M::acc_t;
-    using vec_t = typename M::vec_t;
-    constexpr int VEC = M::VEC;
-    constexpr int KSTEP = 4 * VEC;
-    const int lb = xcd_block(nblk, per_xcd);
-    if (lb < 0) return;
-    const int tile = lb % tiles;
-    const int ti = tile / tiles_n, tj = tile % tiles_n;
-    const int chunk = lb / tiles;
-    const int64_t k0 = (int64_t)chunk * kchunk;
-    const int64_t k1 = min(k0 + kchunk, ng);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int li = lane & 15, g = lane >> 4;
-    const int i0 = ti * 64 + (wave >> 1) * 32;
-    const int j0 = tj * (32 * TN) + (wave & 1) * (16 * TN);
-
-    const T *pa[2], *pb[TN];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int ia = i0 + 16 * s + li;
-        pa[s] = ia < m ? col_ptr<T>(A, ia, ng) : nullptr;
-    }
-#pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        const int jb = j0 + 16 * t + li;
-        pb[t] = jb < n ? col_ptr<T>(B, jb, ng) : nullptr;
-    }
-    acc_t acc[2][TN];
-    double acc64[2][TN][4];
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            acc[s][t] = acc_t{0, 0, 0, 0};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc64[s][t][r] = 0.0;
-        }
-
-    int steps = 0;
-    int64_t k = k0;
-    for (; k + KSTEP <= k1; k += KSTEP) {
-        T va[2][VEC], vb[TN][VEC];
-        if constexpr (VECLOAD) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                vec_t a = pa[s] ? *reinterpret_cast<const vec_t *>(pa[s] + k + VEC * g) : vec_t{};
-#pragma unroll
-                for (int c = 0; c < VEC; ++c) va[s][c] = a[c];
-            }
-#pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                vec_t bb = pb[t] ? *reinterpret_cast<const vec_t *>(pb[t] + k + VEC * g) : vec_t{};
-#pragma unroll
-                for (int c = 0; c < VEC; ++c) vb[t][c] = bb[c];
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < VEC; ++c) {
-#pragma unroll
-                for (int s = 0; s < 2; ++s) va[s][c] = pa[s] ? pa[s][k + VEC * g + c] : T(0);
-#pragma unroll
-                for (int t = 0; t < TN; ++t) vb[t][c] = pb[t] ? pb[t][k + VEC * g + c] : T(0);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < VEC; ++c)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int t = 0; t < TN; ++t) acc[s][t] = M::mma(va[s][c], vb[t][c], acc[s][t]);
-        if constexpr (sizeof(T) == 4) {
-            if (++steps == GRAM_FLUSH) {
-                steps = 0;
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-#pragma unroll
-                    for (int t = 0; t < TN; ++t) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc64[s][t][r] += (double)acc[s][t][r];
-                        acc[s][t] = acc_t{0, 0, 0, 0};
-                    }
-            }
-        }
-    }
-    if (k < k1) {  // tail: guarded scalar loads
-        T va[2][VEC], vb[TN][VEC];
-#pragma unroll
-        for (int c = 0; c < VEC; ++c) {
-            const int64_t kk = k + VEC * g + c;
-#pragma unroll
-            for (int s = 0; s < 2; ++s) va[s][c] = (pa[s] && kk < k1) ? pa[s][kk] : T(0);
-#pragma unroll
-            for (int t = 0; t < TN; ++t) vb[t][c] = (pb[t] && kk < k1) ? pb[t][kk] : T(0);
-        }
-#pragma unroll
-        for (int c = 0; c < VEC; ++c)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int t = 0; t < TN; ++t) acc[s][t] = M::mma(va[s][c], vb[t][c], acc[s][t]);
-    }
-    double *out = partial + (int64_t)chunk * m * n;
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            const int j = j0 + 16 * t + li;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + 16 * s + M::row(g, r);
-                if (i < m && j < n) out[(int64_t)j * m + i] = acc64[s][t][r] + (double)acc[s][t][r];
-            }
-        }
-}
-
-// Large Gram products: workgroup tile 128 x 128 of C = A^T B over a K range,
-// panels of KT rows of the 256 columns staged through LDS (double-buffered),
-// WGM x WGN waves, each (128 / WGM) x (128 / WGN) outputs in 16 x 16 MFMA
+// Gram products: workgroup tile 128 x 128 of C = A^T B over a K range, panels of
+// KT rows of the 256 columns staged through LDS (double-buffered), WGM x WGN waves, each (128 / WGM) x (128 / WGN) outputs in 16 x 16 MFMA
 // tiles.  FP32 accumulators are flushed into FP64 registers every 256 K
 // values (FP32) ; FP64 accumulates in FP64.
 constexpr int GT_M = 128, GT_N = 128;
@@ -206,15 +81,27 @@ template <typename T>
 using GramShape = GramTile<T, sizeof(T) == 4 ? 4 : 2, 4, sizeof(T) == 4 ? 32 : 16>;
 
 // partial[chunk][j * m + i] = sum_{k in chunk} A[k][i] B[k][j] for the tile's
-// 128 x 128 outputs.  Requires ng % KT == 0 and kchunk % KT == 0 (16-byte
-// aligned columns and whole panels).
-template <typename T, typename P>
-__global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColBlocks B, int m, int n, int64_t ng,
+// 128 x 128 outputs; kchunk % KT == 0, any ng, m, n and alignment: columns need no alignment (16-byte loads
+// at any element), the K values behind the last whole panel are loaded singly, and
+// waves whose outputs all lie outside C do no products.  Before, sizes off the
+// tiles ran a kernel without LDS, 64 x 128 outputs a workgroup: 600 x 400 over
+// 157,685 points FP64 4.13 -> 1.53 ms (50 TFLOP/s), FP32 4.02 -> 0.94; 300 x 200 over
+// 135,150 791 -> 428 and 1015 -> 274 us; 90 x 90 over 60,480 166 -> 70 and 100 -> 53
+// us; 24 x 24 over 167,936 210 -> 83 and 129 -> 48 us (reduction included).  Whole
+// tiles and panels: 1536 x 1024 over 262,144 points FP64 12.3 -> 11.5 ms (72 TFLOP/s),
+// over 884,736 FP32 23.7 -> 22.2 (125).  What the loop looks like matters
+// there: FP32 takes the next panel's loads and stores in a branch, and with WHOLE
+// (m, n and ng all whole) none around the products (26.9 ms unconditional, 519
+// instead of 484 us for 384 x 256 over 262,144 with the branch around the products);
+// FP64 repeats the last panel's loads instead (882 us against 820 there).
+template <typename T, typename P, bool WHOLE>
+__global__ __launch_bounds__(P::THREADS, 4) void gram_tile_kernel(ColBlocks A, ColBlocks B, int m, int n, int64_t ng,
                                                                int64_t kchunk, int tiles_n, int tiles, int nblk,
                                                                int per_xcd, double *__restrict__ partial) {
     using M = Mfma<T>;
     using acc_t = typename M::acc_t;
     using vec_t = typename M::vec_t;
+    typedef T uvec_t __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));  // load at any element
     constexpr int KT = P::KT, VEC = P::VEC, LD = P::LD, TA = P::TA, TB = P::TB, THREADS = P::THREADS;
     __shared__ __align__(16) T lds[2][GT_M + GT_N][LD];
     const int lb = xcd_block(nblk, per_xcd);
@@ -225,43 +112,43 @@ __global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColB
     const int chunk = lb / tiles;
     const int64_t k0 = (int64_t)chunk * kchunk;
     const int64_t k1 = min(k0 + kchunk, ng);
-    const int npanel = (int)((k1 - k0) / KT);
+    const int npanel = (int)((k1 - k0) / KT), rest = (int)((k1 - k0) % KT);
 
     // loader: thread t loads 16-byte pieces (VEC values) of columns; KT / VEC
-    // consecutive threads cover one column's panel rows
+    // consecutive threads cover one column's panel rows.  Columns past the end
+    // are read from the last one; their products are not stored.
     constexpr int PER_COL = KT / VEC;
-    const T *src[P::LOADS];
+    GlobalPtr<T> src[P::LOADS];
     int dcol[P::LOADS];
     const int piece = threadIdx.x % PER_COL;
+    {
+        const Cols<T> ca(A, ng), cb(B, ng);
 #pragma unroll
-    for (int q = 0; q < P::LOADS; ++q) {
-        const int c = threadIdx.x / PER_COL + q * (THREADS / PER_COL);  // 0 .. 255
-        dcol[q] = c;
-        const T *p = nullptr;
-        if (c < GT_M) {
-            const int i = ti * GT_M + c;
-            if (i < m) p = col_ptr<T>(A, i, ng);
-        } else {
-            const int j = tj * GT_N + (c - GT_M);
-            if (j < n) p = col_ptr<T>(B, j, ng);
+        for (int q = 0; q < P::LOADS; ++q) {
+            const int c = threadIdx.x / PER_COL + q * (THREADS / PER_COL);  // 0 .. 255
+            dcol[q] = c;
+            src[q] = (c < GT_M ? ca.at(min(ti * GT_M + c, m - 1)) : cb.at(min(tj * GT_N + c - GT_M, n - 1))) + k0 + piece * VEC;
         }
-        src[q] = p ? p + k0 + piece * VEC : nullptr;
     }
     vec_t stage[P::LOADS];
     auto fetch = [&](int panel) {
 #pragma unroll
-        for (int q = 0; q < P::LOADS; ++q)
-            stage[q] = src[q] ? *reinterpret_cast<const vec_t *>(src[q] + (int64_t)panel * KT) : vec_t{};
+        for (int q = 0; q < P::LOADS; ++q) {
+            const uvec_t v = *(GlobalPtr<const uvec_t>)(src[q] + (int64_t)panel * KT);
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) stage[q][e] = v[e];
+        }
     };
     auto store = [&](int buf) {
 #pragma unroll
         for (int q = 0; q < P::LOADS; ++q) *reinterpret_cast<vec_t *>(&lds[buf][dcol[q]][piece * VEC]) = stage[q];
     };
 
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, g = lane >> 4;
     const int wm = (wave / P::WN) * 16 * TA;  // wave's first output row in the tile
     const int wn = (wave % P::WN) * 16 * TB;  // wave's first output column in the tile
+    const bool any = ti * GT_M + wm < m && tj * GT_N + wn < n;  // the wave's outputs reach into C
     acc_t acc[TA][TB];
     double acc64[TA][TB][4];
 #pragma unroll
@@ -272,15 +159,7 @@ __global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColB
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc64[a][b][r] = 0.0;
         }
-
-    if (npanel > 0) {
-        fetch(0);
-        store(0);
-    }
-    __syncthreads();
-    for (int p = 0; p < npanel; ++p) {
-        const int cur = p & 1;
-        if (p + 1 < npanel) fetch(p + 1);  // next panel's loads in flight during this panel's MFMAs
+    auto products = [&](int cur) {
         // K steps of 4 VEC values: lane group g holds k = 4g .. (VEC values per lane)
 #pragma unroll
         for (int ks = 0; ks < KT; ks += 4 * VEC) {
@@ -298,6 +177,18 @@ __global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColB
 #pragma unroll
                     for (int b = 0; b < TB; ++b) acc[a][b] = M::mma(av[a][c], bv[b][c], acc[a][b]);
         }
+    };
+
+    if (npanel > 0) {
+        fetch(0);
+        store(0);
+    }
+    __syncthreads();
+    for (int p = 0; p < npanel; ++p) {
+        const int cur = p & 1;
+        const bool more = sizeof(T) == 8 || p + 1 < npanel;
+        if (more) fetch(min(p + 1, npanel - 1));  // next panel's loads in flight during this panel's MFMAs
+        if (WHOLE || any) products(cur);
         if constexpr (sizeof(T) == 4) {
             if ((p + 1) % P::FLUSH == 0) {
 #pragma unroll
@@ -310,8 +201,18 @@ __global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColB
                     }
             }
         }
-        if (p + 1 < npanel) store(cur ^ 1);  // the other buffer: last read one panel ago, before the barrier
+        if (more) store(cur ^ 1);  // the other buffer: last read one panel ago, before the barrier
         __syncthreads();
+    }
+    if (!WHOLE && rest > 0) {
+#pragma unroll
+        for (int q = 0; q < P::LOADS; ++q)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+                stage[q][e] = piece * VEC + e < rest ? src[q][(int64_t)npanel * KT + e] : T(0);
+        store(npanel & 1);
+        __syncthreads();
+        if (any) products(npanel & 1);
     }
     double *out = partial + (int64_t)chunk * m * n;
 #pragma unroll
@@ -327,13 +228,29 @@ __global__ __launch_bounds__(P::THREADS) void gram_tile_kernel(ColBlocks A, ColB
         }
 }
 
-__global__ void gram_reduce_kernel(double *__restrict__ C, const double *__restrict__ partial, int64_t mn,
-                                   int nchunk) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= mn) return;
+// Four waves of a workgroup sum a quarter of the chunks each for 64 outputs, eight
+// loads in flight: one thread per output, adding one load after the other, took
+// 62 us for 384 x 384 of 128 chunks.
+__global__ __launch_bounds__(256) void gram_reduce_kernel(double *__restrict__ C, const double *__restrict__ partial,
+                                                          int64_t mn, int nchunk) {
+    __shared__ double part[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+    const int c0 = nchunk * w / 4, c1 = nchunk * (w + 1) / 4;
+    const double *p = partial + min(e, mn - 1);
     double s = 0.0;
-    for (int c = 0; c < nchunk; ++c) s += partial[(int64_t)c * mn + e];
-    C[e] = s;
+    int c = c0;
+    for (; c + 8 <= c1; c += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(c + u) * mn];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; c < c1; ++c) s += p[(int64_t)c * mn];
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && e < mn) C[e] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
 }
 
 // Y^T (n x Ng) = C^T (n x m) Z^T (m x Ng).  Workgroup: 64 output columns x 128
@@ -413,13 +330,10 @@ constexpr int UT_N = 128, UT_P = 128, UT_THREADS = 512;
 
 template <typename T, int KTV, int PADV>
 struct UpdTile {
-    static constexpr int KT = KTV;                                   // K rows (Z columns) per panel
-    static constexpr int VEC = 16 / sizeof(T);
-    static constexpr int ZLOADS = KT * UT_P / VEC / UT_THREADS;  // 16-byte Z loads per thread per panel
-    static constexpr int CLOADS = KT * UT_N / VEC / UT_THREADS;  // 16-byte C loads per thread per panel
-    static constexpr int PAD = PADV;                             // LDS row padding (values)
-    static_assert(ZLOADS * VEC * UT_THREADS == KT * UT_P && CLOADS * VEC * UT_THREADS == KT * UT_N,
-                  "whole 16-byte loads per panel");
+    static constexpr int KT = KTV;                           // K rows (Z columns) per panel
+    static constexpr int LOADS = KT * UT_P / UT_THREADS;     // values of Z, and of C, per thread per panel
+    static constexpr int PAD = PADV;                         // LDS row padding (values)
+    static_assert(UT_N == UT_P && LOADS * UT_THREADS == KT * UT_P && KT % (16 / (int)sizeof(T)) == 0, "whole loads");
 };
 // the shape in use: 16 (FP32) / 8 (FP64) K rows per panel, rows padded by 4.
 // Shallow panels leave room for more resident workgroups (FP32: 64 VGPRs,
@@ -430,16 +344,19 @@ struct UpdTile {
 template <typename T>
 using UpdShape = UpdTile<T, sizeof(T) == 4 ? 16 : 8, 4>;
 
-// Requires ng % UT_P == 0 and m % KT == 0 (whole tiles and panels; the caller
-// checks) and 16-byte aligned column blocks.
-template <typename T, typename P>
+// Any ng, m and alignment: points and columns past the end are
+// read from the last one and not stored, K past m is cleared, and waves whose
+// columns all lie past n do no products.
+// VL: 16-byte loads of Z and C, for 16-byte aligned blocks, ng a multiple of a
+// load and m of a panel (384 x 256 over 262,144 points FP64: 905 us, 950 with
+// single loads; over 258,049 points 950 us, 1250 untiled).
+template <typename T, typename P, bool VL>
 __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, ColBlocks Y, const T *__restrict__ Cm,
                                                                  int m, int n, int64_t ng, int tiles_n, int nblk,
                                                                  int per_xcd) {
     using M = Mfma<T>;
     using acc_t = typename M::acc_t;
-    using vec_t = typename M::vec_t;
-    constexpr int KT = P::KT, VEC = P::VEC;
+    constexpr int KT = P::KT;
     __shared__ __align__(16) T zs[2][KT][UT_P + P::PAD];
     __shared__ __align__(16) T cs[2][KT][UT_N + P::PAD];
     const int lb = xcd_block(nblk, per_xcd);
@@ -448,48 +365,48 @@ __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, Co
     const int64_t gt = lb / tiles_n;
     const int c0 = tj * UT_N;
     const int64_t p0 = gt * UT_P;
-    const int npanel = m / KT;
+    const int npanel = (m + KT - 1) / KT;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const Cols<T> zcols(Z, ng);
 
-    // Z loader: UT_P / VEC consecutive threads cover one Z column's 128 points
-    constexpr int ZPER = UT_P / VEC;
-    const int zpiece = threadIdx.x % ZPER;
-    // C loader: KT / VEC consecutive threads cover KT consecutive rows of one C column
-    constexpr int CPER = KT / VEC;
-    const int cpiece = threadIdx.x % CPER;
-    vec_t zst[P::ZLOADS], cst[P::CLOADS];
+    constexpr int V = VL ? 16 / (int)sizeof(T) : 1;  // values per load
+    typedef T load_t __attribute__((ext_vector_type(V)));
+    constexpr int LOADS = P::LOADS / V;
+    // Z: UT_P / V consecutive threads take the points of one row; C: KT / V
+    // consecutive threads take KT consecutive rows of one column
+    constexpr int ZPER = UT_P / V, CPER = KT / V;
+    constexpr int ZROWS = UT_THREADS / ZPER, CCOLS = UT_THREADS / CPER;  // per load of the workgroup
+    const int zp = threadIdx.x % ZPER * V;
+    int zk = threadIdx.x / ZPER;
+    if constexpr (ZPER >= 64) zk = __builtin_amdgcn_readfirstlane(zk);  // one row per wave
+    const int64_t zoff = min(p0 + zp, ng - V);
+    const int ck = threadIdx.x % CPER * V, cc = threadIdx.x / CPER;
+    load_t zst[LOADS], cst[LOADS];
     auto fetch = [&](int panel) {
         const int k0 = panel * KT;
 #pragma unroll
-        for (int q = 0; q < P::ZLOADS; ++q) {
-            const int kk = threadIdx.x / ZPER + q * (UT_THREADS / ZPER);
-            const T *zc = col_ptr<T>(Z, k0 + kk, ng);
-            zst[q] = *reinterpret_cast<const vec_t *>(zc + p0 + zpiece * VEC);
-        }
+        for (int q = 0; q < LOADS; ++q)
+            zst[q] = *(GlobalPtr<const load_t>)(zcols.at(min(k0 + zk + ZROWS * q, m - 1)) + zoff);
 #pragma unroll
-        for (int q = 0; q < P::CLOADS; ++q) {
-            const int cc = threadIdx.x / CPER + q * (UT_THREADS / CPER);
-            cst[q] = (c0 + cc < n) ? *reinterpret_cast<const vec_t *>(Cm + (int64_t)(c0 + cc) * m + k0 + cpiece * VEC)
-                                   : vec_t{};
-        }
+        for (int q = 0; q < LOADS; ++q)
+            cst[q] = *reinterpret_cast<const load_t *>(Cm + (int64_t)min(c0 + cc + q * CCOLS, n - 1) * m +
+                                                       min(k0 + ck, m - V));
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, int panel) {
+        const int left = VL ? KT : m - panel * KT;  // K rows of the panel
 #pragma unroll
-        for (int q = 0; q < P::ZLOADS; ++q) {
-            const int kk = threadIdx.x / ZPER + q * (UT_THREADS / ZPER);
-            *reinterpret_cast<vec_t *>(&zs[buf][kk][zpiece * VEC]) = zst[q];
-        }
+        for (int q = 0; q < LOADS; ++q)
+            *reinterpret_cast<load_t *>(&zs[buf][zk + ZROWS * q][zp]) = zk + ZROWS * q < left ? zst[q] : load_t(0);
 #pragma unroll
-        for (int q = 0; q < P::CLOADS; ++q) {
-            const int cc = threadIdx.x / CPER + q * (UT_THREADS / CPER);
+        for (int q = 0; q < LOADS; ++q)
 #pragma unroll
-            for (int v = 0; v < VEC; ++v) cs[buf][cpiece * VEC + v][cc] = cst[q][v];
-        }
+            for (int v = 0; v < V; ++v) cs[buf][ck + v][cc + q * CCOLS] = ck < left ? cst[q][v] : T(0);
     };
 
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int li = lane & 15, g = lane >> 4;
     const int wc = (wave >> 2) * 64;  // wave's first output column in the tile
     const int wp = (wave & 3) * 32;   // wave's first grid point in the tile
+    const bool any = c0 + wc < n;     // the wave has columns to compute
     acc_t acc[4][2];
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -497,13 +414,13 @@ __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, Co
         for (int b = 0; b < 2; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
 
     fetch(0);
-    store(0);
+    store(0, 0);
     __syncthreads();
     for (int p = 0; p < npanel; ++p) {
         const int cur = p & 1;
-        if (p + 1 < npanel) fetch(p + 1);
+        fetch(min(p + 1, npanel - 1));
 #pragma unroll
-        for (int ks = 0; ks < KT; ks += 4) {
+        for (int ks = 0; any && ks < KT; ks += 4) {
             T av[4], bv[2];
 #pragma unroll
             for (int a = 0; a < 4; ++a) av[a] = cs[cur][ks + g][wc + 16 * a + li];  // A[col][k = g]
@@ -514,19 +431,21 @@ __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, Co
 #pragma unroll
                 for (int b = 0; b < 2; ++b) acc[a][b] = M::mma(av[a], bv[b], acc[a][b]);
         }
-        if (p + 1 < npanel) store(cur ^ 1);
+        store(cur ^ 1, min(p + 1, npanel - 1));
         __syncthreads();
     }
     // D[row = out column 16a + row(g, r)][col = grid point 16b + li]
+    const Cols<T> ycols(Y, ng);
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int col = c0 + wc + 16 * a + M::row(g, r);
             if (col >= n) continue;
-            T *yc = col_ptr_out<T>(Y, col, ng);
+            const GlobalPtr<T> yc = ycols.at(col);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) yc[p0 + wp + 16 * b + li] = acc[a][b][r];
+            for (int b = 0; b < 2; ++b)
+                if (p0 + wp + 16 * b + li < ng) yc[p0 + wp + 16 * b + li] = acc[a][b][r];
         }
 }
 
@@ -611,10 +530,6 @@ int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
 }  // namespace
 
-// Gram products with both sides >= 128 columns over whole panels take the
-// LDS-tiled 128 x 128 kernel: each panel row is read once per workgroup tile
-// and shared by its 8 waves, and the tiles of one tile row (the same A panel)
-// run consecutively on one XCD.  K is split so that about 1024 workgroups run.
 // K rows per chunk are a multiple of this (whole flush intervals for FP32)
 template <typename T>
 constexpr int gram_kround() { return sizeof(T) == 4 ? GT_FLUSH_K : 128; }
@@ -654,16 +569,21 @@ inline int64_t gram_chunks(int tiles, int64_t ng, int64_t kround, int cus, int p
     return best_nc;
 }
 
-template <typename T, typename P = GramShape<T>>
-int gram_tiled(DevBuf &partial, double *C, const ColBlocks &A, const ColBlocks &B, int m, int n, int64_t ng,
+template <typename T>
+int gram(DevBuf &partial, double *C, const ColBlocks &A, const ColBlocks &B, int m, int n, int64_t ng,
                hipStream_t st) {
+    using P = GramShape<T>;
     static_assert(gram_kround<T>() % P::KT == 0, "chunks of whole panels");
     const int tiles_m = (m + GT_M - 1) / GT_M, tiles_n = (n + GT_N - 1) / GT_N;
     const int tiles = tiles_m * tiles_n;
     int dev = 0, cus = 0, per_cu = 0;
     QM_HIP(hipGetDevice(&dev));
     QM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    QM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gram_tile_kernel<T, P>, P::THREADS, 0));
+    auto kernel = gram_tile_kernel<T, P, false>;
+    if constexpr (sizeof(T) == 4) {
+        if (m % GT_M == 0 && n % GT_N == 0 && ng % P::KT == 0) kernel = gram_tile_kernel<T, P, true>;
+    }
+    QM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, P::THREADS, 0));
     // dense MFMA peak per CU and microsecond: FP32 157.3, FP64 78.6 TFLOP/s over 256 CUs
     const double cu_flops_us = (sizeof(T) == 4 ? 157.3e6 : 78.6e6) / 256.0;
     int64_t kchunk = 0;
@@ -673,11 +593,11 @@ int gram_tiled(DevBuf &partial, double *C, const ColBlocks &A, const ColBlocks &
     const int64_t nblk = (int64_t)tiles * nchunk;
     QM_CHECK(nblk < ((int64_t)1 << 30), QM_ERR_ARG, "gram: grid too large");
     const int per_xcd = (int)((nblk + 7) / 8);
-    hipLaunchKernelGGL((gram_tile_kernel<T, P>), dim3((unsigned)(8 * per_xcd)), dim3(P::THREADS), 0, st, A, B, m, n,
-                       ng, kchunk, tiles_n, tiles, (int)nblk, per_xcd, partial.as<double>());
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * per_xcd)), dim3(P::THREADS), 0, st, A, B, m, n, ng, kchunk, tiles_n,
+                       tiles, (int)nblk, per_xcd, partial.as<double>());
     QM_HIP(hipGetLastError());
     const int64_t mn = (int64_t)m * n;
-    hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, C,
+    hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)((mn + 63) / 64)), dim3(256), 0, st, C,
                        partial.as<double>(), mn, (int)nchunk);
     QM_HIP(hipGetLastError());
     return QM_OK;
@@ -690,51 +610,17 @@ bool aligned16(const ColBlocks &c) {
     return true;
 }
 
-template <typename T>
-int gram(DevBuf &partial, double *C, const ColBlocks &A, const ColBlocks &B, int m, int n, int64_t ng,
-         hipStream_t st) {
-    const bool al = aligned16(A) && aligned16(B);
-    if (al && m >= GT_M && n >= GT_N && ng % GramShape<T>::KT == 0)
-        return gram_tiled<T>(partial, C, A, B, m, n, ng, st);
-    constexpr int KSTEP = 4 * Mfma<T>::VEC;
-    constexpr int TN = kGramTN;  // 16-column MFMA tiles per wave along n
-    const int tiles_m = (m + 63) / 64, tiles_n = (n + 32 * TN - 1) / (32 * TN);
-    const int tiles = tiles_m * tiles_n;
-    // enough workgroups to fill the 256 CUs a few times (up to 128 K chunks: the
-    // 384 x 256 LOBPCG Gram over 64^3 points has 12 tiles, and 128 chunks instead
-    // of 64 measured 969 -> 830 us FP32, 2311 -> 1800 us FP64); K chunks of >= 1024
-    int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>(128, 2048 / tiles));
-    int64_t kchunk = round_up((ng + nchunk - 1) / nchunk, (int64_t)KSTEP * GRAM_FLUSH);
-    kchunk = std::max<int64_t>(kchunk, 1024);
-    nchunk = (ng + kchunk - 1) / kchunk;
-    QM_TRY(partial.reserve(sizeof(double) * (size_t)nchunk * m * n));
-    const bool vec = al && (ng % Mfma<T>::VEC) == 0;
-    const int64_t nblk = (int64_t)tiles * nchunk;
-    QM_CHECK(nblk < ((int64_t)1 << 30), QM_ERR_ARG, "gram: grid too large");
-    const int per_xcd = (int)((nblk + 7) / 8);
-    const dim3 grid((unsigned)(8 * per_xcd));
-    if (vec)
-        hipLaunchKernelGGL((gram_partial_kernel<T, true, TN>), grid, dim3(256), 0, st, A, B, m, n, ng, kchunk, tiles_n,
-                           tiles, (int)nblk, per_xcd, partial.as<double>());
-    else
-        hipLaunchKernelGGL((gram_partial_kernel<T, false, TN>), grid, dim3(256), 0, st, A, B, m, n, ng, kchunk, tiles_n,
-                           tiles, (int)nblk, per_xcd, partial.as<double>());
-    QM_HIP(hipGetLastError());
-    const int64_t mn = (int64_t)m * n;
-    hipLaunchKernelGGL(gram_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, C,
-                       partial.as<double>(), mn, (int)nchunk);
-    QM_HIP(hipGetLastError());
-    return QM_OK;
-}
-
 template <typename T, typename P = UpdShape<T>>
 int update_tiled(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int n, int64_t ng, hipStream_t st) {
     const int tiles_n = (n + UT_N - 1) / UT_N;
-    const int64_t nblk = (ng / UT_P) * tiles_n;
+    const int64_t nblk = (ng + UT_P - 1) / UT_P * tiles_n;
     QM_CHECK(nblk < ((int64_t)1 << 30), QM_ERR_ARG, "update: grid too large");
     const int per_xcd = (int)((nblk + 7) / 8);
-    hipLaunchKernelGGL((update_tile_kernel<T, P>), dim3((unsigned)(8 * per_xcd)), dim3(UT_THREADS), 0, st, Z, Y, Cm, m,
-                       n, ng, tiles_n, (int)nblk, per_xcd);
+    const bool vl = ng % (16 / sizeof(T)) == 0 && m % P::KT == 0 && aligned16(Z) &&
+                    reinterpret_cast<uintptr_t>(Cm) % 16 == 0;
+    const auto kernel = vl ? update_tile_kernel<T, P, true> : update_tile_kernel<T, P, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * per_xcd)), dim3(UT_THREADS), 0, st, Z, Y, Cm, m, n, ng, tiles_n,
+                       (int)nblk, per_xcd);
     QM_HIP(hipGetLastError());
     return QM_OK;
 }
@@ -747,8 +633,9 @@ int update(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int n, in
         // 60,480, 237: 83 and 119 us)
         if (n >= 128 && split_update_fits(Z, m, n, ng)) return split_update(Z, Y, Cm, m, n, ng, st);
     }
-    if (n >= UT_N && ng % UT_P == 0 && m % UpdShape<T>::KT == 0 && aligned16(Z) && aligned16(Y) &&
-        reinterpret_cast<uintptr_t>(Cm) % 16 == 0)
+    // up to 64 columns the untiled kernel's 64-column workgroups do less padding
+    // (24 over 96^3 points FP64: 164 us, 185 tiled; 90 over 60,480: 88 and 73 us)
+    if (n > 64)
         return update_tiled<T>(Z, Y, Cm, m, n, ng, st);
     const int tiles_n = (n + 63) / 64;
     const int64_t gtiles = (ng + 127) / 128;

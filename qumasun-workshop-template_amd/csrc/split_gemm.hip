@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "qm_cols.h"
 #include "qm_internal.h"
 
 namespace qm {
@@ -69,35 +70,6 @@ __device__ __forceinline__ Split split8(const float (&x)[8], float &top) {
 __device__ __forceinline__ bool out_of_split(float top) {
     return top >= 3.3895e38f || (top > 0.0f && top < 7.8886e-31f);
 }
-
-// Column j of a chain of blocks, without branches: the first column of each block
-// is found once per workgroup
-struct Cols {
-    const float *p[kMaxColBlocks];
-    int first[kMaxColBlocks];
-    __device__ __forceinline__ Cols(const ColBlocks &c) {
-        int f = 0;
-#pragma unroll
-        for (int b = 0; b < kMaxColBlocks; ++b) {
-            p[b] = static_cast<const float *>(c.ptr[b]);
-            first[b] = b < c.nblk ? f : INT32_MAX;
-            f += c.ncols[b];
-        }
-    }
-    __device__ __forceinline__ const float *at(int j, int64_t ng, int *last = nullptr) const {
-        const float *q = p[0];
-        int f = 0, l = first[1];
-#pragma unroll
-        for (int b = 1; b < kMaxColBlocks; ++b) {
-            const bool in = j >= first[b];
-            q = in ? p[b] : q;
-            f = in ? first[b] : f;
-            l = in ? (b + 1 < kMaxColBlocks ? first[b + 1] : INT32_MAX) : l;
-        }
-        if (last) *last = l;  // the block ends before this column
-        return q + (int64_t)(j - f) * ng;
-    }
-};
 
 __device__ __forceinline__ int xcd_block(int nblk, int per_xcd) {
     const int b = blockIdx.x;
@@ -169,7 +141,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     const int ci = (threadIdx.x >> 1) & (UN - 1), ch = threadIdx.x & 1;
     // points and columns past the end are computed on the last one and not stored
     const int64_t zp = min(p0 + zi, ng - 1);
-    const Cols zcols(Z), ycols(Y);
+    const Cols<float> zcols(Z, ng);
     const uint32_t coff = ((uint32_t)min(c0 + ci, n - 1) * m + 8 * ch) * 4u;
     // C through a buffer resource: the last panel may read past a column's end,
     // and past the array's end it gets zeros
@@ -180,9 +152,9 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     // at its end, and wait there.  K past m is read from column m - 1 (cleared in store).
     auto fetch = [&](int p) {
         const int kz = p * SG_K + 8 * zh;
-        int end;
-        const float *zc = zcols.at(min(kz, m - 1), ng, &end);
-        const float *znext = zcols.at(min(end, m - 1), ng);
+        const int end = zcols.end(min(kz, m - 1));
+        GlobalPtr<float> zc = zcols.at(min(kz, m - 1));
+        const GlobalPtr<float> znext = zcols.at(min(end, m - 1));
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             zv[e] = zc[zp];
@@ -244,6 +216,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
         __syncthreads();
     }
     const int i = lane & 31, kh = lane >> 5;
+    const Cols<float> ycols(Y, ng);
     if (__syncthreads_or(out_of_split(top_z) || out_of_split(top_c))) {
         for (int a = 0; a < TA; ++a)
             for (int b = 0; b < TB; ++b) {
@@ -253,13 +226,13 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
                 for (int k = 0; k < m; k += 2) {
                     const int kk = k + kh;
                     const float av = (col < n && kk < m) ? Cm[(int64_t)col * m + kk] : 0.0f;
-                    const float bv = (pt < ng && kk < m) ? zcols.at(kk, ng)[pt] : 0.0f;
+                    const float bv = (pt < ng && kk < m) ? zcols.at(kk)[pt] : 0.0f;
                     s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
                 }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int cr = c0 + wc + 32 * a + sg_row(r, lane);
-                    if (cr < n && pt < ng) const_cast<float *>(ycols.at(cr, ng))[pt] = s[r];
+                    if (cr < n && pt < ng) ycols.at(cr)[pt] = s[r];
                 }
             }
         return;
@@ -270,7 +243,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
         for (int r = 0; r < 16; ++r) {
             const int col = c0 + wc + 32 * a + sg_row(r, lane);
             if (col >= n) continue;
-            float *yc = const_cast<float *>(ycols.at(col, ng)) + p0;
+            const GlobalPtr<float> yc = ycols.at(col) + p0;
 #pragma unroll
             for (int b = 0; b < TB; ++b)
                 if (p0 + wp + 32 * b + i < ng) yc[wp + 32 * b + i] = acc[a][b][r];
