@@ -328,8 +328,8 @@ __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
         if (cg + q < ncol) hpsi[(int64_t)(cg + q) * ng + g] = hv[q];
 }
 
-// The same sums on the matrix cores, for FP64 and for more than 16 projectors,
-// where nl_scatter_kernel is bound by its broadcast LDS reads of the
+// The same sums on the matrix cores, for many projectors and small launches, where
+// nl_scatter_kernel is bound by its broadcast LDS reads of the
 // coefficients (one per point, column and projector).  A wave owns 16 PT
 // covered points x 16 CT columns and takes the atoms of its tile one after the
 // other: columns are the rows of the result (A: coefficients), points its
@@ -341,12 +341,12 @@ __global__ __launch_bounds__(kScatterBlock) void nl_scatter_kernel(
 // an atom's results are added only at the points its sphere covers.  The sums
 // then change lanes through LDS, so that Hpsi is read and written with lanes
 // along the points (without it 64^3 x 64 complex took 110 us instead of 95).
-// Hpsi's lines bound it: 64^3 x 64 complex FP64, 16 atoms, 0.41 GB of 128 B
-// lines, 103 -> 95 us (4.3 TB/s); 45x54x50 x 37 complex FP64, 32 projectors,
-// 45 -> 29 us (FP32 34 -> 22; 64^3 x 128 FP32 116 -> 82); 32^3 x 24 FP64 6.5 ->
-// 5.2 us.  FP32 with up to 16 projectors
-// stays with nl_scatter_kernel (64^3 x 128: 53 us there, 61 here; 160^3 x 512:
-// 3.19 and 3.41 ms): half the LDS bytes a coefficient, and 32 columns a thread.
+// 45x54x50 x 37 complex FP64, 32 projectors, 45 -> 29 us (FP32 34 -> 22; 64^3 x 128
+// FP32 116 -> 82); 32^3 x 24 FP64 6.5 -> 5.2 us.  Large launches with up to 9
+// projectors are bound by Hpsi's lines (64^3 x 128 FP64: 0.41 GB of them in 97 us,
+// 4.2 TB/s; 106 us here) and stay with nl_scatter_kernel, as does FP32 up to 16
+// (half the LDS bytes a coefficient, and 32 columns a thread: 64^3 x 128 53 us
+// there, 61 here; 160^3 x 512 3.19 and 3.41 ms).
 template <typename T, int NC, bool PH, int KS, int CT, int PT>
 __global__ __launch_bounds__(256) void nl_scatter_mfma_kernel(
     T *__restrict__ hpsi, const T *__restrict__ coef, int64_t ng, int ncol, int ntile,
@@ -818,45 +818,55 @@ int launch_scatter_mfma(qm_ctx *ctx, T *hpsi, const T *coef, int ncol, const T *
     return QM_OK;
 }
 
+// Waves of the MFMA scatter with 32 points x 32 columns each
+inline int64_t scatter_waves(const Projectors &p, int ncol) { return (int64_t)p.ntile * 2 * ((ncol + 31) / 32); }
+
 // 32 points x 32 columns a wave; 16 x 16 where that leaves less than 2 waves a
 // SIMD (32^3 x 24 FP64: 576 waves 6.9 us, 2272 waves 5.2 us; 36x40x42 x 45
 // complex: 3100 waves 21 us, 12400 waves 24 us)
-constexpr int64_t kScatterWaves = 2048;
 template <typename T, int NC, bool PH, int KS>
 int scatter_mfma(qm_ctx *ctx, T *hpsi, const T *coef, int ncol, const T *phase, hipStream_t st) {
-    const int64_t waves = (int64_t)ctx->proj.ntile * 2 * ((ncol + 31) / 32);
-    if (waves >= kScatterWaves) return launch_scatter_mfma<T, NC, PH, KS, 2, 2>(ctx, hpsi, coef, ncol, phase, st);
+    if (scatter_waves(ctx->proj, ncol) >= 2048)
+        return launch_scatter_mfma<T, NC, PH, KS, 2, 2>(ctx, hpsi, coef, ncol, phase, st);
     return launch_scatter_mfma<T, NC, PH, KS, 1, 1>(ctx, hpsi, coef, ncol, phase, st);
+}
+
+// columns per scatter tile (16; 64 per thread measured 1.9x slower on 64^3 x
+// 128) and tiles per workgroup (the staged coefficients, entry lists and table
+// rows serve all of them)
+template <typename T, int NC, bool PH, int MP>
+int scatter_points(qm_ctx *ctx, T *hpsi, const T *coef, int ncol, const T *phase, hipStream_t st) {
+    const Projectors &p = ctx->proj;
+    constexpr int NBS = 16, SGT = sizeof(T) == 8 ? 1 : 2;
+    const int sgroups = (ncol + NBS * SGT - 1) / (NBS * SGT);
+    const int64_t nblk = (int64_t)p.nsblock * sgroups;
+    QM_CHECK(nblk < (int64_t)INT32_MAX / 16, QM_ERR_ARG, "nonlocal apply: too many bands per call");
+    const int per_xcd = (int)((nblk + 7) / 8);
+    hipLaunchKernelGGL((nl_scatter_kernel<T, NC, PH, NBS, SGT, MP>), dim3(8 * per_xcd), dim3(kScatterBlock), 0, st,
+                       hpsi, coef, ctx->ng, ncol, p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox, p.d_cov_slot,
+                       p.d_block_atom_off, p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off, tabp_of<T>(p), phase,
+                       sgroups, (int)nblk, per_xcd);
+    QM_HIP(hipGetLastError());
+    return QM_OK;
 }
 
 template <typename T, int NC, bool PH>
 int nonlocal_scatter(qm_ctx *ctx, T *hpsi, const T *coef, int nb, const T *phase, hipStream_t st) {
-    const Projectors &p = ctx->proj;
-    const int ncol = nb * NC;
-    if (p.max_m > 16) return scatter_mfma<T, NC, PH, 8>(ctx, hpsi, coef, ncol, phase, st);
+    const int ncol = nb * NC, m = ctx->proj.max_m;
+    if (m > 16) return scatter_mfma<T, NC, PH, 8>(ctx, hpsi, coef, ncol, phase, st);
     if constexpr (sizeof(T) == 8) {
-        if (p.max_m > 12) return scatter_mfma<T, NC, PH, 4>(ctx, hpsi, coef, ncol, phase, st);
-        return scatter_mfma<T, NC, PH, 3>(ctx, hpsi, coef, ncol, phase, st);
+        if (m > 12) return scatter_mfma<T, NC, PH, 4>(ctx, hpsi, coef, ncol, phase, st);
+        // up to 9 projectors the thread-per-point kernel wins on large launches
+        // (36x40x42 x 45 complex, 3100 waves: 22.9 us there, 20.4 here; 64^3 x 32
+        // complex, 8512: 50 and 54; 64^3 x 128 real, 17024: 97 and 106), not with 16
+        // (64^3 x 64 complex: 109 and 101)
+        if (m > 9 || scatter_waves(ctx->proj, ncol) < 4096)
+            return scatter_mfma<T, NC, PH, 3>(ctx, hpsi, coef, ncol, phase, st);
+        return scatter_points<T, NC, PH, 9>(ctx, hpsi, coef, ncol, phase, st);
     } else {
-        // columns per scatter tile (16; 64 per thread measured 1.9x slower on
-        // 64^3 x 128) and tiles per workgroup (the staged coefficients, entry lists
-        // and table rows serve all of them)
-        constexpr int NBS = 16, SGT = 2;
-        const int sgroups = (ncol + NBS * SGT - 1) / (NBS * SGT);
-        const int64_t nblk = (int64_t)p.nsblock * sgroups;
-        QM_CHECK(nblk < (int64_t)INT32_MAX / 16, QM_ERR_ARG, "nonlocal apply: too many bands per call");
-        const int per_xcd = (int)((nblk + 7) / 8);
-        auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(8 * per_xcd), dim3(kScatterBlock), 0, st, hpsi, coef, ctx->ng, ncol,
-                               p.ncov, p.d_cov_grid, p.d_cov_off, p.d_cov_vox, p.d_cov_slot, p.d_block_atom_off,
-                               p.d_block_atoms, p.d_vox_atom, p.d_nproj, p.d_proj_off, tabp_of<T>(p), phase, sgroups,
-                               (int)nblk, per_xcd);
-        };
-        if (p.max_m <= 9) launch(nl_scatter_kernel<T, NC, PH, NBS, SGT, 9>);
-        else launch(nl_scatter_kernel<T, NC, PH, NBS, SGT, 16>);
+        if (m > 9) return scatter_points<T, NC, PH, 16>(ctx, hpsi, coef, ncol, phase, st);
+        return scatter_points<T, NC, PH, 9>(ctx, hpsi, coef, ncol, phase, st);
     }
-    QM_HIP(hipGetLastError());
-    return QM_OK;
 }
 
 // which: 1 = projection coefficients, 2 = scatter, 3 = both.  coef / part are
