@@ -296,12 +296,12 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
             QM_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
             return scatter();
         };
-        // mean time of `reps` applies after a warm-up
+        // mean time of `reps` applies after a warm-up (none for reps = 1)
         hipEvent_t ev[2] = {nullptr, nullptr};
         int status = QM_OK;
         auto timed = [&](auto &&run, int reps) -> float {
             float ms = 0.0f;
-            status = run();
+            status = reps > 1 ? run() : QM_OK;
             if (status == QM_OK && hipEventRecord(ev[0], st) != hipSuccess) status = QM_ERR_HIP;
             for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
             if (status == QM_OK && hipEventRecord(ev[1], st) != hipSuccess) status = QM_ERR_HIP;
@@ -329,9 +329,14 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 if (capturing || g_internal_capture) return overlapped();
                 QM_TRY(in_order());  // the projection's shape is tuned alone first
                 QM_TRY(events.create());
-                const float ms = timed(in_order, 3);
+                // one apply each: the two schedules differ by up to a tenth, single
+                // applies by 1 %, and the first apply of a shape pays for all of them
+                const float ms = timed(in_order, 1);
                 bool beside = false;
-                if (status == QM_OK && ms > kOverlapMinMs) beside = timed(overlapped, 3) < ms;
+                if (status == QM_OK && ms > kOverlapMinMs) {
+                    QM_TRY(side_stream(ctx));
+                    beside = timed(overlapped, 1) < ms;
+                }
                 if (status == QM_ERR_HIP) set_error("H.psi schedule tuning: HIP event failure");
                 if (status != QM_OK) return status;
                 it = ctx->apply_overlapped.emplace(key, beside).first;
