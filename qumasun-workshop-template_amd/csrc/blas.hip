@@ -335,20 +335,19 @@ struct UpdTile {
     static constexpr int PAD = PADV;                         // LDS row padding (values)
     static_assert(UT_N == UT_P && LOADS * UT_THREADS == KT * UT_P && KT % (16 / (int)sizeof(T)) == 0, "whole loads");
 };
-// the shape in use: 16 (FP32) / 8 (FP64) K rows per panel, rows padded by 4.
-// Shallow panels leave room for more resident workgroups (FP32: 64 VGPRs,
-// 34 KB of LDS): the 1536 -> 1024 column update over 884,736 points ran
-// 21.4 ms against 23.2 with 32 K rows (FP64 44.6 against 45.1 with 16), the
-// 384 -> 256 one over 262,144 points 0.49 against 0.57 ms (FP64 0.93 against
-// 1.02); 64 K rows and wider padding were slower.  Same bits for every depth.
+// the shape in use: 16 K rows per panel, rows padded by 4 (FP32: 64 VGPRs, 34 KB of
+// LDS).  FP32, 1536 -> 1024 columns over 884,736 points: 21.4 ms against 23.2 with 32
+// K rows, 384 -> 256 over 262,144 0.49 against 0.57; FP64, over 262,144 points: 12.92
+// and 0.870 ms against 13.12 and 0.884 with 8 K rows (13.31 and 0.892 with rows
+// padded by 16).  Same bits for every depth.
 template <typename T>
-using UpdShape = UpdTile<T, sizeof(T) == 4 ? 16 : 8, 4>;
+using UpdShape = UpdTile<T, 16, 4>;
 
 // Any ng, m and alignment: points and columns past the end are
 // read from the last one and not stored, K past m is cleared, and waves whose
 // columns all lie past n do no products.
-// VL: 16-byte loads of Z and C, for 16-byte aligned blocks, ng a multiple of a
-// load and m of a panel (384 x 256 over 262,144 points FP64: 905 us, 950 with
+// VL: 16-byte loads of Z and C, for 16-byte aligned blocks and ng and m that are
+// multiples of a load (384 x 256 over 262,144 points FP64: 905 us, 950 with
 // single loads; over 258,049 points 950 us, 1250 untiled).
 template <typename T, typename P, bool VL>
 __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, ColBlocks Y, const T *__restrict__ Cm,
@@ -393,7 +392,7 @@ __global__ __launch_bounds__(UT_THREADS) void update_tile_kernel(ColBlocks Z, Co
                                                        min(k0 + ck, m - V));
     };
     auto store = [&](int buf, int panel) {
-        const int left = VL ? KT : m - panel * KT;  // K rows of the panel
+        const int left = m - panel * KT;  // K rows of the panel
 #pragma unroll
         for (int q = 0; q < LOADS; ++q)
             *reinterpret_cast<load_t *>(&zs[buf][zk + ZROWS * q][zp]) = zk + ZROWS * q < left ? zst[q] : load_t(0);
@@ -616,7 +615,7 @@ int update_tiled(const ColBlocks &Z, const ColBlocks &Y, const T *Cm, int m, int
     const int64_t nblk = (ng + UT_P - 1) / UT_P * tiles_n;
     QM_CHECK(nblk < ((int64_t)1 << 30), QM_ERR_ARG, "update: grid too large");
     const int per_xcd = (int)((nblk + 7) / 8);
-    const bool vl = ng % (16 / sizeof(T)) == 0 && m % P::KT == 0 && aligned16(Z) &&
+    const bool vl = ng % (16 / sizeof(T)) == 0 && m % (16 / sizeof(T)) == 0 && aligned16(Z) &&
                     reinterpret_cast<uintptr_t>(Cm) % 16 == 0;
     const auto kernel = vl ? update_tile_kernel<T, P, true> : update_tile_kernel<T, P, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * per_xcd)), dim3(UT_THREADS), 0, st, Z, Y, Cm, m, n, ng, tiles_n,
