@@ -595,6 +595,7 @@ void qm_destroy(qm_ctx *ctx) {
     ctx->td_work.release();
     ctx->scf_part.release();
     if (ctx->h_dot) (void)hipHostFree(ctx->h_dot);
+    if (ctx->h_force) (void)hipHostFree(ctx->h_force);
     fft_destroy(ctx);
     if (ctx->blas) rocblas_destroy_handle((rocblas_handle)ctx->blas);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);

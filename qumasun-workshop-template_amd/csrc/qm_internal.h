@@ -146,6 +146,8 @@ struct qm_ctx {
     qm::DevBuf td_work;                     // two band blocks of the Taylor propagator
     qm::DevBuf scf_part;                    // partial sums of qm_grid_dot_f64
     double *h_dot = nullptr;                // its result: pinned host memory the device writes
+    double *h_force = nullptr;              // force sums: pinned host memory the device writes
+    size_t h_force_n = 0;                   // its size in values
     // second stream of a full H.psi apply: the nonlocal projection runs on it
     // beside the stencil, joined by events (created on first use)
     hipStream_t side = nullptr;
