@@ -226,7 +226,7 @@ int qm_nonlocal_choice(qm_ctx *ctx, int precision, int ncomp, int kt, int nb, in
 
 /* d_rho[i] += sum_n occ[n] |psi_n(i)|^2 (FP64 accumulation).  dE_band/dV_loc(i) is
  * d_rho[i]*dV.  Replaces SetDensityOne (qumasun_SetDensityOne.h:9-41).  occ: host,
- * nb values, read before the call returns.  Asynchronous on `stream`. */
+ * nb values.  Synchronises `stream`: d_rho is complete when the call returns. */
 int qm_band_density_f64(qm_ctx *ctx, double *d_rho, const double *d_psi, const double *occ, int nb,
                         int ncomp, void *stream);
 int qm_band_density_f32(qm_ctx *ctx, double *d_rho, const float *d_psi, const double *occ, int nb,

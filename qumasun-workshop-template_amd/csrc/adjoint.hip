@@ -12,9 +12,8 @@
 namespace qm {
 namespace {
 
-// Occupations of one launch, by value (no staging buffer, no upload, so the
-// call needs no synchronisation): bands beyond kDensityBands take further
-// launches.
+// Occupations of one launch, by value (no staging buffer, no upload): bands
+// beyond kDensityBands take further launches.
 constexpr int kDensityBands = 256;
 struct DensityOcc {
     double occ[kDensityBands];

@@ -435,8 +435,11 @@ int band_density_impl(qm_ctx *ctx, double *rho, const T *psi, const double *occ,
     if (nb == 0) return QM_OK;
     QM_TRY(activate(ctx));
     hipStream_t st = (hipStream_t)stream;
-    if constexpr (sizeof(T) == 8) return launch_band_density_f64(ctx, rho, psi, occ, nb, ncomp, st);
-    else return launch_band_density_f32(ctx, rho, psi, occ, nb, ncomp, st);
+    if constexpr (sizeof(T) == 8) QM_TRY(launch_band_density_f64(ctx, rho, psi, occ, nb, ncomp, st));
+    else QM_TRY(launch_band_density_f32(ctx, rho, psi, occ, nb, ncomp, st));
+    // callers read rho on other streams, or with a blocking copy, once this returns
+    QM_HIP(hipStreamSynchronize(st));
+    return QM_OK;
 }
 
 template <typename T>

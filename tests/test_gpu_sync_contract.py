@@ -1,0 +1,43 @@
+"""Calls that return finished work: qm_band_density_* synchronises the stream it
+is given.
+
+It is called on a non-blocking stream behind products of about a tenth of a
+second; when it returns, the stream has nothing left to do."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _idle_after(torch, call):
+    """Whether `call`, made behind long work on a stream of its own, leaves that stream idle."""
+    a = torch.rand((8192, 8192), device="cuda")
+    b = torch.empty_like(a)
+    torch.mm(a, a, out=b)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            torch.mm(a, a, out=b)
+        assert not stream.query()
+        call()
+        idle = stream.query()
+    torch.cuda.synchronize()
+    return idle
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_band_density_synchronises(qm, orc, torch_cuda, prec):
+    torch = torch_cuda
+    s = qm.system.small_system(n=11, L=4.0, natoms=1, nbands=5)
+    print(f"case density behind long work {prec}", flush=True)
+    H = qm.hamiltonian.Hamiltonian(s)
+    rng = np.random.default_rng(4)
+    psi = rng.uniform(-0.5, 0.5, (5, s.ng)).astype(np.float32).astype(np.float64)
+    x = torch.from_numpy(psi).to("cuda", torch.float64 if prec == "f64" else torch.float32)
+    rho = torch.zeros(s.ng, dtype=torch.float64, device="cuda")
+    occ = np.linspace(2.0, 0.5, 5)
+    assert _idle_after(torch, lambda: H.band_density(x, occ, rho=rho))
+    want = orc.band_density(s, psi, occ)
+    assert np.abs(rho.cpu().numpy() - want).max() <= 1e-13 * np.abs(want).max()
+    H.close()
