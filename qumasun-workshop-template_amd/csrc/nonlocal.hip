@@ -954,7 +954,10 @@ int nonlocal_forces(qm_ctx *ctx, const T *psi, const double *occ, int nb, int nc
     QM_CHECK(ncomp == 2 || !ph, QM_ERR_ARG, "real (ncomp=1) bands need a Gamma k-point");
     *e_nl = 0.0;
     for (int i = 0; i < 3 * p.natoms; ++i) forces[i] = 0.0;
-    if (p.nchunk == 0 || p.max_m == 0) return QM_OK;  // no voxels or no projectors: nothing to sum
+    if (p.nchunk == 0 || p.max_m == 0) {  // no voxels or no projectors: nothing to sum
+        QM_HIP(hipStreamSynchronize(st));
+        return QM_OK;
+    }
     // MFMA row tiles of the 4 max_m projections (1, 3, 4 or 8 are built: up to
     // 4, 12, 16 and 32 projectors per atom)
     const int need = (4 * p.max_m + 15) / 16;

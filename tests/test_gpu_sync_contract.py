@@ -1,8 +1,11 @@
-"""Calls that return finished work: qm_band_density_* synchronises the stream it
-is given.
+"""Calls that return finished work: qm_band_density_* and qm_nonlocal_forces_*
+synchronise the stream they are given.
 
-It is called on a non-blocking stream behind products of about a tenth of a
-second; when it returns, the stream has nothing left to do."""
+Each is called on a non-blocking stream behind products of about a tenth of a
+second; when it returns, the stream has nothing left to do.  The forces also for
+atoms without projectors, where there is nothing to sum."""
+import types
+
 import numpy as np
 import pytest
 
@@ -40,4 +43,22 @@ def test_band_density_synchronises(qm, orc, torch_cuda, prec):
     assert _idle_after(torch, lambda: H.band_density(x, occ, rho=rho))
     want = orc.band_density(s, psi, occ)
     assert np.abs(rho.cpu().numpy() - want).max() <= 1e-13 * np.abs(want).max()
+    H.close()
+
+@pytest.mark.parametrize("projectors", [True, False])
+def test_forces_synchronise(qm, torch_cuda, projectors):
+    torch = torch_cuda
+    s = qm.system.small_system(n=11, L=4.0, natoms=1, nbands=5)
+    print(f"case forces behind long work, projectors {projectors}", flush=True)
+    H = qm.hamiltonian.Hamiltonian(s)
+    if not projectors:
+        none = np.zeros(0)
+        H.set_projectors(types.SimpleNamespace(
+            natoms=1, nproj=[0], vox_off=[0, 4], vox_xyz=np.zeros((4, 3), np.int32), table=none,
+            dtable=none, tab_off=[0, 0], energy=none, proj_off=[0, 0]))
+    x = torch.rand((5, s.ng), dtype=torch.float64, device="cuda")
+    out = []
+    assert _idle_after(torch, lambda: out.append(H.nonlocal_forces(x, np.ones(5))))
+    e, f = out[0]
+    assert (np.abs(f).max() > 0.0 and e != 0.0) if projectors else (e == 0.0 and not f.any())
     H.close()
