@@ -481,6 +481,12 @@ __global__ __launch_bounds__(256) void nl_scatter_mfma_kernel(
 // group g takes the 16 consecutive voxels 16 g .. 16 g + 15 of a 64-voxel
 // sub-chunk: a lane's A operands of 16 K steps are then contiguous, and the
 // K order of the sum is free as long as A and B agree on it.
+//
+// FP32 bands are summed on the FP64 matrix cores too: a wave's 128 voxels in one
+// FP32 chain lost up to ten times what the earlier form's FP64 sum over threads
+// did (bands of one sign, 4 atoms, forces: 3.6e-6 of the largest one, 5.4e-7 so).
+// The gather hides the slower products: 64 real bands, 8 atoms 47.8 -> 49.7 us,
+// 96^3, 64 complex bands, 40 atoms with 32 projectors 424 -> 443 us a call.
 
 // Column slice of one launch and the occupations of its bands, by value: no
 // staging buffer, no upload.
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(256) void nl_grad_project_kernel(
     const int *__restrict__ vox_grid, const T *__restrict__ table, const T *__restrict__ dtable,
     const T *__restrict__ phase, const int *__restrict__ item_order, int groups, int nblk, int per_xcd) {
     constexpr int AS = MT == 1 ? 16 : (MT <= 4 ? 8 : 4);  // K steps whose A operands are held at once
-    using M = Mfma<T>;
+    using M = Mfma<double>;
     using acc_t = typename M::acc_t;
     __shared__ T stage[4][PJ_SUB][16 + 1];
     __shared__ double red[4][16 * 16];
@@ -592,9 +598,9 @@ __global__ __launch_bounds__(256) void nl_grad_project_kernel(
             }
 #pragma unroll
             for (int s = 0; s < AS; ++s) {
-                const T b = stage[wave][16 * g + h + s][j];
+                const double b = (double)stage[wave][16 * g + h + s][j];
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[mt] = M::mma(av[mt][s], b, acc[mt]);
+                for (int mt = 0; mt < MT; ++mt) acc[mt] = M::mma((double)av[mt][s], b, acc[mt]);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -603,7 +609,7 @@ __global__ __launch_bounds__(256) void nl_grad_project_kernel(
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave][M::row(g, r) * 16 + j] = (double)acc[mt][r];
+        for (int r = 0; r < 4; ++r) red[wave][M::row(g, r) * 16 + j] = acc[mt][r];
         __syncthreads();
         const int e = threadIdx.x;  // 256 = 16 rows x 16 columns
         const int r = 16 * mt + (e >> 4), col = c0 + (e & 15);
