@@ -228,6 +228,14 @@ int execute(FftState &f, FftPlan &p, void *in[], void *out[], hipStream_t st) {
     return QM_OK;
 }
 
+// Whether the context's spectrum buffer may be reserved at this size.  A graph
+// that holds an apply of the context may hold the buffer, so that it is not
+// replaced then; it may be made: an apply on the plane and line kernels
+// (spectral.hip) has none.
+bool may_reserve(const qm_ctx *ctx, size_t bytes) {
+    return ctx->capture_pins == 0 || !ctx->fft || !ctx->fft->spec.p || ctx->fft->spec.bytes >= bytes;
+}
+
 // spec = FFT(psi) (nb bands, ncomp 1 or 2); returns the spectrum and its size per band
 template <typename T>
 int forward(qm_ctx *ctx, const T *psi, int nb, int ncomp, FftPair **pair, C2<T> **spec, int64_t *per_band,
@@ -235,7 +243,7 @@ int forward(qm_ctx *ctx, const T *psi, int nb, int ncomp, FftPair **pair, C2<T> 
     QM_TRY(get_pair<T>(ctx, nb, ncomp, pair));
     FftState &f = *ctx->fft;
     const int64_t pb = ncomp == 2 ? ctx->ng : (int64_t)(ctx->nx / 2 + 1) * ctx->ny * ctx->nz;
-    QM_CHECK(ctx->capture_pins == 0 || f.spec.bytes >= sizeof(C2<T>) * (size_t)pb * nb, QM_ERR_STATE,
+    QM_CHECK(may_reserve(ctx, sizeof(C2<T>) * (size_t)pb * nb), QM_ERR_STATE,
              "FFT kinetic: larger spectrum buffer needed while a graph holds an apply of this context; destroy it "
              "and call qm_release_captures first");
     QM_TRY(f.spec.reserve(sizeof(C2<T>) * (size_t)pb * nb));
@@ -364,7 +372,7 @@ int fft_poisson(qm_ctx *ctx, const double *rho, double *vh, hipStream_t st) {
     SpectralTables *t = nullptr;
     QM_TRY(own_tables<double>(ctx, st, &t));
     const size_t need = sizeof(C2<double>) * (size_t)ctx->ng;
-    if (t && (ctx->capture_pins == 0 || (ctx->fft && ctx->fft->spec.bytes >= need))) {
+    if (t && may_reserve(ctx, need)) {
         if (!ctx->fft) ctx->fft = new FftState();
         QM_TRY(ctx->fft->spec.reserve(need));
         return spectral_poisson(ctx, t, ctx->fft->spec.p, vh, rho, st);
