@@ -70,6 +70,7 @@ __global__ __launch_bounds__(256) void dc_init_kernel(DcWork w, const double *__
     m = red[0];
     int ex = 0;
     if (!bad && m > 0.0) (void)frexp(m, &ex);
+    ex = min(ex, 1023);  // 2^ex is multiplied back in; entries from 2^1023 on become at most 2
     for (int i = threadIdx.x; i < n; i += 256) {
         double a = bad ? 0.0 : ldexp(d[i], -ex);
         const double b = bad || i + 1 >= n ? 0.0 : ldexp(e[i], -ex);

@@ -1,11 +1,9 @@
-"""qm_sygvd_f64 at the ends of FP64's range, and with the factor written over B.
+"""qm_sygvd_f64 at the ends of FP64's range.
 
 Matrices with entries of 1e150 and 1e-150 (orders on both sides of the leaf size
 and of a tile), and eigenvalues above 2^1023: a power of two is taken off the
 tridiagonal matrix before it is solved, and put back.  Tolerances as for the
 ordinary sizes: (64 + 8 n) eps of the norm."""
-import ctypes
-
 import numpy as np
 import pytest
 
@@ -20,7 +18,7 @@ def _sygvd(qm, torch, H, a, b, nev):
 
 
 @pytest.mark.parametrize("scale", [1e150, 1e-150])
-@pytest.mark.parametrize("n", [2, 15, 17, 63, 130])
+@pytest.mark.parametrize("n", [15, 17, 63, 130])
 def test_sygvd_scaled(qm, torch_cuda, n, scale):
     torch = torch_cuda
     print(f"case sygvd n {n} scale {scale:g}", flush=True)
