@@ -557,6 +557,12 @@ int own_eig_max_n() { return kMaxN; }
 namespace qm {
 namespace {
 
+// Whether two arrays of this size share memory (a factor written over its matrix)
+bool overlap(const void *a, const void *b, size_t bytes) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + bytes && y < x + bytes;
+}
+
 // C = A with the upper triangle mirrored into the lower one
 __global__ void symmetrize_upper_kernel(double *__restrict__ C, const double *__restrict__ A, int n) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -613,7 +619,12 @@ int qm_sygvd_f64(qm_ctx *ctx, int n, const double *d_A, const double *d_B, doubl
     QM_HIP(hipGetLastError());
     const bool own = subspace_route() < 0 && chol_inverse_supported(n);
     if (own) {
-        QM_TRY(chol_inverse(n, false, d_B, T, d_U, Ui, info, st));
+        const void *B = d_B;
+        if (overlap(d_B, d_U, sizeof(double) * nn)) {  // workgroups read B while others write U
+            QM_HIP(hipMemcpyAsync(Z, d_B, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
+            B = Z;
+        }
+        QM_TRY(chol_inverse(n, false, B, T, d_U, Ui, info, st));
     } else {
         QM_HIP(hipMemcpyAsync(d_U, d_B, sizeof(double) * nn, hipMemcpyDeviceToDevice, st));
         QM_TRY(potrf_upper(h, n, d_U, n, info, st));
@@ -667,7 +678,13 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
     QM_HIP(hipMemcpyAsync(C, d_A, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
     const bool own = subspace_route() < 0 && chol_inverse_supported(n);
     if (own) {
-        QM_TRY(chol_inverse(n, true, d_B, Z, U, Ui, info, st));
+        const void *B = d_B;
+        if (overlap(d_B, d_U, sizeof(zc) * nn)) {  // (as in qm_sygvd_f64; the tridiagonal solver's work is free)
+            static_assert(sizeof(zc) == 2 * sizeof(double), "2 n^2 doubles of work hold B");
+            QM_HIP(hipMemcpyAsync(dcw, d_B, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
+            B = dcw;
+        }
+        QM_TRY(chol_inverse(n, true, B, Z, U, Ui, info, st));
     } else {
         QM_HIP(hipMemcpyAsync(U, d_B, sizeof(zc) * nn, hipMemcpyDeviceToDevice, st));
         QM_EIG_BLAS(rocsolver_zpotrf(h, rocblas_fill_upper, n, U, n, info));
