@@ -392,6 +392,15 @@ int qm_subspace_force(int route);
 int qm_coop_set_spin_limit(long polls);
 long qm_coop_spin_limit_default(void);
 
+/* Bound of the steps of a root and of a leaf in the tridiagonal divide and
+ * conquer, process-wide; no reference counterpart (a diagnostic and test
+ * control).  A solve in which one runs out is done again by rocSOLVER's stedc,
+ * and steqr where that does not converge either (counted by
+ * qm_lobpcg_eigen_retries).  By default the bound is above what any matrix can
+ * take; 0 makes every such solve run out, which the tests use to exercise
+ * that path.  INT_MAX restores the default.  QM_ERR_ARG for steps < 0. */
+int qm_dc_set_step_limit(int steps);
+
 /* HIP graphs for the iteration segments that hold no host decision (no
  * reference counterpart: the reference launches every kernel from the host).
  * Within one qm_lobpcg_solve call, A.R and the Gram products of an iteration

@@ -450,6 +450,25 @@ int sytrd_lower(void *blas, int n, double *C, int lda, double *trd, double *VW, 
     return QM_OK;
 }
 
+// Eigenpairs of the tridiagonal matrix in trd (d, e, then 2 n more doubles of
+// which the last n are work) by rocSOLVER: w ascending, Z n x n (ldz >= n)
+static int stedc_steqr(rocblas_handle h, int n, double *w, double *Z, int ldz, double *trd, int *info,
+                       hipStream_t st) {
+    double *e_copy = trd + 3 * n;  // stedc overwrites e
+    QM_HIP(hipMemcpyAsync(e_copy, trd + n, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+    QM_HIP(hipMemcpyAsync(w, trd, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+    QM_EIG_BLAS(rocsolver_dstedc(h, rocblas_evect_tridiagonal, n, w, trd + n, Z, ldz, info));
+    int h_info = 0;
+    QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
+    QM_HIP(hipStreamSynchronize(st));
+    if (h_info == 0) return QM_OK;
+    // divide and conquer did not converge (it can on nearly degenerate
+    // spectra): implicit QL/QR on the same tridiagonal instead
+    QM_HIP(hipMemcpyAsync(w, trd, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+    QM_EIG_BLAS(rocsolver_dsteqr(h, rocblas_evect_tridiagonal, n, w, e_copy, Z, ldz, info));
+    return QM_OK;
+}
+
 // Eigenvalues (all, ascending, into w) and the eigenvectors of the nev lowest
 // into Z[:, :nev] (ldz >= n) of the symmetric matrix whose upper triangle C
 // holds (C overwritten).
@@ -458,7 +477,8 @@ int sytrd_lower(void *blas, int n, double *C, int lda, double *trd, double *VW, 
 // order) and the own back-transformation; else n <= kMaxN: the single-workgroup panel
 // reduction below, stedc + ormtr (Z must hold n x n in both); larger n:
 // rocSOLVER syevd.  info receives rocSOLVER's status (or the cooperative
-// reduction's barrier error, -77).  trd holds 4 n doubles (d, e, tau, and a
+// reduction's barrier error, -77, or kDcUnconverged: dcw = nullptr takes
+// rocSOLVER's solver from the start).  trd holds 4 n doubles (d, e, tau, and a
 // copy of e for the steqr retry after a stedc failure).
 int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double *Z, int ldz, double *trd,
                double *VW, void *dcw, int *info, hipStream_t st) {
@@ -467,25 +487,13 @@ int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double
         trd_coop_work_bytes(n, false) <= sizeof(double) * (size_t)kTrdPanelCols * n) {
         const int r = trd_coop_f64(n, C, lda, trd, trd + n, trd + 2 * n, VW,
                                    sizeof(double) * (size_t)kTrdPanelCols * n, st);
-        if (r == QM_OK && tridiag_dc_supported(n)) {
+        if (r == QM_OK && dcw && tridiag_dc_supported(n)) {
             QM_TRY(tridiag_dc(n, nev, trd, trd + n, w, Z, ldz, false, dcw, info, st));
             QM_TRY(trd_coop_check(VW, info, st));
             return ormtr_lower_f64(n, nev, C, lda, trd + 2 * n, Z, ldz, VW, st);
         }
         if (r == QM_OK) {
-            double *e_copy = trd + 3 * n;  // stedc overwrites e
-            QM_HIP(hipMemcpyAsync(e_copy, trd + n, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-            QM_HIP(hipMemcpyAsync(w, trd, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-            QM_EIG_BLAS(rocsolver_dstedc(h, rocblas_evect_tridiagonal, n, w, trd + n, Z, ldz, info));
-            int h_info = 0;
-            QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
-            QM_HIP(hipStreamSynchronize(st));
-            if (h_info != 0) {
-                // divide and conquer did not converge (it can on nearly degenerate
-                // spectra): implicit QL/QR on the same tridiagonal instead
-                QM_HIP(hipMemcpyAsync(w, trd, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-                QM_EIG_BLAS(rocsolver_dsteqr(h, rocblas_evect_tridiagonal, n, w, e_copy, Z, ldz, info));
-            }
+            QM_TRY(stedc_steqr(h, n, w, Z, ldz, trd, info, st));
             QM_TRY(trd_coop_check(VW, info, st));
             QM_TRY(ormtr_lower_f64(n, nev, C, lda, trd + 2 * n, Z, ldz, VW, st));
             return QM_OK;
@@ -556,6 +564,10 @@ int own_eig_max_n() { return kMaxN; }
 
 namespace qm {
 namespace {
+
+const char *const kInfoMeaning =
+    ": 1 on the own route for a matrix that is not finite, -77 where the cooperative reduction's grid barrier timed "
+    "out, else rocSOLVER's)";
 
 // Whether two arrays of this size share memory (a factor written over its matrix)
 bool overlap(const void *a, const void *b, size_t bytes) {
@@ -639,9 +651,15 @@ int qm_sygvd_f64(qm_ctx *ctx, int n, const double *d_A, const double *d_B, doubl
     QM_TRY(chol_back(h, n, nev, Ui, Z, n, d_Z, n));
     QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
     QM_HIP(hipStreamSynchronize(st));
+    if (h_info == kDcUnconverged) {  // rocSOLVER on the same (d, e); C still holds the reflectors
+        QM_TRY(stedc_steqr(h, n, d_w, Z, n, trd, info, st));
+        QM_TRY(ormtr_lower_f64(n, nev, C, n, trd + 2 * n, Z, n, VW, st));
+        QM_TRY(chol_back(h, n, nev, Ui, Z, n, d_Z, n));
+        QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
+        QM_HIP(hipStreamSynchronize(st));
+    }
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
-             "qm_sygvd_f64: tridiagonal eigensolve failed (info " + std::to_string(h_info) +
-                 ": rocSOLVER stedc, or -77 where the cooperative reduction's grid barrier timed out)");
+             "qm_sygvd_f64: tridiagonal eigensolve failed (info " + std::to_string(h_info) + kInfoMeaning);
     return QM_OK;
 }
 
@@ -713,20 +731,37 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
     int r = QM_ERR_STATE;
     if (subspace_route() != 0 && trd_coop_supported(n, true))
         r = trd_coop_z64(n, C, n, d, e, tau, coop, coopb, st);
-    if (r == QM_OK && tridiag_dc_supported(n)) {
-        QM_TRY(tridiag_dc(n, nev, d, e, d_w, reinterpret_cast<double *>(Z), n, true, dcw, info, st));
-        QM_TRY(trd_coop_check(coop, info, st));
-        QM_TRY(unmtr_lower_z64(n, nev, C, n, tau, Z, n, coop, st));
-    } else if (r == QM_OK) {
+    auto library_tridiag = [&]() -> int {
         QM_HIP(hipMemcpyAsync(e_copy, e, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
         QM_HIP(hipMemcpyAsync(d_w, d, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
         QM_EIG_BLAS(rocsolver_zstedc(h, rocblas_evect_tridiagonal, n, d_w, e, Z, n, info));
         QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
         QM_HIP(hipStreamSynchronize(st));
-        if (h_info != 0) {  // divide and conquer did not converge: QL/QR instead
-            QM_HIP(hipMemcpyAsync(d_w, d, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-            QM_EIG_BLAS(rocsolver_zsteqr(h, rocblas_evect_tridiagonal, n, d_w, e_copy, Z, n, info));
+        if (h_info == 0) return QM_OK;
+        // divide and conquer did not converge: QL/QR instead
+        QM_HIP(hipMemcpyAsync(d_w, d, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+        QM_EIG_BLAS(rocsolver_zsteqr(h, rocblas_evect_tridiagonal, n, d_w, e_copy, Z, n, info));
+        return QM_OK;
+    };
+    // z = U^-1 y for the nev lowest, and the status
+    auto back = [&]() -> int {
+        if (own) {
+            QM_EIG_BLAS(rocblas_zgemm(h, rocblas_operation_none, rocblas_operation_none, n, nev, n, &one, Ui, n, Z, n,
+                                      &zero, static_cast<zc *>(d_Z), n));
+        } else {
+            QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_none,
+                                      rocblas_diagonal_non_unit, n, nev, &one, U, n, Z, n));
+            QM_HIP(hipMemcpyAsync(d_Z, Z, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
         }
+        QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
+        QM_HIP(hipStreamSynchronize(st));
+        return QM_OK;
+    };
+    if (r == QM_OK) {
+        if (tridiag_dc_supported(n))
+            QM_TRY(tridiag_dc(n, nev, d, e, d_w, reinterpret_cast<double *>(Z), n, true, dcw, info, st));
+        else
+            QM_TRY(library_tridiag());
         QM_TRY(trd_coop_check(coop, info, st));
         QM_TRY(unmtr_lower_z64(n, nev, C, n, tau, Z, n, coop, st));
     } else {
@@ -734,19 +769,14 @@ int qm_hegvd_z64(qm_ctx *ctx, int n, const void *d_A, const void *d_B, double *d
         QM_EIG_BLAS(rocsolver_zheevd(h, rocblas_evect_original, rocblas_fill_upper, n, C, n, d_w, e, info));
         QM_HIP(hipMemcpyAsync(Z, C, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
     }
-    // z = U^-1 y for the nev lowest
-    if (own) {
-        QM_EIG_BLAS(rocblas_zgemm(h, rocblas_operation_none, rocblas_operation_none, n, nev, n, &one, Ui, n, Z, n,
-                                  &zero, static_cast<zc *>(d_Z), n));
-    } else {
-        QM_EIG_BLAS(rocblas_ztrsm(h, rocblas_side_left, rocblas_fill_upper, rocblas_operation_none,
-                                  rocblas_diagonal_non_unit, n, nev, &one, U, n, Z, n));
-        QM_HIP(hipMemcpyAsync(d_Z, Z, sizeof(zc) * n * nev, hipMemcpyDeviceToDevice, st));
+    QM_TRY(back());
+    if (h_info == kDcUnconverged) {  // rocSOLVER on the same (d, e); C still holds the reflectors
+        QM_TRY(library_tridiag());
+        QM_TRY(unmtr_lower_z64(n, nev, C, n, tau, Z, n, coop, st));
+        QM_TRY(back());
     }
-    QM_HIP(hipMemcpyAsync(&h_info, info, sizeof(int), hipMemcpyDeviceToHost, st));
-    QM_HIP(hipStreamSynchronize(st));
     QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
-             "qm_hegvd_z64: tridiagonal eigensolve failed (rocSOLVER info " + std::to_string(h_info) + ")");
+             "qm_hegvd_z64: tridiagonal eigensolve failed (info " + std::to_string(h_info) + kInfoMeaning);
     return QM_OK;
 }
 

@@ -659,8 +659,9 @@ int chol_factor(qm_lobpcg *s, int n3, hipStream_t st) {
     return QM_OK;
 }
 
+// own_td: by the own divide and conquer where it fits, else by rocSOLVER's solvers
 template <bool CPLX>
-int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
+int chol_solve(qm_lobpcg *s, int n3, bool own_td, hipStream_t st) {
     const int N = s->na;
     if constexpr (CPLX) {
         const rocblas_double_complex one{1.0, 0.0};
@@ -690,7 +691,7 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
             const int r = trd_coop_z64(n3, C, n3, d, e, tau, s->VW, sizeof(double) * (size_t)kTrdPanelCols * n3, st);
             if (r == QM_OK) {
                 double *e_copy = s->trd + 4 * n3;  // stedc overwrites e
-                const bool dc = tridiag_dc_supported(n3);
+                const bool dc = own_td && tridiag_dc_supported(n3);
                 std::vector<double> hde(dc ? 0 : 2 * (size_t)n3);
                 if (dc) {
                     QM_TRY(tridiag_dc(n3, N, d, e, s->evals, reinterpret_cast<double *>(Z), n3, true, s->dcw, s->info,
@@ -727,7 +728,7 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
                     s->evec_t1 = false;
                     return QM_OK;
                 }
-                if (h_info != 0 && !dc) {  // an unconverged root of the own solver is left to the caller's check
+                if (h_info != 0 && !dc) {  // (the own solver's status is the caller's to act on)
                     // divide and conquer did not converge (it can on nearly degenerate
                     // spectra): implicit QL/QR on the same tridiagonal instead
                     ++s->stedc_retries;
@@ -763,7 +764,8 @@ int chol_solve(qm_lobpcg *s, int n3, hipStream_t st) {
             // and conquer and back-transformation (eigenvectors in T1), then c = U^-1 y into Hw
             auto *Ui = (double *)s->Ev, *Z = (double *)s->T1;
             QM_TRY(chol_transform(s->blas, n3, U, C, Ui, own_chol(n3), Z, st));
-            QM_TRY(syev_lower(s->blas, n3, N, C, n3, s->evals, Z, n3, s->trd, s->VW, s->dcw, s->info, st));
+            QM_TRY(syev_lower(s->blas, n3, N, C, n3, s->evals, Z, n3, s->trd, s->VW, own_td ? s->dcw : nullptr,
+                              s->info, st));
             QM_TRY(chol_back(s->blas, n3, N, Ui, Z, n3, C, n3));
             s->evec_t1 = false;
             return QM_OK;
@@ -1300,6 +1302,7 @@ int solve_impl(qm_lobpcg *s, T *x_user, double *eigenvalues, double *residual_no
         QM_HIP(hipGetLastError());
         hipLaunchKernelGGL(penalty_kernel, dim3(1), dim3(256), 0, st, s->pen, (const double *)s->svw, N);
         QM_HIP(hipGetLastError());
+        bool own_td = true;
         for (int attempt = 0;; ++attempt) {
             const int n3a = nbk_used * N;
             hipLaunchKernelGGL((assemble_kernel<CPLX>), dim3(nblk((int64_t)n3a * n3a)), dim3(256), 0, st,
@@ -1311,7 +1314,7 @@ int solve_impl(qm_lobpcg *s, T *x_user, double *eigenvalues, double *residual_no
             double h_ratio = 0.0;
             QM_TRY(read_status(s, s->svals, &h_info, &h_ratio, st));
             if (h_info == 0 && h_ratio >= cond_limit) {
-                QM_TRY(chol_solve<CPLX>(s, n3a, st));
+                QM_TRY(chol_solve<CPLX>(s, n3a, own_td, st));
                 // a tridiagonal eigensolve that does not converge (a barely
                 // definite S makes U^-H H U^-1 badly scaled), or Ritz vectors
                 // that have lost their S-orthonormality (S too ill-conditioned
@@ -1342,6 +1345,15 @@ int solve_impl(qm_lobpcg *s, T *x_user, double *eigenvalues, double *residual_no
                     evec = cv;
                     break;
                 }
+                if (h_info == kDcUnconverged && own_td) {
+                    // the own divide and conquer ran out of steps: the same problem
+                    // once more with rocSOLVER's stedc and steqr
+                    ++s->stedc_retries;
+                    s->eig_note += " (divide and conquer of order " + std::to_string(n3a) +
+                                   " out of steps, redone by rocSOLVER)";
+                    own_td = false;
+                    continue;
+                }
                 if (h_info == 0) {
                     ++s->ortho_rejects;
                     s->eig_note += " (Cholesky-route Ritz vectors of order " + std::to_string(n3a) +
@@ -1359,7 +1371,7 @@ int solve_impl(qm_lobpcg *s, T *x_user, double *eigenvalues, double *residual_no
             QM_TRY(svqb_eig<CPLX>(s, n3a, sizeof(T) == 8 ? 1.0e-12 : cond_limit, st));
             QM_TRY(read_status(s, nullptr, &h_info, nullptr, st));
             QM_CHECK(h_info == 0, QM_ERR_NUMERIC,
-                     "qm_lobpcg_solve: subspace eigensolve failed (rocSOLVER info " + std::to_string(h_info) +
+                     "qm_lobpcg_solve: subspace eigensolve failed (heevd / syevd and Jacobi, info " + std::to_string(h_info) +
                          "; " + s->eig_note + ")");
             evec = s->Ev;
             ++s->fallbacks;

@@ -198,8 +198,11 @@ int syev_lower(void *blas, int n, int nev, double *C, int lda, double *w, double
 // tridiag_dc.hip: all eigenvalues (ascending, w) and the nev lowest eigenvectors
 // (Z[:, :nev], ldz >= n; interleaved complex with zero imaginary parts when
 // cplx) of the symmetric tridiagonal (d, e), which is left as it is.  *info
-// (device): 0, 1 for a non-finite matrix, 2 where a root did not converge.
+// (device): 0, 1 for a non-finite matrix, kDcUnconverged where a leaf or a root ran
+// out of steps (qm_dc_set_step_limit: by default more than any can take): the
+// caller then takes rocSOLVER's stedc and steqr on the same (d, e).
 // work: tridiag_dc_work_bytes; n up to tridiag_dc_max.
+constexpr int kDcUnconverged = -78;
 int tridiag_dc_max();
 int tridiag_dc_supported(int n);
 size_t tridiag_dc_work_bytes(int n);

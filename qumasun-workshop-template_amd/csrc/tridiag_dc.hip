@@ -18,19 +18,20 @@
 // vector and reads its status back: n = 384 with 128 vectors 1780 -> 275 us,
 // n = 135 with 45 820 -> 190 us (kernel time).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <cstdint>
 
 #include "qm_internal.h"
 #include "qm_mfma.h"
 #include "qm_wave.h"
+#include "secular.h"
 
 namespace qm {
 namespace {
 
 constexpr int kLeaf = 16;
 constexpr int kMaxOrder = 1024;         // LDS of the prep and root kernels
-constexpr double kEps = 0x1p-53;        // unit roundoff
-constexpr int kMaxIter = 100;           // secular iterations; bisection alone needs fewer
 
 // Device arrays of one solve (n values each), in the work buffer after the two
 // n x n eigenvector buffers.
@@ -111,7 +112,7 @@ __device__ __forceinline__ void put(double *q, int64_t ld, int r, int64_t c, dou
 // rotations; cyclic Jacobi on the same leaves (12 rows) took 149 us, this 79.
 template <bool CPLX>
 __global__ __launch_bounds__(64) void dc_leaf_kernel(DcWork w, double *__restrict__ q, int ld, int n, int L, int nev,
-                                                     double *wout, int *info) {
+                                                     double *wout, int max_steps, int *info) {
     __shared__ double V[kLeaf][kLeaf + 1], a[kLeaf + 2], b[kLeaf + 2];
     const int s0 = node_start(n, L, blockIdx.x), m = node_start(n, L, blockIdx.x + 1) - s0;
     const int lane = threadIdx.x, row = lane & (kLeaf - 1);
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(DcWork w, double *__restric
     for (int i = lane; i < kLeaf * kLeaf; i += 64) V[i / kLeaf][i % kLeaf] = i / kLeaf == i % kLeaf ? 1.0 : 0.0;
     __syncthreads();
     int hi = m - 1, steps = 0;
-    while (hi > 0 && steps < 40 * kLeaf) {
+    while (hi > 0 && steps < max_steps) {
         // the unreduced block [lo, hi]: negligible couplings are zeroed
         int lo = hi;
         while (lo > 0 && fabs(b[lo - 1]) > kEps * (fabs(a[lo - 1]) + fabs(a[lo]))) --lo;
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(DcWork w, double *__restric
         if (rank < nev)
             for (int r = 0; r < m; ++r) put<CPLX>(q, ld, s0 + r, s0 + rank, V[r][lane]);
     }
-    if (lane == 0 && hi > 0) *info = 2;
+    if (lane == 0 && hi > 0) *info = kDcUnconverged;
 }
 
 // exclusive prefix sum of one flag per element over nn <= kMaxOrder elements,
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(256) void dc_prep_kernel(DcWork w, const double *__
 // y < yroot, 4 roots a block); the blocks after them apply the node's deflating
 // rotations to its old eigenvectors, a thread per row.
 __global__ __launch_bounds__(256) void dc_root_kernel(DcWork w, double *__restrict__ q, int n, int l, int yroot,
-                                                      int *info) {
+                                                      int max_steps, int *info) {
     __shared__ double d[kMaxOrder], z2[kMaxOrder];
     const int node = blockIdx.x, s0 = node_start(n, l, node), s1 = node_start(n, l, node + 1), tid = threadIdx.x;
     if ((int)blockIdx.y >= yroot) {
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(256) void dc_root_kernel(DcWork w, double *__restri
     const int k = w.k[node];
     if ((int)blockIdx.y * 4 >= k) return;
     const int mid = node_start(n, l + 1, 2 * node + 1);
-    const double rho = 2.0 * fabs(w.e[mid - 1]), rinv = 1.0 / rho;
+    const double rho = 2.0 * fabs(w.e[mid - 1]);
     for (int i = tid; i < k; i += 256) {
         const double z = w.zl[s0 + i];
         d[i] = w.dl[s0 + i];
@@ -363,94 +364,14 @@ __global__ __launch_bounds__(256) void dc_root_kernel(DcWork w, double *__restri
     __syncthreads();
     const int j = blockIdx.y * 4 + (tid >> 6), lane = tid & 63;
     if (j >= k) return;  // no barrier below
-    const bool end = j == k - 1;
-    double lo, hi, tau;
-    int org = j;
-    if (!end) {
-        const double del = d[j + 1] - d[j], h = 0.5 * del;
-        double c0 = 0.0;
-        for (int i = lane; i < k; i += 64)
-            if (i != j && i != j + 1) c0 += z2[i] / ((d[i] - d[j]) - h);
-        c0 = rinv + wave_sum(c0);
-        const double f = c0 + (z2[j + 1] - z2[j]) / h;
-        if (f > 0.0) {
-            lo = 0.0;
-            hi = h;
-            const double a = c0 * del + z2[j] + z2[j + 1], b = z2[j] * del, s = sqrt(fabs(a * a - 4.0 * b * c0));
-            tau = a > 0.0 ? 2.0 * b / (a + s) : (a - s) / (2.0 * c0);
-        } else {
-            org = j + 1;
-            lo = -h;
-            hi = 0.0;
-            const double a = c0 * del - z2[j] - z2[j + 1], b = z2[j + 1] * del, s = sqrt(fabs(a * a + 4.0 * b * c0));
-            tau = a < 0.0 ? 2.0 * b / (a - s) : -(a + s) / (2.0 * c0);
-        }
-    } else {
-        double s = 0.0;
-        for (int i = lane; i < k; i += 64) s += z2[i];
-        lo = 0.0;
-        hi = rho * wave_sum(s) * (1.0 + 8.0 * kEps);
-        double c0 = 0.0;
-        for (int i = lane; i < k - 1; i += 64) c0 += z2[i] / ((d[i] - d[j]) - hi);
-        c0 = rinv + wave_sum(c0);
-        tau = c0 > 0.0 ? z2[j] / c0 : hi;
-    }
-    if (!(tau > lo && tau < hi)) tau = 0.5 * (lo + hi);
-    const double d0 = d[org];
-    const double dj = d[j] - d0, dj1 = end ? 0.0 : d[j + 1] - d0;
-    bool ok = false;
-    for (int it = 0; it < kMaxIter; ++it) {
-        double psi = 0.0, dpsi = 0.0, phi = 0.0, dphi = 0.0;
-        for (int i = lane; i < k; i += 64) {
-            const double g = 1.0 / ((d[i] - d0) - tau), t = z2[i] * g;
-            if (i <= j) {
-                psi += t;
-                dpsi += t * g;
-            } else {
-                phi += t;
-                dphi += t * g;
-            }
-        }
-        psi = wave_sum(psi);
-        dpsi = wave_sum(dpsi);
-        phi = wave_sum(phi);
-        dphi = wave_sum(dphi);
-        const double f = rinv + psi + phi, df = dpsi + dphi;
-        if (fabs(f) <= kEps * (8.0 * (phi - psi) + rinv + fabs(tau) * df)) {
-            ok = true;
-            break;
-        }
-        if (f > 0.0) hi = fmin(hi, tau);
-        else lo = fmax(lo, tau);
-        double eta;
-        const double a1 = dj - tau, a2 = dj1 - tau;
-        if (!end) {
-            const double c = f - a1 * dpsi - a2 * dphi, a = (a1 + a2) * f - a1 * a2 * df, b = a1 * a2 * f;
-            const double s = sqrt(fabs(a * a - 4.0 * b * c));
-            if (c == 0.0) eta = b / a;
-            else eta = a <= 0.0 ? (a - s) / (2.0 * c) : 2.0 * b / (a + s);
-        } else {
-            const double c = f - a1 * dpsi;  // one pole, at d_k
-            eta = a1 + a1 * a1 * dpsi / c;
-        }
-        if (!(f * eta < 0.0)) eta = -f / df;
-        double x = tau + eta;
-        if (!(x > lo && x < hi) || it % 4 == 3) {
-            // bisection; towards a pole at 0 in powers of 8, as the root may be any size
-            const double y = lo == 0.0 ? hi * 0.125 : (hi == 0.0 ? lo * 0.125 : 0.5 * (lo + hi));
-            if (!(x > lo && x < hi) || it > 16) x = y;
-        }
-        if (x == tau || hi - lo <= 2.0 * kEps * fmax(fabs(lo), fabs(hi))) {
-            ok = true;
-            break;
-        }
-        tau = x;
-    }
+    int org;
+    double tau;
+    const bool ok = secular_root(j, k, d, z2, rho, lane, 64, [](double v) { return wave_sum(v); }, max_steps, &org, &tau);
     if (lane == 0) {
         w.tau[s0 + j] = tau;
         w.org[s0 + j] = org;
-        w.lam[s0 + j] = d0 + tau;
-        if (!ok) *info = 2;
+        w.lam[s0 + j] = d[org] + tau;
+        if (!ok) *info = kDcUnconverged;
     }
 }
 
@@ -559,6 +480,9 @@ int depth_of(int n) {
     return L;
 }
 
+// qm_dc_set_step_limit, process-wide
+std::atomic<int> g_dc_step_limit{INT32_MAX};
+
 }  // namespace
 
 int tridiag_dc_max() { return kMaxOrder; }
@@ -586,12 +510,14 @@ static int solve(int n, int nev, const double *d, const double *e, double *w, do
         *a = ip;
         ip += m;
     }
+    // steps of a secular root, and of a leaf's QR iteration (~2 a row)
+    const int root_steps = std::min(g_dc_step_limit.load(), kMaxSteps);
+    const int leaf_steps = std::min(g_dc_step_limit.load(), 40 * kLeaf);
     const int L = depth_of(n);
     hipLaunchKernelGGL(dc_init_kernel, dim3(1), dim3(256), 0, st, k, d, e, n, L, info);
     QM_HIP(hipGetLastError());
     if (L == 0) {
-        hipLaunchKernelGGL(dc_leaf_kernel<CPLX>, dim3(1), dim3(64), 0, st, k, Z, ldz, n, 0, nev, w,
-                           info);
+        hipLaunchKernelGGL(dc_leaf_kernel<CPLX>, dim3(1), dim3(64), 0, st, k, Z, ldz, n, 0, nev, w, leaf_steps, info);
         QM_HIP(hipGetLastError());
         return QM_OK;
     }
@@ -600,7 +526,7 @@ static int solve(int n, int nev, const double *d, const double *e, double *w, do
                        dim3(256), 0, st, buf[0], 2 * (int64_t)n * n);
     QM_HIP(hipGetLastError());
     hipLaunchKernelGGL(dc_leaf_kernel<false>, dim3(1 << L), dim3(64), 0, st, k, buf[0], n, n, L, n, (double *)nullptr,
-                       info);
+                       leaf_steps, info);
     QM_HIP(hipGetLastError());
     int cur = 0;
     for (int l = L - 1; l >= 0; --l) {
@@ -609,7 +535,8 @@ static int solve(int n, int nev, const double *d, const double *e, double *w, do
         double *q = buf[cur];
         hipLaunchKernelGGL(dc_prep_kernel, dim3(nodes), dim3(256), 0, st, k, q, n, l);
         QM_HIP(hipGetLastError());
-        hipLaunchKernelGGL(dc_root_kernel, dim3(nodes, y4 + y256), dim3(256), 0, st, k, q, n, l, y4, info);
+        hipLaunchKernelGGL(dc_root_kernel, dim3(nodes, y4 + y256), dim3(256), 0, st, k, q, n, l, y4, root_steps,
+                           info);
         QM_HIP(hipGetLastError());
         hipLaunchKernelGGL(dc_zhat_kernel, dim3(nodes, y4 + y256), dim3(256), 0, st, k, n, l, y4,
                            l == 0 ? w : nullptr);
@@ -636,3 +563,9 @@ int tridiag_dc(int n, int nev, const double *d, const double *e, double *w, doub
 }
 
 }  // namespace qm
+
+extern "C" int qm_dc_set_step_limit(int steps) {
+    QM_CHECK(steps >= 0, QM_ERR_ARG, "qm_dc_set_step_limit: steps must be >= 0");
+    qm::g_dc_step_limit.store(steps);
+    return QM_OK;
+}

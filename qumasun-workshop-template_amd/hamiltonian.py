@@ -39,6 +39,12 @@ def coop_spin_limit(polls=None):
     _lib.check(L.qm_coop_set_spin_limit(int(L.qm_coop_spin_limit_default() if polls is None else polls)))
 
 
+def dc_step_limit(steps=None):
+    """Bound of the steps of a root and a leaf in the tridiagonal divide and
+    conquer, process-wide (qm_dc_set_step_limit); None restores the default."""
+    _lib.check(_lib.load().qm_dc_set_step_limit(2 ** 31 - 1 if steps is None else int(steps)))
+
+
 class Hamiltonian:
     def __init__(self, system, device=0):
         self.lib = _lib.load()
