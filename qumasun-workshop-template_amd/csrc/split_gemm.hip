@@ -7,10 +7,17 @@
 // (m l, l m, l l: below 2^-26 of the product together, where an FP32 product
 // rounds at 2^-24) are left out; the other six are accumulated in FP32.
 //
+// The bf16 MFMA rounds its sums downward, where the FP32 one rounds to nearest: left
+// alone the mean error of all outputs is -0.10 of their rms error at m = 1024, -0.18
+// at 3072.  The panels of the second and third quarter of K are therefore summed with
+// the other sign (C's values and the accumulators turn there and back), which takes
+// out a constant as well as a linearly growing drift: at most 0.01 on inputs of
+// mixed or one sign, 0.04 where the terms grow along K.  It costs 2 %.
+//
 // Measured (before: the FP32 MFMA kernels of blas.hip): 1536 x 1024 over 884,736
-// points 21.4 -> 14.1 ms (130 -> 197 TFLOP/s), 384 x 256 over 262,144 points 507 -> 410
-// us, 600 x 400 over 157,685 points (no multiple of their tiles) 1153 -> 631 us.  Error
-// against 64 bits 3.5e-7 .. 7.0e-7 -> 2.9e-7 .. 6.0e-7.  The matrix core is busy for half
+// points 21.5 -> 14.3 ms (130 -> 195 TFLOP/s), 384 x 256 over 262,144 points 440 -> 329
+// us, 600 x 400 over 157,685 points (no multiple of their tiles) 1128 -> 550 us.  Error
+// against 64 bits 2.2e-7 .. 9.9e-7 -> 1.8e-7 .. 8.4e-7 (m = 256 .. 3072).  The matrix core is busy for half
 // of the time (at 2.1 GHz); the splits and the barrier of each panel take the rest.
 // Reading each operand a group of products earlier changed nothing; 128 columns
 // a workgroup throughout, two workgroups a CU, cost 11 %.
@@ -135,6 +142,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     const int c0 = (lb % tiles_n) * UN;  // column tile fastest: neighbours share Z in one XCD's L2
     const int64_t p0 = (int64_t)(lb / tiles_n) * SU_P;
     const int npanel = (m + SG_K - 1) / SG_K;
+    const int turn = npanel / 4;  // panels from turn to 3 turn are summed with the other sign (see the file comment)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int zi = threadIdx.x & (SU_P - 1), zh = wave >> 2;
     const bool cload = threadIdx.x < 2 * UN;  // whole waves
@@ -172,6 +180,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
         }
     };
     auto store = [&](int buf, int p) {
+        const uint32_t sign = p >= turn && p < 3 * turn ? 0x80000000u : 0u;
         if ((p + 1) * SG_K > m) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -184,6 +193,8 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
         zs[buf][1][zh][zi] = __builtin_bit_cast(bf8_t, z.m);
         zs[buf][2][zh][zi] = __builtin_bit_cast(bf8_t, z.l);
         if (cload) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) cv[e] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, cv[e]) ^ sign);
             const Split c = split8(cv, top_c);
             cs[buf][0][ch][ci] = __builtin_bit_cast(bf8_t, c.h);
             cs[buf][1][ch][ci] = __builtin_bit_cast(bf8_t, c.m);
@@ -196,12 +207,19 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     for (int a = 0; a < TA; ++a)
 #pragma unroll
         for (int b = 0; b < TB; ++b) acc[a][b] = f16_t{};
+    auto turn_sign = [&]() {
+#pragma unroll
+        for (int a = 0; a < TA; ++a)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) acc[a][b] = -acc[a][b];
+    };
     fetch(0);
     store(0, 0);
     fetch(min(1, npanel - 1));
     __syncthreads();
     for (int p = 0; p < npanel; ++p) {
         const int cur = p & 1;
+        if (turn > 0 && (p == turn || p == 3 * turn)) turn_sign();
         // the two waves of a SIMD split the next panel on either side of their
         // products, so that one of them keeps the matrix core busy
         if (wave < 4) {
