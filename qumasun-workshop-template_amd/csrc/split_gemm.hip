@@ -12,23 +12,27 @@
 // at 3072.  The panels of the second and third quarter of K are therefore summed with
 // the other sign (C's values and the accumulators turn there and back), which takes
 // out a constant as well as a linearly growing drift: at most 0.01 on inputs of
-// mixed or one sign, 0.04 where the terms grow along K.  It costs 2 %.
+// mixed or one sign, 0.04 where the terms grow along K.
 //
 // Measured (before: the FP32 MFMA kernels of blas.hip): 1536 x 1024 over 884,736
-// points 21.5 -> 14.3 ms (130 -> 195 TFLOP/s), 384 x 256 over 262,144 points 440 -> 329
-// us, 600 x 400 over 157,685 points (no multiple of their tiles) 1128 -> 550 us.  Error
-// against 64 bits 2.2e-7 .. 9.9e-7 -> 1.8e-7 .. 8.4e-7 (m = 256 .. 3072).  The matrix core is busy for half
-// of the time (at 2.1 GHz); the splits and the barrier of each panel take the rest.
-// Reading each operand a group of products earlier changed nothing; 128 columns
-// a workgroup throughout, two workgroups a CU, cost 11 %.
+// points 21.5 -> 14.0 ms (130 -> 199 TFLOP/s), 384 x 256 over 262,144 points 440 -> 329
+// us, 600 x 400 over 157,685 points (no multiple of their tiles) 1128 -> 540 us.  Error
+// against 64 bits 2.2e-7 .. 9.9e-7 -> 1.8e-7 .. 8.4e-7 (m = 256 .. 3072).  The matrix
+// core is busy for half of the time (at 2.1 GHz); the splits and the barrier of each
+// panel take the rest.  Reading each operand a group of products earlier changed
+// nothing; 128 columns a workgroup throughout, two workgroups a CU, cost 11 %.
 //
-// The split holds for finite values whose low parts do not underflow.  A
-// workgroup watches the largest magnitude that each of its threads has split;
-// where that is beyond bf16's largest finite value (so also for infinities) or
-// below 2^-100, it computes its tile again on the FP32 MFMA, so that such inputs
-// give what they always gave.  (Smaller values beside larger ones are held to
-// 2^-133, 2^-33 of the largest.)  NaN stays NaN in every product.
+// Three bf16 values hold 24 bits from 2^-110 on (the last bit of l is then a bf16
+// value).  Both operands are therefore multiplied by 2^40 as they are split, which
+// brings FP32's smallest subnormal there, and the sums by 2^-80 as they are stored:
+// no value loses bits, also where tiny ones stand beside ordinary ones.  (Before,
+// values below 2^-110 did: a column of 1e-36 among ordinary ones was passed on with
+// 14 bits.)  What leaves the range at its other end (values from 2^88, sums from 2^48,
+// infinities) leaves a sum that is not finite; the workgroup then computes its tile
+// again on the FP32 MFMA, so that such inputs give what they always gave.  That takes
+// 3.5 times as long (50 ms for the first shape above).  NaN stays NaN in every product.
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "qm_cols.h"
@@ -43,7 +47,7 @@ typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef float f16_t __attribute__((ext_vector_type(16)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
-// x = h + m + l, 8 values at a time, and the largest |x| so far
+// x scale = h + m + l, 8 values at a time
 typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 struct Split {
     u4_t h, m, l;  // 8 bf16 values each
@@ -54,12 +58,12 @@ __device__ __forceinline__ float wide_lo(bf2_t p) {
 __device__ __forceinline__ float wide_hi(bf2_t p) {
     return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, p) & 0xffff0000u);
 }
-__device__ __forceinline__ Split split8(const float (&x)[8], float &top) {
+__device__ __forceinline__ Split split8(const float (&x)[8], float scale) {
     Split s;
     // in pairs: one conversion instruction each
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-        const f2_t v = {x[e], x[e + 1]};
+        const f2_t v = {x[e] * scale, x[e + 1] * scale};
         const bf2_t h = __builtin_convertvector(v, bf2_t);
         const f2_t r = {v[0] - wide_lo(h), v[1] - wide_hi(h)};
         const bf2_t m = __builtin_convertvector(r, bf2_t);
@@ -68,14 +72,8 @@ __device__ __forceinline__ Split split8(const float (&x)[8], float &top) {
         s.h[e / 2] = __builtin_bit_cast(uint32_t, h);
         s.m[e / 2] = __builtin_bit_cast(uint32_t, m);
         s.l[e / 2] = __builtin_bit_cast(uint32_t, l);
-        top = fmaxf(top, fmaxf(fabsf(v[0]), fabsf(v[1])));
     }
     return s;
-}
-
-// whether values up to `top` leave the range in which the split is exact
-__device__ __forceinline__ bool out_of_split(float top) {
-    return top >= 3.3895e38f || (top > 0.0f && top < 7.8886e-31f);
 }
 
 __device__ __forceinline__ int xcd_block(int nblk, int per_xcd) {
@@ -84,6 +82,7 @@ __device__ __forceinline__ int xcd_block(int nblk, int per_xcd) {
     return lb < nblk ? lb : -1;
 }
 
+constexpr float kScale = 0x1p40f, kUnscale = 0x1p-80f;  // of each operand, and of the sums
 constexpr int SG_THREADS = 512, SG_K = 16;  // 8 waves; K rows per panel (one MFMA deep)
 constexpr int SG_PAD = 8;  // puts the two K halves of an index on different LDS banks
 
@@ -145,7 +144,7 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     const int turn = npanel / 4;  // panels from turn to 3 turn are summed with the other sign (see the file comment)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int zi = threadIdx.x & (SU_P - 1), zh = wave >> 2;
-    const bool cload = threadIdx.x < 2 * UN;  // whole waves
+    const bool cload = 2 * UN == SG_THREADS || threadIdx.x < 2 * UN;  // whole waves
     const int ci = (threadIdx.x >> 1) & (UN - 1), ch = threadIdx.x & 1;
     // points and columns past the end are computed on the last one and not stored
     const int64_t zp = min(p0 + zi, ng - 1);
@@ -155,9 +154,10 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
     // and past the array's end it gets zeros
     const __amdgpu_buffer_rsrc_t crsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(Cm), 0,
                                                                           (int)((uint32_t)m * n * 4u), 0x20000);
-    float zv[8], cv[8], top_z = 0.0f, top_c = 0.0f;
+    float zv[8], cv[8];
     // Straight-line: a branch around the loads would make their results meet
-    // at its end, and wait there.  K past m is read from column m - 1 (cleared in store).
+    // at its end, and wait there.  K past m is read from column m - 1 (cleared in
+    // store), and threads without a column of C read another's again.
     auto fetch = [&](int p) {
         const int kz = p * SG_K + 8 * zh;
         const int end = zcols.end(min(kz, m - 1));
@@ -168,19 +168,16 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
             zv[e] = zc[zp];
             zc = kz + e + 1 == end ? znext : (kz + e + 1 < m ? zc + ng : zc);
         }
-        if (cload) {
-            const uint32_t o = coff + p * (SG_K * 4);
-            const f4_t v0 = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(crsrc, o, 0, 0));
-            const f4_t v1 = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(crsrc, o + 16, 0, 0));
+        const uint32_t o = coff + p * (SG_K * 4);
+        const f4_t v0 = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(crsrc, o, 0, 0));
+        const f4_t v1 = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(crsrc, o + 16, 0, 0));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                cv[e] = v0[e];
-                cv[4 + e] = v1[e];
-            }
+        for (int e = 0; e < 4; ++e) {
+            cv[e] = v0[e];
+            cv[4 + e] = v1[e];
         }
     };
     auto store = [&](int buf, int p) {
-        const uint32_t sign = p >= turn && p < 3 * turn ? 0x80000000u : 0u;
         if ((p + 1) * SG_K > m) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -188,14 +185,12 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
                 cv[e] = p * SG_K + 8 * ch + e < m ? cv[e] : 0.0f;
             }
         }
-        const Split z = split8(zv, top_z);
+        const Split z = split8(zv, kScale);
         zs[buf][0][zh][zi] = __builtin_bit_cast(bf8_t, z.h);
         zs[buf][1][zh][zi] = __builtin_bit_cast(bf8_t, z.m);
         zs[buf][2][zh][zi] = __builtin_bit_cast(bf8_t, z.l);
         if (cload) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) cv[e] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, cv[e]) ^ sign);
-            const Split c = split8(cv, top_c);
+            const Split c = split8(cv, p >= turn && p < 3 * turn ? -kScale : kScale);
             cs[buf][0][ch][ci] = __builtin_bit_cast(bf8_t, c.h);
             cs[buf][1][ch][ci] = __builtin_bit_cast(bf8_t, c.m);
             cs[buf][2][ch][ci] = __builtin_bit_cast(bf8_t, c.l);
@@ -222,38 +217,61 @@ __global__ __launch_bounds__(SG_THREADS) void split_update_kernel(ColBlocks Z, C
         if (turn > 0 && (p == turn || p == 3 * turn)) turn_sign();
         // the two waves of a SIMD split the next panel on either side of their
         // products, so that one of them keeps the matrix core busy
+        // (the fetch's scheduling apart: mixed with the splits, its results were copied,
+        // and waited for, right behind the loads, 15.4 ms instead of 14.0)
         if (wave < 4) {
             store(cur ^ 1, p + 1);
+            __builtin_amdgcn_sched_barrier(0);
             fetch(min(p + 2, npanel - 1));
+            __builtin_amdgcn_sched_barrier(0);
         }
         panel_products<TA, TB>(acc, cs[cur], zs[cur], wc, wp, lane);
         if (wave >= 4) {
             store(cur ^ 1, p + 1);
+            __builtin_amdgcn_sched_barrier(0);
             fetch(min(p + 2, npanel - 1));
+            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
     }
     const int i = lane & 31, kh = lane >> 5;
     const Cols<float> ycols(Y, ng);
-    if (__syncthreads_or(out_of_split(top_z) || out_of_split(top_c))) {
-        for (int a = 0; a < TA; ++a)
-            for (int b = 0; b < TB; ++b) {
-                f16_t s = f16_t{};
-                const int col = c0 + wc + 32 * a + i;
-                const int64_t pt = p0 + wp + 32 * b + i;
-                for (int k = 0; k < m; k += 2) {
-                    const int kk = k + kh;
-                    const float av = (col < n && kk < m) ? Cm[(int64_t)col * m + kk] : 0.0f;
-                    const float bv = (pt < ng && kk < m) ? zcols.at(kk)[pt] : 0.0f;
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, s, 0, 0, 0);
-                }
+    bool finite = true;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int cr = c0 + wc + 32 * a + sg_row(r, lane);
-                    if (cr < n && pt < ng) ycols.at(cr)[pt] = s[r];
-                }
+    for (int a = 0; a < TA; ++a)
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                finite = finite && fabsf(acc[a][b][r]) < HUGE_VALF;
+                acc[a][b][r] *= kUnscale;
             }
-        return;
+    if (__syncthreads_or(!finite)) {
+#pragma unroll
+        for (int a = 0; a < TA; ++a)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) acc[a][b] = f16_t{};
+#pragma unroll 4
+        for (int k = 0; k < m; k += 2) {
+            const int kk = k + kh;
+            float av[TA], bv[TB];
+#pragma unroll
+            for (int a = 0; a < TA; ++a) {
+                const float v = Cm[(int64_t)min(c0 + wc + 32 * a + i, n - 1) * m + min(kk, m - 1)];
+                av[a] = kk < m ? v : 0.0f;
+            }
+            const GlobalPtr<float> zc = zcols.at(min(kk, m - 1));
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                const float v = zc[min(p0 + wp + 32 * b + i, ng - 1)];
+                bv[b] = kk < m ? v : 0.0f;
+            }
+#pragma unroll
+            for (int a = 0; a < TA; ++a)
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+        }
     }
 #pragma unroll
     for (int a = 0; a < TA; ++a)
