@@ -170,7 +170,9 @@ int qm_nonlocal_add_f32(qm_ctx *ctx, float *d_out, const float *d_psi, int nb, i
  *                            kt bit 1: the shape of full qm_hpsi_apply_* calls).
  * A full qm_hpsi_apply_* runs the stencil after the nonlocal projection or
  * beside it; its shape and that order are tuned separately, on full applies,
- * the first time that shape of call is seen (and synchronises the stream then). */
+ * the first time that shape of call is seen (and synchronises the stream then),
+ * and again once qm_set_projectors has changed the set's voxels times projectors
+ * by more than a factor of 2. */
 int qm_stencil_num_candidates(void);
 int qm_stencil_candidate_name(int candidate, char *buf, int buflen);
 int qm_stencil_force(qm_ctx *ctx, int candidate);

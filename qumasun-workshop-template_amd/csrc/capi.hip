@@ -247,6 +247,9 @@ constexpr float kOverlapMinMs = 0.1f;
 // them decide on a shape as well as four, in three fifths of the tuning's time
 constexpr float kLongMs = 0.3f;
 
+// What the nonlocal part's time goes with
+int64_t nl_work(const Projectors &p) { return p.vtot * p.mpad; }
+
 // part: 3 = local + nonlocal (overwrite), 1 = local only (overwrite), 2 = nonlocal only (accumulate)
 template <typename T>
 int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, void *stream, int part = 3) {
@@ -346,6 +349,7 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 }
                 if (status == QM_ERR_HIP) set_error("H.psi schedule tuning: HIP event failure");
                 if (status != QM_OK) return status;
+                if (ctx->apply_overlapped.empty()) ctx->tuned_nl_work = nl_work(ctx->proj);
                 it = ctx->apply_overlapped.emplace(key, beside).first;
             }
             return it->second ? overlapped() : in_order();
@@ -405,6 +409,7 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 if (status == QM_ERR_HIP) set_error("H.psi shape tuning: HIP event failure");
                 if (status != QM_OK) return status;
                 ctx->stencil_choice[key] = cand;
+                if (ctx->apply_overlapped.empty()) ctx->tuned_nl_work = nl_work(ctx->proj);
                 ctx->apply_overlapped[key] = beside;
             }
         }
@@ -694,6 +699,15 @@ int qm_set_projectors(qm_ctx *ctx, int natoms, const int *nproj, const int64_t *
     free_kpoints(ctx);
     ctx->proj = np;
     ctx->kpts = nk;
+    // full applies are tuned again where the nonlocal part has changed by more than
+    // a factor of 2 since: which order and which stencil shape beside it win
+    // depends on its share (64^3 x 128 FP32, overlapped against in order: 0.86 of
+    // the time with 16 atoms, 0.91 with 2).  Atoms that only move keep the choice.
+    const int64_t work = nl_work(np), then = ctx->tuned_nl_work;
+    if (work > 2 * then || 2 * work < then) {
+        for (const auto &kv : ctx->apply_overlapped) ctx->stencil_choice.erase(kv.first);
+        ctx->apply_overlapped.clear();
+    }
     cleanup.p = nullptr;
     cleanup.k = nullptr;
     return QM_OK;

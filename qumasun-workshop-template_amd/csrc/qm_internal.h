@@ -137,6 +137,7 @@ struct qm_ctx {
     std::map<int64_t, int> stencil_choice;  // autotuned stencil candidate per shape
     std::map<int64_t, std::vector<float>> stencil_ms;  // each candidate's time when its shape was tuned (ms)
     std::map<int64_t, bool> apply_overlapped;  // tuned schedule of full applies (by their stencil_choice key)
+    int64_t tuned_nl_work = 0;  // voxels x padded projectors of the set they were tuned with
     int stencil_force = -1;                 // >= 0: use this candidate, no tuning
     std::map<int64_t, int> nl_choice;       // autotuned column tiles per projection workgroup per shape
     int nl_force = 0;                       // > 0: use this many column tiles, no tuning
