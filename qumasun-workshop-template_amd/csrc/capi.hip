@@ -241,7 +241,8 @@ int launch_local(qm_ctx *ctx, T *out, const T *in, int nb, int ncomp, const doub
 // Applies that take less than this one after the other never overlap: the
 // fork and the join cost ~12 us, more than the overlap gives there (32^3 x 24
 // FP64: 28 us in order, 45-50 us overlapped; at 64^3 x 128 FP32 the overlap
-// wins, 143 against 158 us on warm caches).
+// wins, 152 against 176 us, as it did, by up to 14 %, in all 17 shapes measured
+// above this line).
 constexpr float kOverlapMinMs = 0.1f;
 // Applies longer than this differ by less than 1 % from one to the next: two of
 // them decide on a shape as well as four, in three fifths of the tuning's time
@@ -302,12 +303,11 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
             QM_HIP(hipStreamWaitEvent(st, ctx->ev_join, 0));
             return scatter();
         };
-        // mean time of `reps` applies after a warm-up (none for reps = 1)
-        hipEvent_t ev[2] = {nullptr, nullptr};
+        // mean time of `reps` applies
+        hipEvent_t ev[4] = {};
         int status = QM_OK;
         auto timed = [&](auto &&run, int reps) -> float {
             float ms = 0.0f;
-            status = reps > 1 ? run() : QM_OK;
             if (status == QM_OK && hipEventRecord(ev[0], st) != hipSuccess) status = QM_ERR_HIP;
             for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
             if (status == QM_OK && hipEventRecord(ev[1], st) != hipSuccess) status = QM_ERR_HIP;
@@ -315,15 +315,38 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
             if (status == QM_OK && hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) status = QM_ERR_HIP;
             return ms / (float)reps;
         };
+        // whether `reps` applies of b take less time than the mean of those of a before
+        // and after them, and a's more than kOverlapMinMs; all queued at once: applies
+        // right after a shape's first ones run up to 20 % faster or slower than the
+        // same ones later, and after a wait the overlapped form pays for its launches
+        auto faster = [&](auto &&b, auto &&a, int reps) -> bool {
+            auto mark = [&](int i) {
+                if (status == QM_OK && hipEventRecord(ev[i], st) != hipSuccess) status = QM_ERR_HIP;
+            };
+            auto turn = [&](auto &&run) {
+                for (int rep = 0; rep < reps && status == QM_OK; ++rep) status = run();
+            };
+            float t[3] = {0.0f, 0.0f, 0.0f};
+            mark(0);
+            turn(a);
+            mark(1);
+            turn(b);
+            mark(2);
+            turn(a);
+            mark(3);
+            if (status == QM_OK && hipEventSynchronize(ev[3]) != hipSuccess) status = QM_ERR_HIP;
+            for (int i = 0; i < 3; ++i)
+                if (status == QM_OK && hipEventElapsedTime(&t[i], ev[i], ev[i + 1]) != hipSuccess) status = QM_ERR_HIP;
+            return t[2] > kOverlapMinMs * (float)reps && 2.0f * t[1] < t[0] + t[2];
+        };
         struct Events {
             hipEvent_t *e;
             int create() {
-                QM_HIP(hipEventCreate(&e[0]));
-                QM_HIP(hipEventCreate(&e[1]));
+                for (int i = 0; i < 4; ++i) QM_HIP(hipEventCreate(&e[i]));
                 return QM_OK;
             }
             ~Events() {
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 4; ++i)
                     if (e[i]) (void)hipEventDestroy(e[i]);
             }
         } events{ev};
@@ -339,18 +362,13 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 if (capturing || g_internal_capture) return overlapped();
                 QM_TRY(in_order());  // the projection's shape is tuned alone first
                 QM_TRY(events.create());
-                // one apply each: the two schedules differ by up to a tenth, single
-                // applies by 1 %, and the first apply of a shape pays for all of them
-                const float ms = timed(in_order, 1);
-                bool beside = false;
-                if (status == QM_OK && ms > kOverlapMinMs) {
-                    QM_TRY(side_stream(ctx));
-                    beside = timed(overlapped, 1) < ms;
-                }
+                QM_TRY(side_stream(ctx));
+                const bool beside = faster(overlapped, in_order, 1);
                 if (status == QM_ERR_HIP) set_error("H.psi schedule tuning: HIP event failure");
                 if (status != QM_OK) return status;
                 if (ctx->apply_overlapped.empty()) ctx->tuned_nl_work = nl_work(ctx->proj);
-                it = ctx->apply_overlapped.emplace(key, beside).first;
+                ctx->apply_overlapped[key] = beside;
+                return QM_OK;  // the timed applies have left the result
             }
             return it->second ? overlapped() : in_order();
         }
@@ -383,25 +401,30 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 cand = alone;
                 beside = false;
                 ctx->stencil_force = alone;
-                const float best_ms = timed(in_order, 4);
-                if (best_ms > kOverlapMinMs) {
-                    const int reps = best_ms > kLongMs ? 2 : 4;
-                    const float in_order_ms = best_ms;
+                const float ms = timed(in_order, 2);
+                if (status == QM_OK && ms > kOverlapMinMs) {
+                    const int reps = ms > kLongMs ? 2 : 4;
                     float over_ms = 1e30f;
                     int over = alone;
                     for (int c = 0; c < stencil_num_candidates() && status == QM_OK; ++c) {
                         if (!stencil_near_best(ctx, prec, ncomp, kt, nb, c)) continue;
                         ctx->stencil_force = c;
-                        const float ms = timed(overlapped, reps);
-                        if (status == QM_OK && ms < over_ms) {
-                            over_ms = ms;
+                        status = overlapped();
+                        const float t = timed(overlapped, reps);
+                        if (status == QM_OK && t < over_ms) {
+                            over_ms = t;
                             over = c;
                         }
                     }
-                    // in order has to win clearly: four applies right after the
-                    // shapes' tuning have preferred it where fifty later ones ran
-                    // in 160 us against 146 overlapped (64^3 x 128 FP32)
-                    if (status == QM_OK && over_ms < 1.1f * in_order_ms) {
+                    auto plain = [&]() -> int {
+                        ctx->stencil_force = alone;
+                        return in_order();
+                    };
+                    auto forked = [&]() -> int {
+                        ctx->stencil_force = over;
+                        return overlapped();
+                    };
+                    if (status == QM_OK && faster(forked, plain, ms > kLongMs ? 1 : 2)) {
                         cand = over;
                         beside = true;
                     }
@@ -411,6 +434,7 @@ int hpsi_apply(qm_ctx *ctx, T *hpsi, const T *psi, int nb, int ncomp, int ik, vo
                 ctx->stencil_choice[key] = cand;
                 if (ctx->apply_overlapped.empty()) ctx->tuned_nl_work = nl_work(ctx->proj);
                 ctx->apply_overlapped[key] = beside;
+                return QM_OK;  // the timed applies have left the result
             }
         }
         ctx->stencil_force = cand;
