@@ -862,10 +862,12 @@ int nonlocal_scatter(qm_ctx *ctx, T *hpsi, const T *coef, int nb, const T *phase
     if (m > 16) return scatter_mfma<T, NC, PH, 8>(ctx, hpsi, coef, ncol, phase, st);
     if constexpr (sizeof(T) == 8) {
         if (m > 12) return scatter_mfma<T, NC, PH, 4>(ctx, hpsi, coef, ncol, phase, st);
-        // up to 9 projectors the thread-per-point kernel wins on large launches
-        // (36x40x42 x 45 complex, 3100 waves: 22.9 us there, 20.4 here; 64^3 x 32
-        // complex, 8512: 50 and 54; 64^3 x 128 real, 17024: 97 and 106), not with 16
-        // (64^3 x 64 complex: 109 and 101)
+        // up to 9 projectors the thread-per-point kernel wins on large launches, not
+        // with 16 (64^3 x 64 complex: 109 us there, 101 here).  40 applies timed both ways
+        // (us here less us there): 560 - 3000 waves -1.8 .. -0.2 of 15 - 34; 4000 - 4500 real
+        // +1.6 .. +2.6 of 43 - 50, complex -1.3 .. +0.1; 5200 - 8500 real -3.5 .. +6.2 of 53 -
+        // 88 (10 of 12 above 0), complex -2.3 .. +2.4; 11,000 - 17,000 real +2.7 .. +11 of 116 -
+        // 179, complex -0.3 .. +1.7
         if (m > 9 || scatter_waves(ctx->proj, ncol) < 4096)
             return scatter_mfma<T, NC, PH, 3>(ctx, hpsi, coef, ncol, phase, st);
         return scatter_points<T, NC, PH, 9>(ctx, hpsi, coef, ncol, phase, st);

@@ -10,9 +10,10 @@
 // blocks of traffic per kinetic apply (read psi, write out; read psi, read and
 // write out) instead of the ~14 of pack, two 3-D library transforms, scaling
 // and unpack.  64^3 x 64 complex FP64 (268 MB a block): 737 -> 351 us (3.8 TB/s),
-// 128 real FP32 bands 457 -> 191 us.  The error against extended precision is
-// smaller too (64 x 48 x 40: 3.0e-16 for 5.1e-16, FP32 1.35e-7 for 2.20e-7): a
-// transform's rounding is scaled by its own axes' q^2 only.
+// 128 real FP32 bands 457 -> 191 us.  The error against extended precision (80-bit
+// transforms, rms) is smaller too, 64 x 48 x 40 3.0e-16 for 5.1e-16, FP32 1.34e-7 for
+// 2.19e-7: a transform's rounding is scaled by its own axes' q^2 only.  (Against a
+// 64-bit transform, itself 5e-16 off, it can read larger.)
 //
 // Transforms are in place in LDS: decimation in frequency forward (natural
 // order in, digit-reversed out), the mirrored decimation in time back, so

@@ -33,7 +33,7 @@ def subspace_force(route):
 
 
 def coop_spin_limit(polls=None):
-    """Bound of the cooperative kernels' grid-barrier waits in polls,
+    """Bound of the cooperative reduction's grid-barrier waits in polls,
     process-wide (qm_coop_set_spin_limit); None restores the default."""
     L = _lib.load()
     _lib.check(L.qm_coop_set_spin_limit(int(L.qm_coop_spin_limit_default() if polls is None else polls)))
