@@ -337,8 +337,8 @@ int qm_lobpcg_set_conditioning(qm_lobpcg *s, double min_pivot_ratio_fp64, double
  * S-eigenbasis path: a way to exercise the fallback. */
 int qm_lobpcg_fallbacks(qm_lobpcg *s);
 /* Subspace eigensolves of the last qm_lobpcg_solve that had to be redone: a
- * divide-and-conquer tridiagonal solve that did not converge (redone by
- * QL/QR), a heevd / syevd that did not converge (redone by Jacobi), a
+ * divide-and-conquer tridiagonal solve that did not converge (the own one is redone
+ * by rocSOLVER's, that one by QL/QR), a heevd / syevd that did not converge (redone by Jacobi), a
  * tridiagonal reduction with non-finite output (redone by heevd), or Cholesky-
  * route Ritz vectors rejected because max_i |1 - c_i^H S c_i| exceeded 1e-4 (S
  * too ill-conditioned for its Cholesky factor; redone without P, then on the
